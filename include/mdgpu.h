@@ -299,10 +299,10 @@ int mdgpu_get_timing(const mdgpu_domain *d, int *force_launches, double *force_m
                                       candidates at a time (1, the default), or a thread per
                                       row (0); the same masks either way */
 #define MDGPU_OPT_RUN_AHEAD 13  /* mdgpu_calculate queues up to this many fused steps without
-                                   waiting for the host (default 64; 0 = every step waits): a
-                                   device-side gate does each step's validity budget and stops
-                                   the run at the step whose displacement check or construction
-                                   needs the host, which then takes that step; the same
+                                   waiting for the host (default 64; 0 = every step waits): each
+                                   step's validity test, budget and displacement check, runs on
+                                   the device at the end of the step before and stops the run
+                                   where a list has expired, for the host to rebuild; the same
                                    trajectory either way */
 #define MDGPU_OPT_PIPELINE 14  /* FP64 kick with 4, 8 or 16 wavefronts: 1 = persistent workgroups (one
                                   per CU) whose producer wavefronts stage the next brick's

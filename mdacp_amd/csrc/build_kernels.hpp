@@ -142,14 +142,6 @@ __global__ void k_gather_owned(const int *__restrict__ perm, int n, const double
 // vector whose every non-zero component passes its face test.  The box is
 // [s, e) = [0, L) (MDRect::IsInsideEdge, mdrect.cc:24-47: s < q < s + SL and
 // e - SL < q < e).
-__device__ __forceinline__ void face_options(const double4 q, const Replica &R, double SL, int lo[3], int hi[3]) {
-  const double v[3] = {q.x, q.y, q.z};
-  for (int d = 0; d < 3; d++) {
-    lo[d] = (v[d] < 0.0 + SL && v[d] > 0.0);
-    hi[d] = (v[d] > R.L[d] - SL && v[d] < R.L[d]);
-  }
-}
-
 __global__ void k_count_images(const double4 *__restrict__ pos, int n, const int *__restrict__ rep,
                                const Replica *__restrict__ reps, double SL, int *__restrict__ nimg) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;

@@ -111,15 +111,48 @@ struct Replica {
 
 __device__ __forceinline__ int replica_bricks(const Replica &R) { return R.nb[0] * R.nb[1] * R.nb[2]; }
 
-// A run of fused steps queued without waiting for the host.  The gate kernel
-// at the head of each step halts the run when that step's validity test needs
-// the host (a budget spent: the displacement check or a construction is due;
-// or a particle too fast); the step's other kernels then return at once, and
-// so does every step queued after it, which leaves the state of the last
-// completed step for the host to take the halted step from.
+// A run of fused steps queued without waiting for the host.  The validity
+// test of a step (the host's for the first step of the run, the end of the
+// step before it for the others) halts the run when the step needs the host
+// (a budget spent: the displacement check or a construction is due; or a
+// particle too fast); the step's kernels then return at once, and so does
+// every step queued after it, which leaves the state of the last completed
+// step for the host to take the halted step from.
 struct RunGate {
   int halted;  // 0 while the run goes on
   int done;    // steps completed in this run
+  int left;    // steps of the run still to come, the current one included
+};
+
+// The PairList state of one replica while a run goes on, and what the steps'
+// validity tests need of it.  A step whose test may find the budget spent
+// ("measured") also takes the displacements since the construction
+// (pairlist.cc:68-121): its bricks' largest to dmax2, and the entries displaced
+// by more than cthr as candidates.
+struct RunRep {
+  double budget;  // validity budget
+  double v2;      // max |p|^2 after the last step
+  double dmax2;   // measured: the largest squared displacement after the last step
+  double cthr;    // measured: displacement from which entries are candidates
+  int lifetime;
+  int measured;   // the step in progress (or the last one) takes displacements
+  int ncand;      // candidates found (more than the room for them: not all kept)
+};
+
+// A candidate of the displacement test: its position at the construction (w:
+// squared displacement) and now.
+struct RunCand {
+  double4 old, now;
+};
+
+// Where a run's kick puts what a measured step takes (rr == nullptr: nothing).
+struct RunMeasure {
+  RunRep *rr;
+  const double4 *old;  // positions at the construction, owned particles
+  double *dpart;       // per brick: largest squared displacement
+  RunCand *cand;       // cap per replica
+  int cap;
+  double SL;
 };
 
 __device__ __forceinline__ bool run_halted(const RunGate *g) { return g != nullptr && g->halted != 0; }
@@ -139,6 +172,17 @@ __device__ __forceinline__ double3 image_of(double4 q, int code, const double *L
   const double dy = sy > 0 ? L[1] : (sy < 0 ? -L[1] : 0.0);
   const double dz = sz > 0 ? L[2] : (sz < 0 ? -L[2] : 0.0);
   return make_double3(q.x + dx, q.y + dy, q.z + dz);
+}
+
+// The face tests of the halo (strict, mdrect.cc:24-47) for a position of a
+// periodic box [0, L): lo: within SL of the low face (an image at +L), hi: of
+// the high face (an image at -L).
+__device__ __forceinline__ void face_options(const double4 q, const Replica &R, double SL, int lo[3], int hi[3]) {
+  const double v[3] = {q.x, q.y, q.z};
+  for (int d = 0; d < 3; d++) {
+    lo[d] = (v[d] < 0.0 + SL && v[d] > 0.0);
+    hi[d] = (v[d] > R.L[d] - SL && v[d] < R.L[d]);
+  }
 }
 
 }  // namespace mdgpu

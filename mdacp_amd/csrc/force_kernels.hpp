@@ -39,6 +39,8 @@ struct BrickList {
   const long long *sbase;   // first slot of each 64-row slice
   const int *slen;          // slots per slice (multiple of kSliceRound)
   const int *glist;         // staged entry -> particle index (owned, or pn + ghost)
+  const uint32_t *gimg;     // staged entry -> owner and shift (img_entry): images from their owners
+                            // in src; nullptr: through glist, images from `ghost`
   const long long *gbase;   // [brick + 1] first gather-list entry of each brick
   const int *row0, *nrow, *vslice0;
   const int *brep;          // replica of each brick
@@ -56,6 +58,7 @@ struct StepClock {
   uint64_t step;
   const unsigned long long *clock;
   const RunGate *gate;  // a step of a run: nothing to do once the run has halted
+  RunMeasure meas;      // a step of a run: its displacements since the construction, when measured
 };
 
 __device__ __forceinline__ uint64_t step_of(const StepClock &sc) { return sc.clock ? sc.clock[0] : sc.step; }
@@ -128,14 +131,39 @@ __device__ __forceinline__ void unpack_group(const u32x4 g, int e[kGroup]) {
   e[4] = g.z & 0xffff; e[5] = g.z >> 16; e[6] = g.w & 0xffff; e[7] = g.w >> 16;
 }
 
+// Where a pair loop reads the partners of a brick whose neighbourhood does not
+// fit the LDS budget: staged entry u's position through the brick's gather list.
+struct BrickGather {
+  const double4 *src, *ghost;
+  const int *gl;
+  const uint32_t *im;  // the brick's image list, or nullptr
+  const double *L;     // its replica's box
+  int pn, total;
+  __device__ __forceinline__ double4 at(int u) const {
+    if (im != nullptr) return img_of(src[img_index(im[u])], im[u], L);
+    return gather_pos(src, ghost, pn, gl[u]);
+  }
+};
+
+__device__ __forceinline__ BrickGather brick_gather(const BrickList &bl, const double4 *src, long long g0, int total,
+                                                    const Replica &R) {
+  BrickGather G;
+  G.src = src;
+  G.ghost = bl.ghost;
+  G.gl = bl.glist + g0;
+  G.im = bl.gimg != nullptr ? bl.gimg + g0 : nullptr;
+  G.L = R.L;
+  G.pn = bl.pn;
+  G.total = total;
+  return G;
+}
+
 // One group of kGroup list entries of a row: partners from LDS (kStaged) or
 // through the gather list, the smoothed-LJ kick added to a.
 template <bool kStaged>
 __device__ __forceinline__ void group_kick_fp64(const int e[kGroup], const double4 qi,
-                                                const double *__restrict__ lds, const double4 *__restrict__ src,
-                                                const int *__restrict__ gl, int total, const ForceConsts &fc, int pn,
-                                                const double4 *__restrict__ ghost, double &ax, double &ay,
-                                                double &az) {
+                                                const double *__restrict__ lds, const BrickGather &G,
+                                                const ForceConsts &fc, double &ax, double &ay, double &az) {
   double qx[kGroup], qy[kGroup], qz[kGroup];
 #pragma unroll
   for (int u = 0; u < kGroup; u++) {
@@ -144,8 +172,8 @@ __device__ __forceinline__ void group_kick_fp64(const int e[kGroup], const doubl
       qx[u] = q[0];
       qy[u] = q[1];
       qz[u] = q[2];
-    } else if (e[u] < total) {
-      const double4 q = gather_pos(src, ghost, pn, gl[e[u]]);
+    } else if (e[u] < G.total) {
+      const double4 q = G.at(e[u]);
       qx[u] = q.x;
       qy[u] = q.y;
       qz[u] = q.z;
@@ -180,9 +208,8 @@ __device__ __forceinline__ void group_kick_fp64(const int e[kGroup], const doubl
 // entries point at a far sentinel).
 template <bool kStaged, int P>
 __device__ __forceinline__ double3 row_kick_fp64(const uint4 *__restrict__ sg, int lane, int len, const double4 qi,
-                                                 const double *__restrict__ lds, const double4 *__restrict__ src,
-                                                 const int *__restrict__ gl, int total, const ForceConsts &fc,
-                                                 int pn, const double4 *__restrict__ ghost) {
+                                                 const double *__restrict__ lds, const BrickGather &G,
+                                                 const ForceConsts &fc) {
   double ax = 0.0, ay = 0.0, az = 0.0;
   const u32x4 *vg = reinterpret_cast<const u32x4 *>(sg);
   u32x4 ahead[P];
@@ -198,7 +225,7 @@ __device__ __forceinline__ double3 row_kick_fp64(const uint4 *__restrict__ sg, i
       unpack_group(ahead[j], e);
       ahead[j] = (vg + min(k / kGroup + j + P, last) * kWave)[ul];
       __builtin_amdgcn_sched_barrier(0);  // the prefetch is issued before this group's work
-      group_kick_fp64<kStaged>(e, qi, lds, src, gl, total, fc, pn, ghost, ax, ay, az);
+      group_kick_fp64<kStaged>(e, qi, lds, G, fc, ax, ay, az);
       // the buffer unpacked next was loaded P - 1 groups of work ago
       hold_prefetch(ahead[(j + 1) % P], ax, ay, az);
     }
@@ -210,7 +237,7 @@ __device__ __forceinline__ double3 row_kick_fp64(const uint4 *__restrict__ sg, i
     if (k + j * kGroup < len) {
       int e[kGroup];
       unpack_group(ahead[j], e);
-      group_kick_fp64<kStaged>(e, qi, lds, src, gl, total, fc, pn, ghost, ax, ay, az);
+      group_kick_fp64<kStaged>(e, qi, lds, G, fc, ax, ay, az);
     }
   }
   return make_double3(ax, ay, az);
@@ -296,10 +323,7 @@ __device__ __forceinline__ double3 row_kick_mixed(const uint4 *__restrict__ rg, 
 // group sums s).
 template <bool kStaged, int kSum>
 __device__ __forceinline__ void group_kick_mixed_brick(const int e[kGroup], const float4 ri,
-                                                       const float4 *__restrict__ lds,
-                                                       const double4 *__restrict__ src,
-                                                       const double4 *__restrict__ ghost, int pn,
-                                                       const int *__restrict__ gl, int total,
+                                                       const float4 *__restrict__ lds, const BrickGather &G,
                                                        const ForceConstsF &fc, const double3 c, float &ax, float &ay,
                                                        float &az, float &cx, float &cy, float &cz, double &sx,
                                                        double &sy, double &sz) {
@@ -308,8 +332,8 @@ __device__ __forceinline__ void group_kick_mixed_brick(const int e[kGroup], cons
   for (int u = 0; u < kGroup; u++) {
     if (kStaged) {
       rj[u] = lds[e[u]];
-    } else if (e[u] < total) {
-      const double4 q = gather_pos(src, ghost, pn, gl[e[u]]);
+    } else if (e[u] < G.total) {
+      const double4 q = G.at(e[u]);
       rj[u] = make_float4((float)(q.x - c.x), (float)(q.y - c.y), (float)(q.z - c.z), 0.0f);
     } else {
       rj[u] = make_float4(1.0e30f, 1.0e30f, 1.0e30f, 0.0f);
@@ -348,10 +372,8 @@ __device__ __forceinline__ void group_kick_mixed_brick(const int e[kGroup], cons
 template <bool kStaged, int kSum, int P>
 __device__ __forceinline__ double3 row_kick_mixed_brick(const uint4 *__restrict__ sg, int lane, int len,
                                                         const float4 ri, const float4 *__restrict__ lds,
-                                                        const double4 *__restrict__ src,
-                                                        const double4 *__restrict__ ghost, int pn,
-                                                        const int *__restrict__ gl, int total,
-                                                        const ForceConstsF &fc, const double3 c) {
+                                                        const BrickGather &G, const ForceConstsF &fc,
+                                                        const double3 c) {
   float ax = 0.f, ay = 0.f, az = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
   double sx = 0.0, sy = 0.0, sz = 0.0;
   const u32x4 *vg = reinterpret_cast<const u32x4 *>(sg);
@@ -368,8 +390,7 @@ __device__ __forceinline__ double3 row_kick_mixed_brick(const uint4 *__restrict_
       unpack_group(ahead[j], e);
       ahead[j] = (vg + min(k / kGroup + j + P, last) * kWave)[ul];
       __builtin_amdgcn_sched_barrier(0);  // the prefetch is issued before this group's work
-      group_kick_mixed_brick<kStaged, kSum>(e, ri, lds, src, ghost, pn, gl, total, fc, c, ax, ay, az, cx, cy, cz,
-                                            sx, sy, sz);
+      group_kick_mixed_brick<kStaged, kSum>(e, ri, lds, G, fc, c, ax, ay, az, cx, cy, cz, sx, sy, sz);
       hold_prefetch(ahead[(j + 1) % P], ax, ay, az);
     }
   }
@@ -378,8 +399,7 @@ __device__ __forceinline__ double3 row_kick_mixed_brick(const uint4 *__restrict_
     if (k + j * kGroup < len) {
       int e[kGroup];
       unpack_group(ahead[j], e);
-      group_kick_mixed_brick<kStaged, kSum>(e, ri, lds, src, ghost, pn, gl, total, fc, c, ax, ay, az, cx, cy, cz,
-                                            sx, sy, sz);
+      group_kick_mixed_brick<kStaged, kSum>(e, ri, lds, G, fc, c, ax, ay, az, cx, cy, cz, sx, sy, sz);
     }
   }
   if (kSum == kSumGroup64) return make_double3(sx, sy, sz);
@@ -435,6 +455,58 @@ __device__ __forceinline__ double finish_row(int i, double4 p, const double4 qi,
   return p.x * p.x + p.y * p.y + p.z * p.z;
 }
 
+// A measured step of a run (RunRep): the displacements of the brick's particles
+// and of their images, as k_displacement takes them after the step: an owned
+// particle's position at the end of the step (the operations of finish_row), a
+// ghost where the step's halo refresh has it (the owner's half drift, src,
+// plus the shift), each against the construction's.  A particle's images are
+// those its position at the construction gave it (face_options).  A pass of
+// its own after the rows, so that the pair loop's registers do not carry it;
+// it runs in the last steps before a construction only.  Every thread of the
+// workgroup calls it.
+template <int T>
+__device__ __forceinline__ void measure_brick(int b, int r, int row0, int nrow, const double4 *__restrict__ src,
+                                              const double4 *mom, int epilogue, double dt2, const Replica &R,
+                                              const RunMeasure &M) {
+  if (M.rr == nullptr || !M.rr[r].measured) return;
+  __syncthreads();  // the brick's momenta are written
+  const double thr2 = M.rr[r].cthr * M.rr[r].cthr;
+  double dm = 0.0;
+  auto take = [&](const double4 o, const double4 q) {
+    const double dx = o.x - q.x, dy = o.y - q.y, dz = o.z - q.z;
+    const double d2 = dx * dx + dy * dy + dz * dz;
+    dm = fmax(dm, d2);
+    if (d2 > thr2) {
+      const int k = atomicAdd(&M.rr[r].ncand, 1);
+      if (k < M.cap) M.cand[(size_t)r * M.cap + k] = RunCand{make_double4(o.x, o.y, o.z, d2), q};
+    }
+  };
+  for (int v = threadIdx.x; v < nrow; v += T) {
+    const int i = row0 + v;
+    const double4 o = M.old[i], qh = src[i];
+    double4 q = qh;
+    if (epilogue == kKickDrift) {
+      const double4 p = mom[i];
+      q.x += p.x * dt2;
+      q.y += p.y * dt2;
+      q.z += p.z * dt2;
+    }
+    take(o, q);
+    int lo[3], hi[3];
+    face_options(o, R, M.SL, lo, hi);
+    if (!(lo[0] | lo[1] | lo[2] | hi[0] | hi[1] | hi[2])) continue;
+    for (int code = 0; code < 27; code++) {
+      const int s[3] = {code % 3 - 1, (code / 3) % 3 - 1, code / 9 - 1};
+      bool image = code != 13;
+      for (int a = 0; a < 3; a++) image = image && (s[a] == 0 || (s[a] > 0 ? lo[a] : hi[a]));
+      if (!image) continue;
+      const double3 y = image_of(o, code, R.L), z = image_of(qh, code, R.L);
+      take(make_double4(y.x, y.y, y.z, 0.0), make_double4(z.x, z.y, z.z, 0.0));
+    }
+  }
+  block_max_to_partial(dm, M.dpart, b);
+}
+
 // FP64 kick: one workgroup per brick, wavefronts over the brick's slices;
 // U groups of list indices in flight ahead of the group computed.
 // The FP64 kick of brick b by the calling workgroup (the body of
@@ -453,14 +525,15 @@ __device__ __forceinline__ void brick_kick_fp64(const int b, const double4 *__re
   const int nrow = bl.nrow[b], row0 = bl.row0[b], vs0 = bl.vslice0[b];
   if (nrow == 0) {  // a brick without rows: nothing to stage
     if (vpart) block_max_to_partial(0.0, vpart, b);
+    if (sc.meas.rr != nullptr && threadIdx.x == 0) sc.meas.dpart[b] = 0.0;
     return;
   }
   const long long g0 = bl.gbase[b];
   const int total = (int)(bl.gbase[b + 1] - g0);
-  const int *gl = bl.glist + g0;
+  const BrickGather G = brick_gather(bl, src, g0, total, Rp);
   const bool staged = total < bl.lds_cap;  // uniform across the workgroup
   if (threadIdx.x == 0) slice_next = W;
-  if (staged) stage_fp64<T>(gl, total, src, lds64, bl.pn, bl.ghost);
+  if (staged) stage_fp64<T>(G.gl, total, src, lds64, bl.pn, bl.ghost, G.im, G.L);
   __syncthreads();
   const int nsl = (nrow + kWave - 1) / kWave;
   const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -476,8 +549,8 @@ __device__ __forceinline__ void brick_kick_fp64(const int b, const double4 *__re
     const RowExtra x = row_extra(i, epilogue, id, nd);
     const int len = bl.slen[s];
     const uint4 *sg = slice_groups(bl.nbr, bl.sbase[s]);
-    const double3 a = staged ? row_kick_fp64<true, U>(sg, lane, len, qi, lds64, src, gl, total, fc, bl.pn, bl.ghost)
-                             : row_kick_fp64<false, U>(sg, lane, len, qi, lds64, src, gl, total, fc, bl.pn, bl.ghost);
+    const double3 a = staged ? row_kick_fp64<true, U>(sg, lane, len, qi, lds64, G, fc)
+                             : row_kick_fp64<false, U>(sg, lane, len, qi, lds64, G, fc);
     if (ok) {
       p.x += a.x;
       p.y += a.y;
@@ -486,10 +559,13 @@ __device__ __forceinline__ void brick_kick_fp64(const int b, const double4 *__re
     }
   }
   if (vpart) block_max_to_partial(vmax, vpart, b);
+  measure_brick<T>(b, bl.brep[b], row0, nrow, src, mom, epilogue, fc.dt2, Rp, sc.meas);
 }
 
+// At most 128 registers with up to two groups ahead: four wavefronts per SIMD,
+// two 8-wavefront workgroups per CU (one register more halves that).
 template <int W, int U>
-__global__ __launch_bounds__(kWave *W) void k_force_brick_fp64(const double4 *__restrict__ src,
+__global__ __launch_bounds__(kWave *W, U <= 2 ? 4 : 1) void k_force_brick_fp64(const double4 *__restrict__ src,
                                                               double4 *__restrict__ mom,
                                                               double4 *__restrict__ pos_out, BrickList bl,
                                                               ForceConsts fc, int epilogue, StepClock sc,
@@ -688,7 +764,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
         const int row0 = bl.row0[b], vs0 = bl.vslice0[b];
         const long long g0 = bl.gbase[b];
         const int total = (int)(bl.gbase[b + 1] - g0);
-        const int *gl = bl.glist + g0;
+        const BrickGather Gb = brick_gather(bl, src, g0, total, Rp);
         const bool staged = total < cap;  // uniform across the workgroup
         const int nsl = (nrow + kWave - 1) / kWave;
         for (int sl = wv; sl < nsl; sl = take_next(&slice_next[cur], lane)) {
@@ -703,7 +779,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
           const uint4 *rg = reinterpret_cast<const uint4 *>(bl.nbr + bl.sbase[s] + lane * kGroup);
           const double3 a = staged ? row_kick_fp64_buf<U>(rg, len, qi, lbuf, fc)
                                    : row_kick_fp64<false, U>(slice_groups(bl.nbr, bl.sbase[s]), lane, len, qi,
-                                                             nullptr, src, gl, total, fc, bl.pn, bl.ghost);
+                                                             nullptr, Gb, fc);
           if (ok) {
             p.x += a.x;
             p.y += a.y;
@@ -720,6 +796,13 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
       double m = wmax[cur][0];
       for (int k = 1; k < W; k++) m = fmax(m, wmax[cur][k]);
       vpart[b] = m;
+    }
+      if (sc.meas.rr != nullptr) {  // uniform: every wavefront, producers included
+      if (bl.nrow[b] > 0)
+        measure_brick<kWave *(W + P)>(b, bl.brep[b], bl.row0[b], bl.nrow[b], src, mom, epilogue, fc.dt2,
+                                      bl.reps[bl.brep[b]], sc.meas);
+      else if (threadIdx.x == 0)
+        sc.meas.dpart[b] = 0.0;
     }
   }
 }
@@ -752,6 +835,7 @@ __global__ __launch_bounds__(kWave *W) void k_force_brick_mixed(
   const int nrow = bl.nrow[b], row0 = bl.row0[b], vs0 = bl.vslice0[b];
   if (nrow == 0) {  // a brick without rows: nothing to stage
     if (vpart) block_max_to_partial(0.0, vpart, b);
+    if (sc.meas.rr != nullptr && threadIdx.x == 0) sc.meas.dpart[b] = 0.0;
     return;
   }
   const long long g0 = bl.gbase[b];
@@ -805,6 +889,7 @@ __global__ __launch_bounds__(kWave *W) void k_force_brick_mixed(
     }
   }
   if (vpart) block_max_to_partial(vmax, vpart, b);
+  measure_brick<T>(b, bl.brep[b], row0, nrow, pos, mom, epilogue, dt2, Rp, sc.meas);
 }
 
 // Mixed-precision kick in a brick-centred FP32 frame: the workgroup stages its
@@ -831,6 +916,7 @@ __device__ __forceinline__ void brick_kick_mixed_brick(const int b, const double
   const int nrow = bl.nrow[b], row0 = bl.row0[b], vs0 = bl.vslice0[b];
   if (nrow == 0) {  // a brick without rows: nothing to stage
     if (vpart) block_max_to_partial(0.0, vpart, b);
+    if (sc.meas.rr != nullptr && threadIdx.x == 0) sc.meas.dpart[b] = 0.0;
     return;
   }
   const BrickBox X = brick_box(b, Rp);
@@ -839,19 +925,12 @@ __device__ __forceinline__ void brick_kick_mixed_brick(const int b, const double
                                  Rp.o[2] + (X.lo[2] + 0.5 * (X.n[2] - 2)) * Rp.w[2]);
   const long long g0 = bl.gbase[b];
   const int total = (int)(bl.gbase[b + 1] - g0);
-  const int *gl = bl.glist + g0;
+  const BrickGather G = brick_gather(bl, src, g0, total, Rp);
   const bool staged = total < bl.lds_cap;
   if (staged) {
     for (int u0 = threadIdx.x; u0 < total; u0 += T * kStageBatch) {
-      int j[kStageBatch];
-#pragma unroll
-      for (int k = 0; k < kStageBatch; k++) {
-        const int u = u0 + k * T;
-        j[k] = u < total ? gl[u] : 0;
-      }
       double4 q[kStageBatch];
-#pragma unroll
-      for (int k = 0; k < kStageBatch; k++) q[k] = gather_pos(src, bl.ghost, bl.pn, j[k]);
+      gather_batch<T>(u0, total, G.gl, G.im, src, bl.ghost, bl.pn, G.L, q);
 #pragma unroll
       for (int k = 0; k < kStageBatch; k++)
         if (u0 + k * T < total)
@@ -878,10 +957,8 @@ __device__ __forceinline__ void brick_kick_mixed_brick(const int b, const double
     }
     const int len = bl.slen[s];
     const uint4 *sg = slice_groups(bl.nbr, bl.sbase[s]);
-    const double3 a =
-        staged ? row_kick_mixed_brick<true, kSum, U>(sg, lane, len, ri, lds32, src, bl.ghost, bl.pn, gl, total, fc, c)
-               : row_kick_mixed_brick<false, kSum, U>(sg, lane, len, ri, lds32, src, bl.ghost, bl.pn, gl, total, fc,
-                                                      c);
+    const double3 a = staged ? row_kick_mixed_brick<true, kSum, U>(sg, lane, len, ri, lds32, G, fc, c)
+                             : row_kick_mixed_brick<false, kSum, U>(sg, lane, len, ri, lds32, G, fc, c);
     if (ok) {
       // loaded after the pair loop (registers)
       double4 p = mom[i];
@@ -894,6 +971,7 @@ __device__ __forceinline__ void brick_kick_mixed_brick(const int b, const double
     }
   }
   if (vpart) block_max_to_partial(vmax, vpart, b);
+  measure_brick<T>(b, bl.brep[b], row0, nrow, src, mom, epilogue, dt2, Rp, sc.meas);
 }
 
 template <int W, int U, int kSum>

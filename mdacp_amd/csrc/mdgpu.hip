@@ -156,13 +156,20 @@ struct mdgpu_domain {
   bool use_graph = false;   // fused steps replayed from a captured graph (launched directly when false)
   long epoch = 0;  // bumped whenever a captured step may no longer match
   StepGraph graphs[2];
-  // runs of steps queued without waiting for the host (k_gate at the head of
-  // each step): at most run_ahead steps per run (0: every step waits)
+  // runs of steps queued without waiting for the host (each step's validity
+  // test at the end of the step before, k_run_tail): at most run_ahead steps
+  // per run (0: every step waits)
   int run_ahead = 64;
   StepGraph gated[2];
   RunGate *gate = nullptr, *h_gate = nullptr;  // device state and its pinned mirror
-  double *gbudget = nullptr, *h_gbudget = nullptr;  // per replica: validity budget
-  int *glife = nullptr, *h_glife = nullptr;         // per replica: list lifetime
+  RunRep *rr = nullptr, *h_rr = nullptr;       // per replica: list state of a run, and its pinned mirror
+  RunCand *run_cand = nullptr;                 // candidates of the runs' displacement tests
+  int run_cap = 1;                             // ... kept per replica
+  double *dpart = nullptr;                     // one maximum displacement per brick workgroup
+  bool run_halted = false;  // the last run stopped at a step that the host decides
+  bool run_keep = false;    // what the last run's last step measured still holds
+  int since_build = 0;      // run steps since the last construction
+  int list_span = 0;        // ... when the last list expired (0: none has)
 
   // thermostat
   int thermostat = MDGPU_NVE;
@@ -202,6 +209,7 @@ struct mdgpu_domain {
   int *tstart = nullptr, *tbase = nullptr, *nrange = nullptr, *btotal = nullptr;
   long long *gbase = nullptr;  // [nbrick + 1] first gather-list entry of each brick
   int *glist = nullptr;        // staged entry -> particle index, brick by brick
+  uint32_t *gimg = nullptr;    // staged entry -> owner and image shift (none for a unit)
   long long glist_cap = 0;
   // list
   uint16_t *nbr = nullptr;   // staged partner index per list slot
@@ -333,6 +341,7 @@ int check_launch(mdgpu_domain *d, const char *what) {
 void invalidate(mdgpu_domain *d) {
   d->mid_valid = false;
   d->inner_valid = false;
+  d->run_keep = false;
   d->epoch++;
 }
 
@@ -470,6 +479,7 @@ int set_geometry(mdgpu_domain *d) {
   CHK(dalloc(d, &d->vslice0, d->nbrick));
   CHK(dalloc(d, &d->nrange, d->nbrick));
   CHK(dalloc(d, &d->bpart, d->nbrick));
+  CHK(dalloc(d, &d->dpart, d->nbrick));
   CHK(dalloc(d, &d->btotal, d->nbrick));
   CHK(dalloc(d, &d->gbase, d->nbrick + 1));
   CHK(dalloc(d, &d->tstart, (size_t)d->nbrick * kRangesPerCell * d->rmax));
@@ -742,6 +752,15 @@ int recode_list(mdgpu_domain *d) {
   return launch_emit(d, bricks_of(d), search_tables(d));
 }
 
+// The image gather list of the fused step (a unit's images come from other
+// units' particles: its steps refresh the halo).
+int image_glist(mdgpu_domain *d) {
+  if (d->group || d->gtotal == 0) return MDGPU_OK;
+  hipLaunchKernelGGL(k_image_glist, dim3(nblk(d->gtotal)), dim3(kBlock), 0, d->stream, d->glist, d->gtotal, d->pn,
+                     d->gsrc, d->gcode, d->gimg);
+  return check_launch(d, "image gather list");
+}
+
 // Rows of each brick by decreasing list length: permute the owned particles
 // (positions, momenta, ids, cells, row lengths) and remap the indices that
 // point at them (gather lists, ghost sources).  Ghosts keep their places.
@@ -753,7 +772,10 @@ int order_rows(mdgpu_domain *d) {
   const int pn = d->pn, ng = d->ng;
   hipLaunchKernelGGL(k_brick_row_order, dim3(d->nbrick), dim3(kBlock), 0, st, d->row_len, d->row0, d->nrow,
                      d->rowsrc, d->rowinv, d->row_sort);
-  if (d->row_sort == 0) return check_launch(d, "row order");
+  if (d->row_sort == 0) {
+    CHK(image_glist(d));
+    return check_launch(d, "row order");
+  }
   hipLaunchKernelGGL(k_gather_owned, dim3(nblk(pn)), dim3(kBlock), 0, st, d->rowsrc, pn, d->pos, d->mom, d->id,
                      d->cell, d->rep, d->pos_tmp, d->mom_alt, d->id_alt, d->cell_alt, d->rep_alt);
   hipLaunchKernelGGL(k_gather_int, dim3(nblk(pn)), dim3(kBlock), 0, st, d->rowsrc, pn, d->row_len, d->nimg);
@@ -774,6 +796,7 @@ int order_rows(mdgpu_domain *d) {
   std::swap(d->cell, d->cell_alt);
   std::swap(d->rep, d->rep_alt);
   std::swap(d->row_len, d->nimg);
+  CHK(image_glist(d));
   return check_launch(d, "row order");
 }
 
@@ -999,7 +1022,9 @@ int build_lists(mdgpu_domain *d) {
   d->gtotal = gtotal;
   if (gtotal > d->glist_cap) {
     const long long gc = gtotal + gtotal / 8 + 1024;
+    d->glist_cap = 0;
     CHK(dalloc(d, &d->glist, (size_t)gc));
+    if (!d->group) CHK(dalloc(d, &d->gimg, (size_t)gc));
     d->glist_cap = gc;
   }
   hipLaunchKernelGGL(k_brick_glist, dim3(d->nbrick), dim3(kBlock), 0, st, kRangesPerCell * d->rmax, d->tstart,
@@ -1073,6 +1098,7 @@ int build_lists(mdgpu_domain *d) {
     S.lifetime = 0;
   }
   d->vmax_valid = false;
+  d->since_build = 0;
   invalidate(d);
   return MDGPU_OK;
 }
@@ -1155,6 +1181,8 @@ void rearm_after_check(mdgpu_domain *d) {
   std::memcpy(&d2, d->h_u64 + 1, sizeof d2);
   const double left = budget_after_check(d->margin, d2);
   if (left > 0.0) d->buffer_length = left;
+  d->h_rr[0].measured = 1;  // a run goes on from this displacement
+  d->h_rr[0].dmax2 = d2;
 }
 
 int displacement_check_result(const mdgpu_domain *d, int *expired) {
@@ -1282,11 +1310,15 @@ int is_expired_ensemble(mdgpu_domain *d, int *expired) {
     std::memcpy(&d2, &d->h_chk_dmax[k], sizeof d2);
     const double left = budget_after_check(d->margin, d2);
     if (left > 0.0) d->rst[d->h_which[k]].buffer_length = left;
+    d->h_rr[d->h_which[k]].measured = 1;  // a run goes on from this displacement
+    d->h_rr[d->h_which[k]].dmax2 = d2;
   }
   return MDGPU_OK;
 }
 
 int check_expired(mdgpu_domain *d, int *expired) {
+  d->run_keep = false;
+  for (int r = 0; r < d->nrep; r++) d->h_rr[r].measured = 0;
   return d->nrep == 1 ? is_expired(d, expired) : is_expired_ensemble(d, expired);
 }
 
@@ -1318,13 +1350,15 @@ ForceConstsF fconsts32(const mdgpu_domain *d) {
 
 // The list as the brick kernels read it; lds_cap = staged entries per brick
 // that fit the LDS budget (bricks with more read partners from global memory).
-BrickList brick_list(const mdgpu_domain *d, int bytes_per_entry, bool inner = false) {
+// images: the kernel takes ghost images from their owners (gimg).
+BrickList brick_list(const mdgpu_domain *d, int bytes_per_entry, bool inner = false, bool images = false) {
   BrickList bl;
   bl.nbr = inner ? d->nbr_in : d->nbr;
   bl.code = !list_codes(d) ? nullptr : inner ? d->ncode_in : d->ncode;
   bl.sbase = d->sbase;
   bl.slen = inner ? d->slen_in : d->slen;
   bl.glist = d->glist;
+  bl.gimg = images ? d->gimg : nullptr;
   bl.gbase = d->gbase;
   bl.row0 = d->row0;
   bl.nrow = d->nrow;
@@ -1337,10 +1371,19 @@ BrickList brick_list(const mdgpu_domain *d, int bytes_per_entry, bool inner = fa
   return bl;
 }
 
+// Whether the pipelined FP64 kick runs (it stages through the plain gather list).
+bool pipelined(const mdgpu_domain *d) { return d->precision == MDGPU_FP64 && d->pipeline && d->waves >= 4; }
+
+// Whether the fused step's kick takes the ghost images from their owners'
+// half-drifted positions (the image gather list), rather than from the halo
+// refresh: not in the cell frame, whose FP32 copies of the ghosts the refresh
+// writes, nor in the pipelined kick.  The images have the same bits either way.
+bool fused_images(const mdgpu_domain *d) { return !rel_frame(d) && !pipelined(d) && !d->group; }
+
 template <int W, int U>
 void launch_fp64(mdgpu_domain *d, const double4 *src, double4 *pos_out, int epi, const ForceConsts &fc,
                  const StepClock &sc, double *vb, const NextDrift &nd, bool inner) {
-  const BrickList bl = brick_list(d, 3 * sizeof(double), inner);
+  const BrickList bl = brick_list(d, 3 * sizeof(double), inner, nd.pos != nullptr && fused_images(d));
   const size_t shm = (size_t)bl.lds_cap * 3 * sizeof(double);
   allow_lds(k_force_brick_fp64<W, U>, shm);
   hipLaunchKernelGGL((k_force_brick_fp64<W, U>), dim3(d->nbrick), dim3(kWave * W), shm, d->stream, src, d->mom,
@@ -1385,7 +1428,7 @@ void launch_mixed(mdgpu_domain *d, const double4 *src, const float4 *rel, double
 template <int W, int U, int K>
 void launch_mixed_brick(mdgpu_domain *d, const double4 *src, double4 *pos_out, int epi, const ForceConstsF &f32,
                         double dt2, const StepClock &sc, double *vb, const NextDrift &nd, bool inner) {
-  const BrickList bl = brick_list(d, sizeof(float4), inner);
+  const BrickList bl = brick_list(d, sizeof(float4), inner, nd.pos != nullptr && fused_images(d));
   const size_t shm = (size_t)bl.lds_cap * sizeof(float4);
   const NextDrift nd64{nd.pos, nullptr, nd.cell, nd.org};
   allow_lds(k_force_brick_mixed_brick<W, U, K>, shm);
@@ -1413,7 +1456,7 @@ void launch_force_w(mdgpu_domain *d, const double4 *src, const float4 *rel, doub
                     const ForceConsts &fc, const ForceConstsF &f32, const StepClock &sc, double *vb,
                     const NextDrift &nd, bool in) {
   // groups of kGroup list indices in flight: unroll / kGroup (1, 2 or 4)
-  if (d->precision == MDGPU_FP64 && d->pipeline && W >= 4) {
+  if (pipelined(d) && W >= 4) {
     // compute wavefronts: 14 with 16 requested (two producers make 16), else as requested
     constexpr int WP = W > 14 ? 14 : W;
     if (unroll_of(d) == 16) launch_fp64_pipe<WP, 2>(d, src, pos_out, epi, fc, sc, vb, nd, in);
@@ -1431,6 +1474,19 @@ void launch_force_w(mdgpu_domain *d, const double4 *src, const float4 *rel, doub
   }
 }
 
+RunRules run_rules(const mdgpu_domain *d) {
+  RunRules U;
+  U.dt = d->dt;
+  U.margin = d->margin;
+  U.SL2 = d->SL * d->SL;
+  U.CL2 = d->CL2;
+  U.check = d->disp_check;
+  U.list_cap = d->check_list_length;
+  U.cap = d->run_cap;
+  U.single = d->nrep == 1;
+  return U;
+}
+
 // One pair-force launch.  Rows and partners (owned, and ghosts at
 // [pn, pn + ng)) are read from `src` (`rel` in FP32); `pos_out` receives the
 // drifted (or copied) owned positions; `nd` (optional) the next step's first
@@ -1439,12 +1495,14 @@ void launch_force_w(mdgpu_domain *d, const double4 *src, const float4 *rel, doub
 // (a launch that is captured and replayed).
 int launch_force(mdgpu_domain *d, const double4 *src, const float4 *rel, double4 *pos_out, int epilogue,
                  bool want_vmax, const NextDrift &nd, unsigned long long *clock = nullptr, bool inner = false,
-                 RunGate *gate = nullptr) {
+                 bool gated = false) {
   if (d->pn == 0) return MDGPU_OK;
   hipStream_t st = d->stream;
   const ForceConsts fc = fconsts(d);
   const ForceConstsF f32 = fconsts32(d);
-  const StepClock sc{d->dt, d->step, clock, gate};
+  RunMeasure meas{};
+  if (gated) meas = RunMeasure{d->rr, d->pos_old, d->dpart, d->run_cand, d->run_cap, d->SL};
+  const StepClock sc{d->dt, d->step, clock, gated ? d->gate : nullptr, meas};
   double *vb = want_vmax ? d->bpart : nullptr;
   const int ev0 = d->force_launches * 2;
   const bool ev = d->timing && clock == nullptr && ev0 + 1 < (int)d->ev.size();
@@ -1459,11 +1517,18 @@ int launch_force(mdgpu_domain *d, const double4 *src, const float4 *rel, double4
     HIPCHK(d, hipEventRecord(d->ev[ev0 + 1], st));
     d->force_launches++;
   }
-  if (want_vmax) {
-    hipLaunchKernelGGL(k_replica_max, dim3(d->nrep), dim3(kBlock), 0, st, d->bpart, d->reps, d->rep_v2, clock,
-                       gate);
-    // a run's steps keep the maxima on the device for the next step's gate
-    if (!gate) HIPCHK(d, hipMemcpyAsync(d->h_rep_v2, d->rep_v2, d->nrep * sizeof(double), hipMemcpyDeviceToHost, st));
+  if (want_vmax && gated) {
+    // a run's steps keep the maxima on the device, where the step's end takes
+    // the next step's validity test from them
+    const bool own = d->nrep > kTailReplicas;
+    if (own)
+      hipLaunchKernelGGL(k_run_max, dim3(d->nrep), dim3(kBlock), 0, st, d->gate, d->bpart, d->dpart, d->reps, d->rr);
+    hipLaunchKernelGGL(k_run_tail, dim3(1), dim3(kTailThreads), 0, st, d->gate, own ? nullptr : d->bpart, d->dpart,
+                       d->rr, d->nrep, run_rules(d), d->run_cand, d->reps, d->grng, d->ng, d->clock, d->h_gate,
+                       d->h_rr);
+  } else if (want_vmax) {
+    hipLaunchKernelGGL(k_replica_max, dim3(d->nrep), dim3(kBlock), 0, st, d->bpart, d->reps, d->rep_v2, clock);
+    HIPCHK(d, hipMemcpyAsync(d->h_rep_v2, d->rep_v2, d->nrep * sizeof(double), hipMemcpyDeviceToHost, st));
   }
   return check_launch(d, "force");
 }
@@ -1597,16 +1662,27 @@ int launch_prune(mdgpu_domain *d) {
   return check_launch(d, "prune");
 }
 
-// The fused step's launches.  gated: a step of a run, headed by the validity
-// gate (k_gate), whose launches do nothing once the run has halted.
+// The owned positions at the end of a fused step, from its first half drift
+// `qh`.  After a run (gate): of the last completed step, whose half drift is in
+// qh or qh2, with the images as its halo refresh leaves them where the run's
+// kicks took them from their owners.
+int final_positions(mdgpu_domain *d, const double4 *qh, const double4 *qh2 = nullptr, const RunGate *gate = nullptr) {
+  const int ng = gate && fused_images(d) ? d->ng : 0;
+  hipLaunchKernelGGL(k_final_positions, dim3(nblk((long long)d->pn + ng)), dim3(kBlock), 0, d->stream, d->pos, qh,
+                     qh2, d->mom, d->pn, d->dt * 0.5, d->thermostat == MDGPU_LANGEVIN ? 0 : 1, d->gsrc, d->gcode, ng,
+                     d->reps, gate);
+  return check_launch(d, "final positions");
+}
+
+// The fused step's launches.  gated: a step of a run, whose launches do nothing
+// once the run has halted, and which leaves the halo refresh out where the
+// kick takes the images from their owners (run_gated writes the ghosts once
+// after the run).
 int enqueue_fused(mdgpu_domain *d, unsigned long long *clock, bool prune = false, bool gated = false) {
   hipStream_t st = d->stream;
   const bool mixed = rel_frame(d);
   RunGate *gate = gated ? d->gate : nullptr;
-  if (gated)
-    hipLaunchKernelGGL(k_gate, dim3(1), dim3(kBlock), 0, st, d->gate, d->gbudget, d->glife, d->rep_v2, d->nrep, d->dt,
-                       d->margin);
-  if (d->ng > 0) {
+  if (d->ng > 0 && !(gated && fused_images(d))) {
     if (mixed)
       hipLaunchKernelGGL((k_refresh_from_drifted<true>), dim3(nblk(d->ng)), dim3(kBlock), 0, st, d->pos, d->pos_tmp,
                          d->gsrc, d->gcode, d->pn, d->ng, d->reps, d->cell, d->org, d->rel_tmp, gate);
@@ -1623,12 +1699,8 @@ int enqueue_fused(mdgpu_domain *d, unsigned long long *clock, bool prune = false
   // so that the events time the kernel the runs launch
   const bool timed = d->timing && clock == nullptr && !gated;
   CHK(launch_force(d, d->pos_tmp, d->rel_tmp, gated || timed ? nullptr : d->pos, epi, true, nd, clock,
-                   d->prune_delta > 0.0, gate));
-  if (timed && d->pn > 0) {
-    hipLaunchKernelGGL(k_final_positions, dim3(nblk(d->pn)), dim3(kBlock), 0, st, d->pos, d->pos_tmp, d->mom, d->pn,
-                       d->dt * 0.5, d->thermostat == MDGPU_LANGEVIN ? 0 : 1);
-    CHK(check_launch(d, "final positions"));
-  }
+                   d->prune_delta > 0.0, gated));
+  if (timed && d->pn > 0) CHK(final_positions(d, d->pos_tmp));
   return MDGPU_OK;
 }
 
@@ -1704,6 +1776,22 @@ int rebuild_timed(mdgpu_domain *d) {
   return MDGPU_OK;
 }
 
+// The fused step's first half drift, when the last step's kick has not
+// written it: the owned particles' into pos_tmp, the halo with it.
+int first_half_drift(mdgpu_domain *d) {
+  hipStream_t st = d->stream;
+  const int tot = d->pn + d->ng;
+  if (tot > 0) {
+    if (rel_frame(d))
+      hipLaunchKernelGGL((k_drift_refresh<true>), dim3(nblk(tot)), dim3(kBlock), 0, st, d->pos, d->mom, d->pos_tmp,
+                         d->gsrc, d->gcode, d->pn, d->ng, d->dt * 0.5, d->rep, d->reps, d->cell, d->org, d->rel_tmp);
+    else
+      hipLaunchKernelGGL((k_drift_refresh<false>), dim3(nblk(tot)), dim3(kBlock), 0, st, d->pos, d->mom, d->pos_tmp,
+                         d->gsrc, d->gcode, d->pn, d->ng, d->dt * 0.5, d->rep, d->reps, d->cell, d->org, d->rel_tmp);
+  }
+  return check_launch(d, "drift+refresh");
+}
+
 // MDManager::Calculate (mdmanager.cc:116-148): one step of every replica
 int calculate_step(mdgpu_domain *d) {
   hipStream_t st = d->stream;
@@ -1742,20 +1830,7 @@ int calculate_step(mdgpu_domain *d) {
     // fused: [drift into pos_tmp +] halo refresh, then kick (+ drift or Langevin)
     // whose epilogue also writes the next step's first half drift into pos_next
     const bool mixed = rel_frame(d);
-    if (!d->mid_valid) {
-      const int tot = d->pn + d->ng;
-      if (tot > 0) {
-        if (mixed)
-          hipLaunchKernelGGL((k_drift_refresh<true>), dim3(nblk(tot)), dim3(kBlock), 0, st, d->pos, d->mom,
-                             d->pos_tmp, d->gsrc, d->gcode, d->pn, d->ng, d->dt * 0.5, d->rep, d->reps, d->cell,
-                             d->org, d->rel_tmp);
-        else
-          hipLaunchKernelGGL((k_drift_refresh<false>), dim3(nblk(tot)), dim3(kBlock), 0, st, d->pos, d->mom,
-                             d->pos_tmp, d->gsrc, d->gcode, d->pn, d->ng, d->dt * 0.5, d->rep, d->reps, d->cell,
-                             d->org, d->rel_tmp);
-      }
-      CHK(check_launch(d, "drift+refresh"));
-    }
+    if (!d->mid_valid) CHK(first_half_drift(d));
     // the inner list: pruned again once the motion since the last pruning
     // could have brought a pair from beyond rc + delta to within rc
     bool prune = false;
@@ -1787,67 +1862,84 @@ int calculate_step(mdgpu_domain *d) {
   return MDGPU_OK;
 }
 
-// Whether the next steps may be queued without waiting for the host: fused
-// NVE or Langevin steps (replayed from graphs or launched), no inner list, and the last step
-// a fused one (its maxima of |p|^2 and the next first half drift are on the
-// device).
-bool can_run_ahead(const mdgpu_domain *d) {
-  return d->run_ahead > 0 && !d->timing && d->thermostat != MDGPU_NOSEHOOVER &&
-         !(d->prune_delta > 0.0) && d->initialized && d->mid_valid && d->vmax_valid && d->pn > 0;
+// Whether steps may be queued without waiting for the host: fused NVE or
+// Langevin steps (replayed from graphs or launched), no inner list.
+bool can_run(const mdgpu_domain *d) {
+  return d->run_ahead > 0 && !d->timing && d->thermostat != MDGPU_NOSEHOOVER && !(d->prune_delta > 0.0) && d->pn > 0;
 }
 
 double &budget_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->buffer_length : d->rst[r].buffer_length; }
 int &lifetime_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->lifetime : d->rst[r].lifetime; }
 
-// Steps every validity budget lasts at the last maxima of |p| (0: the next
-// step needs the host).  The maxima change from step to step, so a run may
-// still halt earlier, or end before the budgets do.
-int run_length(mdgpu_domain *d, int limit, int *k) {
-  *k = 0;
-  for (int r = 0; r < d->nrep; r++)
-    if (!(budget_of(d, r) > 0.0)) return MDGPU_OK;  // a displacement check is due: no wait for the maxima
-  CHK(sync(d));  // the last step's maxima
-  double steps = (double)limit;
-  for (int r = 0; r < d->nrep; r++) {
-    const double b = budget_of(d, r);
-    const double v = std::sqrt(d->h_rep_v2[r]);
-    if (v > 0.0) steps = std::min(steps, b / (v * 2.0 * d->dt));
+// Steps to queue at once: as many as the list should still last, by what the
+// last one lasted (a list's life varies little from one to the next), or, for
+// the first, by the budgets at the last maxima of |p|.  A run past its list's
+// end wastes two launches that return at once per step (about 6 us), and one
+// that ends before it costs a wait for the host and the final positions (30 to
+// 80 us), hence at least kRunLeast.
+constexpr int kRunLeast = 8;
+
+int run_length(mdgpu_domain *d, int limit) {
+  int k = d->list_span - d->since_build;
+  if (d->list_span == 0) {
+    double steps = (double)limit;
+    if (!d->vmax_valid) steps = 2.0 * kRunLeast;
+    else
+      for (int r = 0; r < d->nrep; r++) {
+        const double v = std::sqrt(d->h_rep_v2[r]);
+        if (v > 0.0) steps = std::min(steps, budget_of(d, r) / (v * 2.0 * d->dt));
+      }
+    k = (int)std::max(0.0, std::min(steps, (double)limit));
   }
-  if (steps >= 1.0) *k = (int)steps;
-  return MDGPU_OK;
+  return std::min(std::max(k, kRunLeast), std::min(limit, d->run_ahead));
 }
 
-// A run of k fused steps queued at once, each headed by k_gate; *done
-// receives the steps completed, fewer than k when a step's validity test
-// needs the host.  The budgets and lifetimes go to the device before the run
-// and come back after it, as do the last maxima of |p|^2.
-int run_gated(mdgpu_domain *d, int k, int *done) {
+// Steps of a run-capable domain, at most `limit` of them: a run of fused steps
+// queued at once, whose validity tests run on the device (k_run_begin,
+// k_run_tail).  The host decides a step only where a run halted, or when the
+// last operation was no fused step (its maxima of |p|, or its next half drift,
+// which moves the ghosts that the check reads, are not there): the
+// displacement check or the construction that step needs, after which the run
+// goes on with it.  *done receives the steps completed.  The lists' state goes to the device with the
+// run's first launch and comes back with its last (pinned memory both ways).
+int run_steps(mdgpu_domain *d, int limit, int *done) {
   hipStream_t st = d->stream;
   const int R = d->nrep;
   const bool mixed = rel_frame(d);
+  *done = 0;
+  bool approved = false;
+  if (!d->initialized || !d->vmax_valid || !d->mid_valid || d->run_halted) {
+    int expired = 0;
+    CHK(check_expired(d, &expired));
+    d->run_halted = false;
+    if (expired) {
+      if (d->initialized) d->list_span = d->since_build;
+      CHK(rebuild_timed(d));
+    }
+    approved = true;
+  }
+  if (!d->mid_valid) CHK(first_half_drift(d));
+  const int k = run_length(d, limit);
+  const bool keep = d->run_keep && !approved;
   for (int r = 0; r < R; r++) {
-    d->h_gbudget[r] = budget_of(d, r);
-    d->h_glife[r] = lifetime_of(d, r);
+    RunRep &S = d->h_rr[r];
+    S.budget = budget_of(d, r);
+    S.lifetime = lifetime_of(d, r);
+    S.v2 = d->vmax_valid ? d->h_rep_v2[r] : 0.0;
+    if (!approved) S.measured = 0;
   }
-  d->h_gate->halted = 0;
-  d->h_gate->done = 0;
-  HIPCHK(d, hipMemcpyAsync(d->gbudget, d->h_gbudget, R * sizeof(double), hipMemcpyHostToDevice, st));
-  HIPCHK(d, hipMemcpyAsync(d->glife, d->h_glife, R * sizeof(int), hipMemcpyHostToDevice, st));
-  HIPCHK(d, hipMemcpyAsync(d->gate, d->h_gate, sizeof(RunGate), hipMemcpyHostToDevice, st));
-  if (d->clock_dirty) {
-    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, d->clock, (unsigned long long)d->step);
-    d->clock_dirty = false;
-  }
+  d->h_gate->done = -1;
+  hipLaunchKernelGGL(k_run_begin, dim3(1), dim3(kTailThreads), 0, st, d->gate, k, d->rr, d->h_rr, R, run_rules(d),
+                     d->run_cand, d->reps, d->grng, d->ng, approved ? 1 : 0, keep ? 1 : 0, d->clock,
+                     (unsigned long long)d->step, d->h_gate);
+  const double4 *qh = d->pos_tmp, *qh2 = d->pos_next;
   for (int j = 0; j < k; j++) {
     if (d->use_graph) CHK(launch_fused_graph(d, true));
     else CHK(enqueue_fused(d, d->clock, false, true));  // the same launches, each queued directly
     std::swap(d->pos_tmp, d->pos_next);
     if (mixed) std::swap(d->rel_tmp, d->rel_next);
   }
-  HIPCHK(d, hipMemcpyAsync(d->h_gate, d->gate, sizeof(RunGate), hipMemcpyDeviceToHost, st));
-  HIPCHK(d, hipMemcpyAsync(d->h_gbudget, d->gbudget, R * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHK(d, hipMemcpyAsync(d->h_glife, d->glife, R * sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPCHK(d, hipMemcpyAsync(d->h_rep_v2, d->rep_v2, R * sizeof(double), hipMemcpyDeviceToHost, st));
+  CHK(final_positions(d, qh, qh2, d->gate));
   CHK(sync(d));
   const int n = d->h_gate->done;
   if (n < 0 || n > k) {
@@ -1858,17 +1950,18 @@ int run_gated(mdgpu_domain *d, int k, int *done) {
     std::swap(d->pos_tmp, d->pos_next);
     if (mixed) std::swap(d->rel_tmp, d->rel_next);
   }
-  for (int r = 0; r < R; r++) {
-    budget_of(d, r) = d->h_gbudget[r];
-    lifetime_of(d, r) = d->h_glife[r];
-  }
-  if (n > 0 && d->pn > 0) {
-    // the final owned positions of the last completed step, whose first half
-    // drift is now in pos_next (the next step's is in pos_tmp)
-    hipLaunchKernelGGL(k_final_positions, dim3(nblk(d->pn)), dim3(kBlock), 0, st, d->pos, d->pos_next, d->mom,
-                       d->pn, d->dt * 0.5, d->thermostat == MDGPU_LANGEVIN ? 0 : 1);
-    CHK(check_launch(d, "final positions"));
-  }
+  if (n > 0)
+    for (int r = 0; r < R; r++) {
+      budget_of(d, r) = d->h_rr[r].budget;
+      lifetime_of(d, r) = d->h_rr[r].lifetime;
+      d->h_rep_v2[r] = d->h_rr[r].v2;
+    }
+  d->run_halted = d->h_gate->halted != 0;
+  d->run_keep = !d->run_halted;
+  d->mid_valid = true;
+  if (n > 0) d->vmax_valid = true;
+  d->clock_dirty = false;
+  d->since_build += n;
   for (int j = 0; j < n; j++) {
     d->sim_time += d->dt;
     d->step++;
@@ -2017,11 +2110,15 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
       for (int k = 0; k < 3; k++) R.bd[k] = d->bd[k];
     }
   }
+  // room for the candidates of the runs' displacement tests (a replica that has
+  // more leaves the test to the host), 64 MB at most over all replicas
+  d->run_cap = std::max(1, std::min(kRunCands, (1 << 20) / nrep));
   int r;
   if ((r = dalloc(d, &d->reps, nrep)) || (r = dalloc(d, &d->rep_v2, nrep)) || (r = dalloc(d, &d->rep_out, 3 * nrep)) ||
       (r = dalloc(d, &d->which, nrep)) || (r = dalloc(d, &d->rep_exp, nrep)) || (r = dalloc(d, &d->grng, nrep)) ||
       (r = dalloc(d, &d->clock, 1)) || (r = dalloc(d, &d->chk_dmax, nrep)) || (r = dalloc(d, &d->chk_cnt, nrep)) ||
-      (r = dalloc(d, &d->gate, 1)) || (r = dalloc(d, &d->gbudget, nrep)) || (r = dalloc(d, &d->glife, nrep)) ||
+      (r = dalloc(d, &d->gate, 1)) || (r = dalloc(d, &d->rr, nrep)) ||
+      (r = dalloc(d, &d->run_cand, (size_t)nrep * d->run_cap)) ||
       (r = dalloc(d, &d->chk_cand, (size_t)nrep * d->check_list_length)) ||
       (r = dalloc(d, &d->rep_factor, nrep))) {
     mdgpu_destroy(d);
@@ -2032,8 +2129,7 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
       hipHostMalloc((void **)&d->h_which, nrep * sizeof(int)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_rep_exp, nrep * sizeof(int)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_gate, sizeof(RunGate)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_gbudget, nrep * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_glife, nrep * sizeof(int)) != hipSuccess ||
+      hipHostMalloc((void **)&d->h_rr, nrep * sizeof(RunRep)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_rep_factor, nrep * sizeof(double)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_chk_dmax, nrep * sizeof(unsigned long long)) != hipSuccess) {
     mdgpu_destroy(d);
@@ -2062,6 +2158,8 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
     mdgpu_destroy(d);
     return MDGPU_ERR_HIP;
   }
+  std::memset(d->h_rr, 0, nrep * sizeof(RunRep));
+  (void)hipMemset(d->rr, 0, nrep * sizeof(RunRep));
   (void)hipMemset(d->i32, 0, 4 * sizeof(int));
   (void)hipMemset(d->u64, 0, 4 * sizeof(unsigned long long));
   (void)hipMemset(d->clock, 0, sizeof(unsigned long long));
@@ -2582,7 +2680,7 @@ int group_temperature(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, do
 // workgroup does what the unit's own kick does to that brick.
 template <int W, int U>
 void launch_group_kick(mdgpu_domain *d, const UnitKicks &uk, int nb, size_t shm) {
-  const StepClock sc{d->dt, d->step, nullptr, nullptr};
+  const StepClock sc{d->dt, d->step, nullptr, nullptr, RunMeasure{}};
   if (d->precision == MDGPU_FP64) {
     allow_lds(k_force_group_fp64<W, U>, shm);
     hipLaunchKernelGGL((k_force_group_fp64<W, U>), dim3(nb), dim3(kWave * W), shm, d->stream, uk, fconsts(d), sc);
@@ -2950,7 +3048,7 @@ int mdgpu_destroy(mdgpu_domain *d) {
                   d->i32,     d->d3,          d->reps,        d->brep,      d->rep,      d->rep_alt,
                   d->grng,    d->rep_v2,      d->rep_out,     d->which,     d->rep_exp,  d->clock,
                   d->perm_in, d->nbr_in,      d->ncode_in,    d->slen_in,   d->chk_dmax, d->chk_cnt,
-                  d->chk_cand, d->gate,       d->gbudget,     d->glife,     d->xfer,     d->gunit,
+                  d->chk_cand, d->gate,       d->gimg,       d->rr,          d->run_cand,  d->dpart,     d->xfer,     d->gunit,
                   d->st_pos,  d->st_mom,      d->st_id,       d->src_tab,   d->ucnt,     d->uoff,
                   d->rep_factor};
   for (StepGraph &g : d->graphs) drop_graph(g);
@@ -2958,7 +3056,7 @@ int mdgpu_destroy(mdgpu_domain *d) {
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   for (void *h : {(void *)d->h_rep_v2, (void *)d->h_rep_out, (void *)d->h_which, (void *)d->h_rep_exp,
-                  (void *)d->h_gate, (void *)d->h_gbudget, (void *)d->h_glife, (void *)d->h_rep_factor,
+                  (void *)d->h_gate, (void *)d->h_rr, (void *)d->h_rep_factor,
                   (void *)d->h_chk_dmax})
     if (h) (void)hipHostFree(h);
   if (d->h_u64) (void)hipHostFree(d->h_u64);
@@ -3275,21 +3373,11 @@ int mdgpu_calculate(mdgpu_domain *d, int nsteps, int *rebuilds) {
   int r = MDGPU_OK;
   int s = 0;
   while (s < nsteps && r == MDGPU_OK) {
-    // steps whose validity the budgets settle run ahead of the host; a step
-    // that needs the host (the displacement check, a construction, an error)
-    // is taken here, one at a time
-    if (can_run_ahead(d) && nsteps - s > 1) {
-      int k = 0;
-      r = run_length(d, std::min(nsteps - s, d->run_ahead), &k);
-      if (r != MDGPU_OK) break;
-      if (k > 0) {
-        int done = 0;
-        r = run_gated(d, k, &done);
-        s += done;
-        if (r != MDGPU_OK || done == k) continue;
-      }
-    }
-    if (s < nsteps) {
+    if (can_run(d)) {
+      int done = 0;
+      r = run_steps(d, nsteps - s, &done);
+      s += done;
+    } else {
       r = calculate_step(d);
       s++;
     }

@@ -130,11 +130,32 @@ __global__ void k_drift_refresh(double4 *__restrict__ pos, const double4 *__rest
 // half drift qh and final momenta: qh + p dt/2 (drift) or qh (Langevin), the
 // operations and roundings of the kick's epilogue (finish_row).  A run's steps
 // leave them out, since no step of the run reads them; the host writes them
-// once after the run, from the last completed step.
+// once after the run, from the last completed step.  With ng > 0 also the
+// ghosts [pn, pn + ng) as that step's halo refresh would have left them
+// (SendBorderParticles: qh of the owner plus its shift), where the run's kicks
+// took the images from their owners.
+//
+// The half drifts of a run's steps alternate between two buffers, the first
+// step's in qh and the second's in qh2, so the count of completed steps (gate)
+// says where the last one's is; gate == nullptr: qh.
 __global__ void k_final_positions(double4 *__restrict__ pos, const double4 *__restrict__ qh,
-                                  const double4 *__restrict__ mom, int pn, double dt2, int drift) {
+                                  const double4 *__restrict__ qh2, const double4 *__restrict__ mom, int pn,
+                                  double dt2, int drift, const int *__restrict__ gsrc, const int *__restrict__ gcode,
+                                  int ng, const Replica *__restrict__ reps, const RunGate *__restrict__ gate) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= pn) return;
+  if (gate != nullptr) {
+    const int done = gate->done;
+    if (done == 0) return;
+    if (!(done & 1)) qh = qh2;
+  }
+  if (i >= pn) {
+    const int k = i - pn;
+    if (k >= ng) return;
+    const int w = gcode[k];
+    const double3 y = image_of(qh[gsrc[k]], ghost_shift(w), reps[ghost_rep(w)].L);
+    pos[i] = make_double4(y.x, y.y, y.z, 0.0);
+    return;
+  }
   double4 q = qh[i];
   if (drift) {
     const double4 p = mom[i];
@@ -396,73 +417,319 @@ __device__ __forceinline__ double block_sum0(double v) {
   return t;  // valid in thread 0
 }
 
-// Largest per-brick value of each replica: out[r] = max of part over the
-// replica's bricks (the force kernel's maxima of |p|^2).  clock (optional) is
-// the step counter of the fused step; it advances by one here.
-__global__ __launch_bounds__(kBlock) void k_replica_max(const double *__restrict__ part,
-                                                        const Replica *__restrict__ reps, double *__restrict__ out,
-                                                        unsigned long long *__restrict__ clock,
-                                                        RunGate *__restrict__ gate) {
-  if (run_halted(gate)) return;
-  const Replica &R = reps[blockIdx.x];
-  const int b0 = R.brick0, nb = replica_bricks(R);
-  double m0 = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;  // four loads in flight per thread
-  int k = threadIdx.x;
-  for (; k + 3 * kBlock < nb; k += 4 * kBlock) {
-    const double a = part[b0 + k], b = part[b0 + k + kBlock];
-    const double c = part[b0 + k + 2 * kBlock], e = part[b0 + k + 3 * kBlock];
+// Largest per-brick value of a replica (the force kernel's maxima of |p|^2),
+// by the T lanes `t` of a workgroup or wavefront; four loads in flight per lane.
+__device__ __forceinline__ double replica_part_max(const double *__restrict__ part, int b0, int nb, int t, int T) {
+  double m0 = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
+  int k = t;
+  for (; k + 3 * T < nb; k += 4 * T) {
+    const double a = part[b0 + k], b = part[b0 + k + T];
+    const double c = part[b0 + k + 2 * T], e = part[b0 + k + 3 * T];
     m0 = fmax(m0, a);
     m1 = fmax(m1, b);
     m2 = fmax(m2, c);
     m3 = fmax(m3, e);
   }
-  for (; k < nb; k += kBlock) m0 = fmax(m0, part[b0 + k]);
-  double m = fmax(fmax(m0, m1), fmax(m2, m3));
-  m = block_max_all(m);
+  for (; k < nb; k += T) m0 = fmax(m0, part[b0 + k]);
+  return fmax(fmax(m0, m1), fmax(m2, m3));
+}
+
+// out[r] = max of part over each replica's bricks, one workgroup per replica.
+// clock (optional) is the step counter of the fused step; it advances by one
+// here.
+__global__ __launch_bounds__(kBlock) void k_replica_max(const double *__restrict__ part,
+                                                        const Replica *__restrict__ reps, double *__restrict__ out,
+                                                        unsigned long long *__restrict__ clock) {
+  const Replica &R = reps[blockIdx.x];
+  const double m = block_max_all(replica_part_max(part, R.brick0, replica_bricks(R), threadIdx.x, kBlock));
   if (threadIdx.x == 0) {
     out[blockIdx.x] = m;
     if (clock != nullptr && blockIdx.x == 0) clock[0] = clock[0] + 1ull;
-    if (gate != nullptr && blockIdx.x == 0) gate->done = gate->done + 1;
   }
 }
 
-// PairList::IsPairListExpired with UpdatePairListValidity (pairlist.cc:26-65)
-// for the next step of a run, every replica at once: the lifetime counts up
-// and a budget still positive shrinks by 2 max|p| dt, from the replica's
-// max |p|^2 after the last step (v2).  When some replica's particles are too
-// fast or its budget ends below zero, nothing is committed and the run halts:
-// the host takes that step (and its displacement check) from the same values.
-// One workgroup.
-__device__ __forceinline__ bool gate_budget(double v2, double dt, double margin, double &b) {
+// The maxima of a run's step into its replicas' RunRep, one workgroup per
+// replica (k_run_tail's first part, for kTailReplicas replicas and more).
+__global__ __launch_bounds__(kBlock) void k_run_max(const RunGate *__restrict__ gate, const double *__restrict__ part,
+                                                    const double *__restrict__ dpart,
+                                                    const Replica *__restrict__ reps, RunRep *__restrict__ rr) {
+  if (run_halted(gate)) return;
+  const int r = blockIdx.x;
+  const Replica &R = reps[r];
+  const double m = block_max_all(replica_part_max(part, R.brick0, replica_bricks(R), threadIdx.x, kBlock));
+  if (threadIdx.x == 0) rr[r].v2 = m;
+  if (!rr[r].measured) return;
+  __syncthreads();
+  const double dm = block_max_all(replica_part_max(dpart, R.brick0, replica_bricks(R), threadIdx.x, kBlock));
+  if (threadIdx.x == 0) rr[r].dmax2 = dm;
+}
+
+// What the validity test of a run's steps depends on besides the replicas.
+struct RunRules {
+  double dt, margin, SL2, CL2;
+  int check;       // the displacement check (MDGPU_OPT_DISPLACEMENT_CHECK)
+  int list_cap;    // CheckListLength
+  int cap;         // room for candidates per replica
+  int single;      // one replica
+};
+
+// PairList::UpdatePairListValidity (pairlist.cc:48-65) for the next step of a
+// run: a budget still positive shrinks by 2 max|p| dt, from the replica's max
+// |p|^2 after the last step (v2).  False: particles too fast.
+__device__ __forceinline__ bool run_budget(double v2, double dt, double margin, double &b) {
   if (b > 0.0) {
     const double vmax = sqrt(v2);
-    if (vmax * 2.0 * dt > margin) return true;
+    if (vmax * 2.0 * dt > margin) return false;
     b = b - vmax * 2.0 * dt;
   }
-  return b < 0.0;
+  return true;
 }
 
-__global__ __launch_bounds__(kBlock) void k_gate(RunGate *__restrict__ gate, double *__restrict__ budget,
-                                                 int *__restrict__ lifetime, const double *__restrict__ v2,
-                                                 int nrep, double dt, double margin) {
-  __shared__ int stop;
+// A list whose displacements were measured after the last step, the largest
+// squared one dmax2, takes a budget again while none has reached half the
+// margin: no entry is then displaced by more than margin - max displacement,
+// so CheckByDisplacement (pairlist.cc:68-121) has no candidate and passes.
+__device__ __forceinline__ double run_rearm(double margin, double dmax2) { return margin - 2.0 * sqrt(dmax2); }
+
+constexpr int kTailThreads = 1024;
+constexpr int kRunCands = 1024;   // entries a replica keeps at most (those above its threshold)
+constexpr int kWaveCands = 64;    // entries one wavefront tests by itself
+constexpr int kGroupCands = 512;  // candidates the whole workgroup tests for one replica
+
+// Shared memory of run_gate: the outcome, the replicas whose candidates are to
+// be tested, and those candidates (position at the construction and now),
+// kWaveCands per wavefront or all of one replica's.
+struct RunShared {
+  int stop, nq, count;
+  int queue[kTailThreads];
+  double c[6][kTailThreads / kWave * kWaveCands];
+};
+static_assert(kTailThreads / kWave * kWaveCands >= kGroupCands, "a replica's candidates fit");
+
+// CheckByDisplacement's last part for one replica, by the T lanes t of a
+// wavefront or workgroup: true when a pair of candidates was beyond SL at the
+// construction and is now inside rc.  The m candidates are at sh.c[.][base..].
+// Candidate a = t % A (A: m rounded up to a power of two) meets every
+// (T / A)-th of those before it, so a pair costs a few LDS reads and no
+// division; read from memory, pair by pair, 300 candidates took 100 us.
+__device__ __forceinline__ bool run_pair_expired(const RunShared &sh, int base, int m, double SL2, double CL2, int t,
+                                                 int T) {
+  int A = 1;
+  while (A < m) A <<= 1;
+  const int a = t & (A - 1), S = T / A;
+  if (a >= m) return false;
+  const double x = sh.c[3][base + a], y = sh.c[4][base + a], z = sh.c[5][base + a];
+  bool hit = false;
+  for (int b = t / A; b < a; b += S) {
+    const double dx = sh.c[3][base + b] - x, dy = sh.c[4][base + b] - y, dz = sh.c[5][base + b] - z;
+    if (!(dx * dx + dy * dy + dz * dz < CL2)) continue;
+    const double ex = sh.c[0][base + b] - sh.c[0][base + a], ey = sh.c[1][base + b] - sh.c[1][base + a],
+                 ez = sh.c[2][base + b] - sh.c[2][base + a];
+    hit = hit || !(ex * ex + ey * ey + ez * ez < SL2);
+  }
+  return hit;
+}
+
+__device__ __forceinline__ void run_put_cand(RunShared &sh, int at, const RunCand &C) {
+  sh.c[0][at] = C.old.x;
+  sh.c[1][at] = C.old.y;
+  sh.c[2][at] = C.old.z;
+  sh.c[3][at] = C.now.x;
+  sh.c[4][at] = C.now.y;
+  sh.c[5][at] = C.now.z;
+}
+
+// PairList::IsPairListExpired (pairlist.cc:26-45) for the next step of a run,
+// every replica at once, from the maxima of the last step: true when the step
+// may go on, its budgets and lifetimes then committed; false when it needs the
+// host (an expired list, a particle too fast, or a test this step was not
+// measured for), with nothing committed.  The host decides such a step from
+// the same state with the same tests.  `approved`: the host has decided the
+// step already.  Either way the next step's measurement is planned: it takes
+// displacements when its budget is nearly spent, and keeps as candidates
+// what is displaced by more than margin - (the largest displacement it can
+// reach), which the test checks against what it did reach.  One workgroup of
+// kTailThreads.
+__device__ __forceinline__ bool run_gate(RunRep *rr, int nrep, const RunRules &U, const RunCand *cand,
+                                         const Replica *__restrict__ reps, const int2 *__restrict__ grng, int ng,
+                                         bool approved, RunShared &sh) {
+  if (threadIdx.x == 0) sh.stop = sh.nq = 0;
+  __syncthreads();
+  if (!approved) {
+    for (int r = threadIdx.x; r < nrep; r += kTailThreads) {
+      const RunRep S = rr[r];
+      double b = S.budget;
+      bool ok = run_budget(S.v2, U.dt, U.margin, b);
+      if (ok && b < 0.0) {
+        ok = U.check && S.measured;
+        if (ok && !(run_rearm(U.margin, S.dmax2) > 0.0)) {
+          // every entry displaced by more than margin - max displacement is there
+          ok = U.margin - sqrt(S.dmax2) >= S.cthr && S.ncand <= U.cap;
+          const int q = ok ? atomicAdd(&sh.nq, 1) : 0;
+          ok = ok && q < kTailThreads;
+          if (ok) sh.queue[q] = r;
+        }
+      }
+      if (!ok) sh.stop = 1;
+    }
+    __syncthreads();
+    if (!sh.stop && sh.nq > 0) {  // uniform
+      const int nq = sh.nq;
+      __syncthreads();
+      const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+      // few entries: a wavefront per replica
+      for (int q = wv; q < nq; q += kTailThreads / kWave) {
+        const int r = sh.queue[q], kept = rr[r].ncand;
+        if (kept > kWaveCands) continue;
+        const double c = U.margin - sqrt(rr[r].dmax2);
+        RunCand C{};
+        if (lane < kept) C = cand[(size_t)r * U.cap + lane];
+        const bool in = lane < kept && C.old.w > c * c;
+        const unsigned long long w = __ballot(in);
+        const int m = __popcll(w);
+        if (in) run_put_cand(sh, wv * kWaveCands + __popcll(w & ((1ull << lane) - 1ull)), C);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the other lanes' candidates
+        __builtin_amdgcn_wave_barrier();
+        const int n = reps[r].pn + (U.single ? ng : grng[r].y);
+        if ((m > 0 && m >= min(n, U.list_cap)) ||
+            run_pair_expired(sh, wv * kWaveCands, m, U.SL2, U.CL2, lane, kWave))
+          sh.stop = 1;
+      }
+      // many: the whole workgroup, one replica after another
+      for (int q = 0; q < nq; q++) {
+        const int r = sh.queue[q], kept = rr[r].ncand;
+        if (kept <= kWaveCands) continue;
+        const double c = U.margin - sqrt(rr[r].dmax2);
+        __syncthreads();
+        if (threadIdx.x == 0) sh.count = 0;
+        __syncthreads();
+        for (int k = threadIdx.x; k < kept; k += kTailThreads) {
+          const RunCand C = cand[(size_t)r * U.cap + k];
+          if (!(C.old.w > c * c)) continue;
+          const int at = atomicAdd(&sh.count, 1);
+          if (at < kGroupCands) run_put_cand(sh, at, C);
+        }
+        __syncthreads();
+        const int m = sh.count, n = reps[r].pn + (U.single ? ng : grng[r].y);
+        if (m > kGroupCands || (m > 0 && m >= min(n, U.list_cap)) ||
+            run_pair_expired(sh, 0, m, U.SL2, U.CL2, threadIdx.x, kTailThreads))
+          sh.stop = 1;
+      }
+    }
+    __syncthreads();
+    if (sh.stop) return false;
+  }
+  for (int r = threadIdx.x; r < nrep; r += kTailThreads) {
+    RunRep S = rr[r];
+    if (!approved) {
+      run_budget(S.v2, U.dt, U.margin, S.budget);
+      if (S.budget < 0.0) {
+        const double left = run_rearm(U.margin, S.dmax2);
+        if (left > 0.0) S.budget = left;
+      }
+      S.lifetime++;
+    }
+    // the next step, measured from two tests before the budget is spent (2
+    // max|p| dt each, a little more if max|p| grows), so that the step that
+    // spends it knows what its displacements can reach: no displacement grows
+    // by more than max|p| dt
+    const double v = sqrt(S.v2), reach = sqrt(S.dmax2) + 1.05 * v * U.dt;
+    const bool bound = S.measured && reach < U.margin;
+    S.cthr = bound ? U.margin - reach : 1.0e200;
+    S.measured = !(S.budget > 4.5 * v * U.dt);
+    S.ncand = 0;
+    rr[r] = S;
+  }
+  return true;
+}
+
+// A run of `left` steps begins: its replicas' budgets, lifetimes and maxima
+// from the host's copies (pinned memory, read here), the step counter, and the
+// first step's validity test (run_gate), unless the host has decided that step
+// (`approved`).  keep: the displacements that the last run's last step
+// measured still hold.  host: where the outcome goes when the run ends here.
+__global__ __launch_bounds__(kTailThreads) void k_run_begin(RunGate *gate, int left, RunRep *rr,
+                                                            const RunRep *__restrict__ from, int nrep, RunRules U,
+                                                            const RunCand *cand, const Replica *__restrict__ reps,
+                                                            const int2 *__restrict__ grng, int ng, int approved,
+                                                            int keep, unsigned long long *clock,
+                                                            unsigned long long step, RunGate *host) {
+  __shared__ RunShared sh;
+  for (int r = threadIdx.x; r < nrep; r += kTailThreads) {
+    rr[r].budget = from[r].budget;
+    rr[r].v2 = from[r].v2;
+    rr[r].lifetime = from[r].lifetime;
+    if (!keep) {  // the displacements the host has checked, if it has
+      rr[r].measured = from[r].measured;
+      rr[r].dmax2 = from[r].dmax2;
+    }
+  }
+  __syncthreads();
+  const bool go = run_gate(rr, nrep, U, cand, reps, grng, ng, approved != 0, sh);
+  if (threadIdx.x == 0) {
+    const RunGate G{go ? 0 : 1, 0, left};
+    *gate = G;
+    if (!go) *host = G;
+    clock[0] = step;
+  }
+}
+
+// The end of a run's step: each replica's max |p|^2 (and, measured, largest
+// displacement) from its bricks' maxima, the step counted, and, when the run
+// has further steps, the next one's validity test (run_gate), which halts the
+// run where the host is needed.  The outcome of a run that ends here goes to
+// the host's pinned copies (host, to).  One workgroup, the whole of it over
+// the bricks of a single replica, or a wavefront per replica: one launch in
+// place of the maxima's and the next step's gate, whose cost per step is their
+// launches (4.6 + 4.3 us and a gap, against 4.6).  From kTailReplicas replicas
+// on, a wavefront would take more than 8 of them in turn, about 1 us each: the
+// maxima then have a launch of their own with a workgroup per replica
+// (k_run_max) and part is nullptr here.
+constexpr int kTailReplicas = 128;
+
+__global__ __launch_bounds__(kTailThreads) void k_run_tail(RunGate *gate, const double *__restrict__ part,
+                                                           const double *__restrict__ dpart, RunRep *rr, int nrep,
+                                                           RunRules U, const RunCand *cand,
+                                                           const Replica *__restrict__ reps,
+                                                           const int2 *__restrict__ grng, int ng,
+                                                           unsigned long long *clock, RunGate *host, RunRep *to) {
+  __shared__ RunShared sh;
   if (gate->halted) return;
-  if (threadIdx.x == 0) stop = 0;
-  __syncthreads();
-  for (int r = threadIdx.x; r < nrep; r += kBlock) {
-    double b = budget[r];
-    if (gate_budget(v2[r], dt, margin, b)) stop = 1;
+  const int left = gate->left - 1, done = gate->done + 1;
+  if (part == nullptr) {
+    // the maxima are in rr
+  } else if (nrep == 1) {
+    const int b0 = reps[0].brick0, nb = replica_bricks(reps[0]);
+    const double m = block_max_all<kTailThreads>(replica_part_max(part, b0, nb, threadIdx.x, kTailThreads));
+    if (threadIdx.x == 0) rr[0].v2 = m;
+    if (rr[0].measured) {
+      __syncthreads();
+      const double dm = block_max_all<kTailThreads>(replica_part_max(dpart, b0, nb, threadIdx.x, kTailThreads));
+      if (threadIdx.x == 0) rr[0].dmax2 = dm;
+    }
+  } else {
+    for (int r = threadIdx.x / kWave; r < nrep; r += kTailThreads / kWave) {
+      const int b0 = reps[r].brick0, nb = replica_bricks(reps[r]);
+      const double m = wave_max(replica_part_max(part, b0, nb, threadIdx.x % kWave, kWave));
+      const double dm =
+          rr[r].measured ? wave_max(replica_part_max(dpart, b0, nb, threadIdx.x % kWave, kWave)) : 0.0;
+      if (threadIdx.x % kWave == 0) {
+        rr[r].v2 = m;
+        if (rr[r].measured) rr[r].dmax2 = dm;
+      }
+    }
   }
   __syncthreads();
-  if (stop) {
-    if (threadIdx.x == 0) gate->halted = 1;
-    return;
+  const bool go = left == 0 || run_gate(rr, nrep, U, cand, reps, grng, ng, false, sh);
+  if (threadIdx.x == 0) {
+    const RunGate G{go ? 0 : 1, done, left};
+    *gate = G;
+    clock[0] = clock[0] + 1ull;
+    if (left == 0 || !go) *host = G;
   }
-  for (int r = threadIdx.x; r < nrep; r += kBlock) {
-    double b = budget[r];
-    gate_budget(v2[r], dt, margin, b);
-    budget[r] = b;
-    lifetime[r] = lifetime[r] + 1;
+  if (left == 0 || !go) {
+    __syncthreads();
+    for (int r = threadIdx.x; r < nrep; r += kTailThreads) to[r] = rr[r];
   }
 }
 

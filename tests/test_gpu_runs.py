@@ -1,0 +1,89 @@
+"""Runs of steps queued ahead of the host (MDGPU_OPT_RUN_AHEAD) against the same steps taken one
+at a time: the validity tests that the device does inside a run, displacement checks and candidate
+pairs included, must leave the constructions, the state and the time as the host's tests do."""
+import math
+
+import numpy as np
+import pytest
+
+from mdacp_amd import mdgpu
+from mdacp_amd.ensemble import build
+
+pytestmark = pytest.mark.gpu
+
+
+def replicas(n, k_of, rho_of):
+    rows = [dict(k=k_of(r), N=4 * k_of(r) ** 3, rho=rho_of(r), T=0.8 + 0.07 * (r % 9), seed=100 + r) for r in range(n)]
+    return build(rows), np.array([row["T"] for row in rows])
+
+
+# name: replicas, cells per axis, density, options
+CASES = {
+    # uneven replicas, each with its own budget, checks and candidates
+    "six": dict(n=6, k_of=lambda r: 4 + r, rho_of=lambda r: 0.35 + 0.08 * r),
+    # one replica of an ensemble: the whole workgroup on it
+    "one": dict(n=1, k_of=lambda r: 8, rho_of=lambda r: 0.5),
+    # lists that expire by the number of candidates alone
+    "few candidates": dict(n=4, k_of=lambda r: 5 + r % 2, rho_of=lambda r: 0.6, cap=5),
+    # more replicas than one launch takes the maxima of, and more than its wavefronts
+    "many": dict(n=131, k_of=lambda r: 3, rho_of=lambda r: 0.30 + 0.001 * r, steps=(1, 60), rebuilds=1),
+    # lists that expire with their budgets
+    "no check": dict(n=5, k_of=lambda r: 4 + r % 3, rho_of=lambda r: 0.5, check=0),
+}
+
+
+@pytest.mark.parametrize("thermostat,precision", [(mdgpu.NVE, mdgpu.FP64), (mdgpu.LANGEVIN, mdgpu.FP64),
+                                                  (mdgpu.LANGEVIN, mdgpu.MIXED)])
+@pytest.mark.parametrize("name", list(CASES))
+def test_runs_of_an_ensemble_match_single_steps(name, thermostat, precision):
+    c = CASES[name]
+    print("case:", name, thermostat, precision, flush=True)
+    (boxes, counts, q, p, ids), T = replicas(c["n"], c["k_of"], c["rho_of"])
+    es = []
+    for ahead in (64, 0):
+        e = mdgpu.Ensemble(boxes, counts, q, p, ids, T=T, gamma=1.0, seed=np.arange(len(T)) + 5,
+                           thermostat=thermostat, dt=0.005, precision=precision, check_list_length=c.get("cap", 500))
+        e.set_option(mdgpu.OPT_RUN_AHEAD, ahead)
+        e.set_option(mdgpu.OPT_DISPLACEMENT_CHECK, c.get("check", 1))
+        es.append(e)
+    a, b = es
+    ra = rb = 0
+    for chunk in c.get("steps", (1, 37, 2, 100)):
+        ra += a.calculate(chunk)
+        rb += b.calculate(chunk)
+        assert ra == rb, (chunk, ra, rb)
+        for x, y in zip(a.particles(), b.particles()):
+            assert np.array_equal(x, y), chunk
+        for x, y in zip(a.observe_replicas_raw(), b.observe_replicas_raw()):
+            assert np.array_equal(x, y), chunk  # the images are those the last halo refresh left
+    assert ra >= c.get("rebuilds", 2), ra
+    assert a.time() == b.time()
+    for e in es:
+        e.close()
+
+
+@pytest.mark.parametrize("cap", [500, 4])
+def test_runs_of_a_domain_match_single_steps(cap):
+    """A box a few cells wide, uneven, whose lists live long past their budgets."""
+    print("case: domain, candidates up to", cap, flush=True)
+    (boxes, counts, q, p, ids), _ = replicas(1, lambda r: 7, lambda r: 0.45)
+    L = boxes[0] * np.array([1.0, 1.1, 0.97])
+    q = q * np.array([1.0, 1.1, 0.97])
+    ds = []
+    for ahead in (64, 0):
+        d = mdgpu.Domain(L, dt=0.002, capacity=len(q), check_list_length=cap)
+        d.add_particles(q, p * math.sqrt(1.3), ids)
+        d.set_option(mdgpu.OPT_RUN_AHEAD, ahead)
+        ds.append(d)
+    a, b = ds
+    ra = rb = 0
+    for chunk in (1, 90, 3, 160):
+        ra += a.calculate(chunk)
+        rb += b.calculate(chunk)
+        assert ra == rb, (chunk, ra, rb)
+        for x, y in zip(a.particles() + a.ghosts(), b.particles() + b.ghosts()):
+            assert np.array_equal(x, y), chunk
+    assert ra >= 4, ra
+    assert a.time() == b.time()
+    for d in ds:
+        d.close()
