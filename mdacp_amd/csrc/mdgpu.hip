@@ -820,7 +820,16 @@ long long axis_staged_cells(int ms, int bd) {
 // the fraction `fill` of kb KiB of LDS (positions, 24 B per staged entry),
 // the ones that stage the fewest cells in all (ties: fewer bricks).  Staging
 // the neighbourhood is the per-brick overhead of the search and force kernels.
+// A box too small to give every CU a workgroup that way takes smaller bricks:
+// the ones that stage the fewest cells among those that reach kBrickFill of
+// the CUs (shared out over the replicas), or, smaller still, the most bricks
+// there are.  With 8 bricks of 5x5x3 cells on 256 CUs a kick of 2,048
+// particles took 15.5 us, with 216 of one cell 12.3 (8,000 particles: 22.1
+// and 14.3; 32,000: 23.5 and 15.6), a construction 360 and 290 us.
+constexpr double kBrickFill = 0.9;
+
 void auto_brick(const mdgpu_domain *d, double rho, const double L[3], int kb, int bd[3], double fill) {
+  const long long least = (long long)(kBrickFill * d->num_cu / d->nrep);
   const double budget = fill * std::min(kb, d->lds_max_kb) * 1024.0;
   int ms[3];
   double vol = 1.0;
@@ -828,7 +837,7 @@ void auto_brick(const mdgpu_domain *d, double rho, const double L[3], int kb, in
     ms[k] = std::max(1, (int)(L[k] / d->SL));
     vol *= L[k] / ms[k];
   }
-  long long best = -1, best_n = 0;
+  long long best = -1, best_n = 0, best_lacks = 0;
   for (int k = 0; k < 3; k++) bd[k] = 1;
   for (int bz = 1; bz <= kMaxBrickEdge; bz++)
     for (int by = 1; by <= kMaxBrickEdge; by++)
@@ -841,7 +850,10 @@ void auto_brick(const mdgpu_domain *d, double rho, const double L[3], int kb, in
           staged *= axis_staged_cells(ms[k], e[k]);
           n *= (ms[k] + e[k]) / e[k];
         }
-        if (best < 0 || staged < best || (staged == best && n < best_n)) {
+        const long long lacks = std::max(0ll, least - n);
+        if (best < 0 || lacks < best_lacks ||
+            (lacks == best_lacks && (staged < best || (staged == best && n < best_n)))) {
+          best_lacks = lacks;
           best = staged;
           best_n = n;
           for (int k = 0; k < 3; k++) bd[k] = e[k];
