@@ -85,54 +85,110 @@ __global__ void k_wrap_bin(double4 *__restrict__ pos, int n, const int *__restri
   slot[i] = cell_slot(ccount, c);
 }
 
-__global__ void k_scatter_perm(const int *__restrict__ cell, const int *__restrict__ slot,
-                               const int *__restrict__ cstart, int n, int *__restrict__ perm) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  perm[cstart[cell[i]] + slot[i]] = i;
+// Zeroes a construction's state and its two cell counters.
+__global__ void k_build_begin(BuildState *__restrict__ bs, int *__restrict__ ocount, int *__restrict__ gcount,
+                              int ncell) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c == 0) *bs = BuildState{};
+  if (c < ncell) {
+    ocount[c] = 0;
+    gcount[c] = 0;
+  }
 }
 
-// Order each cell's members by (key, input index) when `key` is given, else
-// by input index: perm_in holds the items grouped by cell (k_scatter_perm, in
-// atomic order); each thread takes one item, counts the members of its cell
-// that sort before it and writes the item at that rank into perm_out.  Keys
-// are unique, so this is a permutation, and with the slots of k_wrap_bin
-// taken by atomics it makes the order deterministic.  Owned particles are
-// keyed by particle id, so the order after a construction depends only on
+// First particle of each cell: the cells taken in storage order (order[k] =
+// the k-th cell, brick by brick), also by that order in start_r.
+struct ScanCells {
+  const int *count, *order;
+  int *start, *start_r;
+  __device__ __forceinline__ long long in(long long k) const { return count[order[k]]; }
+  __device__ __forceinline__ void out(long long k, long long x, long long) const {
+    start[order[k]] = (int)x;
+    start_r[k] = (int)x;
+  }
+  __device__ __forceinline__ void total(long long) const {}
+};
+
+// Order of a cell's members: by (key, input index) when `key` is given, else
+// by input index.  Keys are unique, so this is a permutation, and with the
+// slots taken by atomics it makes the order deterministic.  Owned particles
+// are keyed by particle id, so the order after a construction depends only on
 // the particles and their ids, not on the order an earlier one left.
 __device__ __forceinline__ unsigned long long sort_key(const int *__restrict__ key, int i) {
   const unsigned long long k = key ? (unsigned long long)((unsigned)key[i] ^ 0x80000000u) : 0ull;
   return (k << 32) | (unsigned)i;
 }
 
-__global__ void k_rank_in_cell(const int *__restrict__ perm_in, const int *__restrict__ cellv,
-                               const int *__restrict__ cstart, const int *__restrict__ ccount,
-                               const int *__restrict__ key, int n, int *__restrict__ perm_out) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int item = perm_in[p];
-  const int c = cellv[item];
-  const int s0 = cstart[c], m = ccount[c];
-  const unsigned long long mine = sort_key(key, item);
-  int rank = 0;
-  for (int q = 0; q < m; q++) rank += sort_key(key, perm_in[s0 + q]) < mine ? 1 : 0;
-  perm_out[s0 + rank] = item;
+// Items grouped by cell, in atomic order, as their sort keys (the item in the
+// low word).  n items, or bs->ng.
+__global__ void k_scatter_keys(const int *__restrict__ cell, const int *__restrict__ slot,
+                               const int *__restrict__ cstart, int n, const int *__restrict__ key,
+                               unsigned long long *__restrict__ keys, const BuildState *__restrict__ bs) {
+  if (bs->err) return;
+  const int m = n >= 0 ? n : (int)bs->ng;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x)
+    keys[cstart[cell[i]] + slot[i]] = sort_key(key, i);
 }
 
-__global__ void k_gather_owned(const int *__restrict__ perm, int n, const double4 *__restrict__ pos_in,
-                               const double4 *__restrict__ mom_in, const int *__restrict__ id_in,
-                               const int *__restrict__ cell_in, const int *__restrict__ rep_in,
-                               double4 *__restrict__ pos_out, double4 *__restrict__ mom_out,
-                               int *__restrict__ id_out, int *__restrict__ cell_out, int *__restrict__ rep_out) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int i = perm[k];
-  pos_out[k] = pos_in[i];
-  mom_out[k] = mom_in[i];
-  id_out[k] = id_in[i];
-  cell_out[k] = cell_in[i];
-  rep_out[k] = rep_in[i];
+// The place of grouped item p in its cell [s0, s0 + m): s0 and the members
+// that sort before it, read four at a time (a chain of single reads took 20 us
+// at any size).
+__device__ __forceinline__ int sorted_place(const unsigned long long *__restrict__ keys, unsigned long long mine,
+                                            int s0, int m) {
+  int rank = 0, q = 0;
+  for (; q + 4 <= m; q += 4) {
+    const unsigned long long a = keys[s0 + q], b = keys[s0 + q + 1], c = keys[s0 + q + 2], d = keys[s0 + q + 3];
+    rank += (a < mine) + (b < mine) + (c < mine) + (d < mine);
+  }
+  for (; q < m; q++) rank += keys[s0 + q] < mine;
+  return s0 + rank;
 }
+
+struct OwnedArrays {
+  double4 *pos, *mom;
+  int *id, *cell, *rep;
+};
+
+// The owned particles in brick order, each cell's by id, and (nimg) the ghost
+// images each will have (face_options).
+__global__ void k_sort_owned(const unsigned long long *__restrict__ keys, const int *__restrict__ cstart,
+                             const int *__restrict__ ccount, int n, OwnedArrays in, OwnedArrays out,
+                             int *__restrict__ nimg, const Replica *__restrict__ reps, double SL,
+                             const BuildState *__restrict__ bs) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n || bs->err) return;
+  const unsigned long long mine = keys[p];
+  const int i = (int)(unsigned)mine;
+  const int c = in.cell[i];
+  const double4 q = in.pos[i], mo = in.mom[i];
+  const int id = in.id[i], r = in.rep[i];
+  const int k = sorted_place(keys, mine, cstart[c], ccount[c]);
+  out.pos[k] = q;
+  out.mom[k] = mo;
+  out.id[k] = id;
+  out.cell[k] = c;
+  out.rep[k] = r;
+  if (nimg) {
+    int lo[3], hi[3];
+    face_options(q, reps[r], SL, lo, hi);
+    nimg[k] = (1 + lo[0] + hi[0]) * (1 + lo[1] + hi[1]) * (1 + lo[2] + hi[2]) - 1;
+  }
+}
+
+// First image of each owned particle; the construction stops when there are
+// more images than room.
+struct ScanImages {
+  const int *nimg;
+  int *goff;
+  BuildState *bs;
+  long long cap;
+  __device__ __forceinline__ long long in(long long i) const { return nimg[i]; }
+  __device__ __forceinline__ void out(long long i, long long x, long long) const { goff[i] = (int)x; }
+  __device__ __forceinline__ void total(long long t) const {
+    bs->ng = t;
+    if (t > cap) atomicOr(&bs->err, kErrGhostCap);
+  }
+};
 
 // Halo of one domain (MDManager::MakePairList's six sequential
 // FindBorderParticles/SendBorderParticlesSub passes, mdmanager.cc:269-275):
@@ -142,75 +198,102 @@ __global__ void k_gather_owned(const int *__restrict__ perm, int n, const double
 // vector whose every non-zero component passes its face test.  The box is
 // [s, e) = [0, L) (MDRect::IsInsideEdge, mdrect.cc:24-47: s < q < s + SL and
 // e - SL < q < e).
-__global__ void k_count_images(const double4 *__restrict__ pos, int n, const int *__restrict__ rep,
-                               const Replica *__restrict__ reps, double SL, int *__restrict__ nimg) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int lo[3], hi[3];
-  face_options(pos[i], reps[rep[i]], SL, lo, hi);
-  nimg[i] = (1 + lo[0] + hi[0]) * (1 + lo[1] + hi[1]) * (1 + lo[2] + hi[2]) - 1;
+struct GhostArrays {
+  int *src, *code;
+  double4 *pos;
+  int *cell, *slot, *count;
+};
+
+__device__ __forceinline__ void put_image(const GhostArrays &G, int k, int i, int code, int r, const double3 y,
+                                          int cl, int slot) {
+  G.src[k] = i;
+  G.code[k] = ghost_word(code, r);
+  G.pos[k] = make_double4(y.x, y.y, y.z, 0.0);
+  G.cell[k] = cl;
+  G.slot[k] = slot;
 }
 
+// The images of each particle from goff[i], in the order of the shifts 0, +1,
+// -1 along x, then y, then z.  A particle near one face of an axis at most has
+// up to seven; their cells' counters are asked for together (one after
+// another, each waiting for its slot, they took 19 us).  One near both faces
+// (a box of two search lengths, to a rounding) takes the general loop.
 __global__ void k_emit_images(const double4 *__restrict__ pos, int n, const int *__restrict__ rep,
-                              const Replica *__restrict__ reps, double SL, const int *__restrict__ goff, int ng,
-                              int *__restrict__ gsrc, int *__restrict__ gcode,
-                              double4 *__restrict__ gpos, int *__restrict__ gcell,
-                              int *__restrict__ gslot, int *__restrict__ gcount) {
+                              const Replica *__restrict__ reps, double SL, const int *__restrict__ goff,
+                              const BuildState *__restrict__ bs, GhostArrays G) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || bs->err) return;
   const int r = rep[i];
   const Replica &R = reps[r];
   const double4 q = pos[i];
   int lo[3], hi[3];
   face_options(q, R, SL, lo, hi);
+  if (!(lo[0] | lo[1] | lo[2] | hi[0] | hi[1] | hi[2])) return;
+  const int ng = (int)bs->ng;
   int k = goff[i];
-  const int sxs[3] = {0, 1, -1};
-  for (int a = 0; a < 3; a++) {
-    const int sx = sxs[a];
-    if ((sx == 1 && !lo[0]) || (sx == -1 && !hi[0])) continue;
-    for (int b = 0; b < 3; b++) {
-      const int sy = sxs[b];
-      if ((sy == 1 && !lo[1]) || (sy == -1 && !hi[1])) continue;
-      for (int c = 0; c < 3; c++) {
-        const int sz = sxs[c];
-        if ((sz == 1 && !lo[2]) || (sz == -1 && !hi[2])) continue;
-        if (!sx && !sy && !sz) continue;
-        if (k >= ng) return;  // cannot happen: goff is the scan of k_count_images
-        const int code = (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1);
-        const double3 y = image_of(q, code, R.L);
-        gsrc[k] = i;
-        gcode[k] = ghost_word(code, r);
-        gpos[k] = make_double4(y.x, y.y, y.z, 0.0);
-        const int cl = cell_of(y.x, y.y, y.z, R);
-        gcell[k] = cl;
-        gslot[k] = cell_slot(gcount, cl);
-        k++;
-      }
+  if ((lo[0] & hi[0]) | (lo[1] & hi[1]) | (lo[2] & hi[2])) {
+    const int sxs[3] = {0, 1, -1};
+    for (int a = 0; a < 3; a++)
+      for (int b = 0; b < 3; b++)
+        for (int c = 0; c < 3; c++) {
+          const int s[3] = {sxs[a], sxs[b], sxs[c]};
+          bool image = (s[0] | s[1] | s[2]) != 0;
+          for (int x = 0; x < 3; x++) image = image && (s[x] == 0 || (s[x] > 0 ? lo[x] : hi[x]));
+          if (!image || k >= ng) continue;  // goff is the scan of the images' count: k < ng
+          const int code = (s[0] + 1) + 3 * (s[1] + 1) + 9 * (s[2] + 1);
+          const double3 y = image_of(q, code, R.L);
+          const int cl = cell_of(y.x, y.y, y.z, R);
+          put_image(G, k, i, code, r, y, cl, atomicAdd(&G.count[cl], 1));
+          k++;
+        }
+    return;
+  }
+  const int s[3] = {lo[0] - hi[0], lo[1] - hi[1], lo[2] - hi[2]};
+  int cl[8], slot[8];
+#pragma unroll
+  for (int j = 1; j < 8; j++) {
+    const int sx = (j & 4) ? s[0] : 0, sy = (j & 2) ? s[1] : 0, sz = (j & 1) ? s[2] : 0;
+    const bool image = (!(j & 4) || s[0]) && (!(j & 2) || s[1]) && (!(j & 1) || s[2]);
+    cl[j] = -1;
+    slot[j] = 0;
+    if (image) {
+      const double3 y = image_of(q, (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1), R.L);
+      cl[j] = cell_of(y.x, y.y, y.z, R);
+      slot[j] = atomicAdd(&G.count[cl[j]], 1);
     }
+  }
+#pragma unroll
+  for (int j = 1; j < 8; j++) {
+    if (cl[j] < 0 || k >= ng) continue;
+    const int sx = (j & 4) ? s[0] : 0, sy = (j & 2) ? s[1] : 0, sz = (j & 1) ? s[2] : 0;
+    const int code = (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1);
+    put_image(G, k, i, code, r, image_of(q, code, R.L), cl[j], slot[j]);
+    k++;
   }
 }
 
-__global__ void k_gather_ghosts(const int *__restrict__ perm, int ng, int pn,
-                                const int *__restrict__ src_in, const int *__restrict__ code_in,
-                                const double4 *__restrict__ gpos_in, const int *__restrict__ gcell_in,
-                                int *__restrict__ gsrc, int *__restrict__ gcode,
-                                double4 *__restrict__ pos, int *__restrict__ cell) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ng) return;
-  const int g = perm[k];
-  gsrc[k] = src_in[g];
-  gcode[k] = code_in[g];
-  pos[pn + k] = gpos_in[g];
-  cell[pn + k] = gcell_in[g];
-}
-
-__global__ void k_set_sentinel(double4 *a, double4 *b, float4 *ra, float4 *rb, int idx) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    const double far = 1.0e200;
-    a[idx] = make_double4(far, far, far, 0.0);
-    b[idx] = make_double4(far, far, far, 0.0);
-    if (ra) ra[idx] = make_float4(1.0e30f, 1.0e30f, 1.0e30f, 0.0f);
-    if (rb) rb[idx] = make_float4(1.0e30f, 1.0e30f, 1.0e30f, 0.0f);
+// The ghosts in cell order, each cell's in the order they were emitted, after
+// the pn owned particles.  gunit (a unit of a group): the source unit, taken
+// out of the code word.
+__global__ void k_sort_ghosts(const unsigned long long *__restrict__ keys, const int *__restrict__ gstart,
+                              const int *__restrict__ gcount, int pn, const int *__restrict__ src_in,
+                              const int *__restrict__ code_in, const double4 *__restrict__ gpos_in,
+                              const int *__restrict__ gcell_in, int *__restrict__ gsrc, int *__restrict__ gcode,
+                              int *__restrict__ gunit, double4 *__restrict__ pos, int *__restrict__ cell,
+                              const BuildState *__restrict__ bs) {
+  if (bs->err) return;
+  const int ng = (int)bs->ng;
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ng; p += gridDim.x * blockDim.x) {
+    const unsigned long long mine = keys[p];
+    const int g = (int)(unsigned)mine;
+    const int c = gcell_in[g], src = src_in[g], w = code_in[g];
+    const double4 q = gpos_in[g];
+    const int k = sorted_place(keys, mine, gstart[c], gcount[c]);
+    gsrc[k] = src;
+    gcode[k] = gunit ? ghost_shift(w) : w;
+    if (gunit) gunit[k] = ghost_rep(w);
+    pos[pn + k] = q;
+    cell[pn + k] = c;
   }
 }
 
@@ -361,23 +444,6 @@ __global__ void k_unit_emit(const SrcUnit *__restrict__ tab, int nsrc, int total
         gslot[k] = cell_slot(gcount, cl);
         k++;
       }
-}
-
-// k_gather_ghosts for a unit: the shift code goes to gcode (replica 0), the
-// source unit to gunit.
-__global__ void k_gather_unit_ghosts(const int *__restrict__ perm, int ng, int pn, const int *__restrict__ src_in,
-                                     const int *__restrict__ word_in, const double4 *__restrict__ gpos_in,
-                                     const int *__restrict__ gcell_in, int *__restrict__ gsrc,
-                                     int *__restrict__ gcode, int *__restrict__ gunit, double4 *__restrict__ pos,
-                                     int *__restrict__ cell) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ng) return;
-  const int g = perm[k];
-  gsrc[k] = src_in[g];
-  gcode[k] = ghost_shift(word_in[g]);
-  gunit[k] = ghost_rep(word_in[g]);
-  pos[pn + k] = gpos_in[g];
-  cell[pn + k] = gcell_in[g];
 }
 
 // Owned positions of every unit of a group, by unit slot.

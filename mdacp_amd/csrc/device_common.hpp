@@ -28,6 +28,28 @@ constexpr int kErrInvalidPosition = 1;
 constexpr int kErrInvalidIndex = 2;
 constexpr int kErrCapacity = 4;
 constexpr int kErrLayout = 8;  // a listed partner outside its brick's staged ranges
+constexpr int kErrSearchCap = 16;   // a row has more candidates than its bitmask holds
+constexpr int kErrGhostCap = 32;    // more ghost images than there is room for
+constexpr int kErrGatherCap = 64;   // ... gather-list entries
+constexpr int kErrSlotCap = 128;    // ... list slots
+// A construction's kernels run one after another without the host, on the
+// room the last construction needed and a little more.  One that finds too
+// little sets its bit; the kernels after it do nothing; and the host, which
+// reads the state once at the end, makes room and queues them again from
+// there.  Bits set before the rows are ordered:
+constexpr int kErrBeforeRows = kErrInvalidPosition | kErrInvalidIndex | kErrSearchCap | kErrGhostCap | kErrGatherCap;
+
+// What a construction's kernels count (device; copied to the host at its end).
+struct BuildState {
+  int err;           // kErr bits
+  int nslice;        // 64-row slices
+  int max_staged;    // largest neighbourhood of a brick
+  int pad;
+  long long ng;      // ghost images
+  long long gtotal;  // gather-list entries
+  long long slots;   // list slots
+  long long entries; // list entries
+};
 
 // Brick kernels serve brick blockIdx.x.  The hardware hands consecutive
 // workgroups to the 8 XCDs in turn, so every XCD (each with its own L2) gets

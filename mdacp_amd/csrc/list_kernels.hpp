@@ -69,53 +69,47 @@ __device__ __forceinline__ BrickBox brick_box(int b, const Replica &R) {
   return X;
 }
 
-// ---- rank order of cells -------------------------------------------------
-__global__ void k_rank_counts(const int *__restrict__ count, const int *__restrict__ rank, int ncell,
-                              int *__restrict__ count_r) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < ncell) count_r[rank[c]] = count[c];
-}
-
-__global__ void k_unrank_starts(const int *__restrict__ start_r, const int *__restrict__ rank, int ncell,
-                                int *__restrict__ start) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < ncell) start[c] = start_r[rank[c]];
-}
-
-// rows of each brick: [row0, row0 + nrow), in 64-row slices
-__global__ void k_brick_rows(const int *__restrict__ brick_rank0, const int *__restrict__ start_r, int nbrick,
-                             int ncell, int pn, int *__restrict__ row0, int *__restrict__ nrow,
-                             int *__restrict__ nsl) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nbrick) return;
-  const int r0 = brick_rank0[b], r1 = brick_rank0[b + 1];
-  const int s0 = r0 < ncell ? start_r[r0] : pn;
-  const int s1 = r1 < ncell ? start_r[r1] : pn;
-  row0[b] = s0;
-  nrow[b] = s1 - s0;
-  nsl[b] = (s1 - s0 + kWave - 1) / kWave;
-}
-
-__global__ void k_slice_brick(const int *__restrict__ vslice0, const int *__restrict__ nsl, int nbrick,
-                              int *__restrict__ slice_brick) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nbrick) return;
-  for (int k = 0; k < nsl[b]; k++) slice_brick[vslice0[b] + k] = b;
-}
+// Rows of each brick, [row0, row0 + nrow), and its first 64-row slice.
+// brick_rank0[b]: the brick's first cell in storage order.
+struct ScanBricks {
+  const int *brick_rank0, *start_r;
+  int ncell, pn;
+  int *row0, *nrow, *vslice0;
+  BuildState *bs;
+  __device__ __forceinline__ int start(int k) const { return k < ncell ? start_r[k] : pn; }
+  __device__ __forceinline__ long long in(long long b) const {
+    return (start(brick_rank0[b + 1]) - start(brick_rank0[b]) + kWave - 1) / kWave;
+  }
+  __device__ __forceinline__ void out(long long b, long long x, long long) const {
+    const int s0 = start(brick_rank0[b]);
+    row0[b] = s0;
+    nrow[b] = start(brick_rank0[b + 1]) - s0;
+    vslice0[b] = (int)x;
+  }
+  __device__ __forceinline__ void total(long long t) const { bs->nslice = (int)t; }
+};
 
 // Staged ranges of each brick, range 2r = owned particles of neighbourhood
 // cell r, range 2r+1 = its ghosts (cells outside the extended grid are
 // empty).  tstart = first index in the owned+ghost arrays (ghosts from pn on),
 // tbase = offset in the staged array (tbase[R] = staged count = pad slot).
 // One wavefront per brick, a lane per neighbourhood cell, the offsets from a
-// wavefront prefix sum; each brick's staged count also goes to total_d.
+// wavefront prefix sum.  A brick without rows stages nothing.
 __global__ __launch_bounds__(kBlock) void k_brick_ranges(Bricks B, CellTables T, int nbrick, int pn,
-                                                         int *__restrict__ tstart, int *__restrict__ tbase,
-                                                         int *__restrict__ nrange, int *__restrict__ btotal,
-                                                         double *__restrict__ total_d) {
+                                                         const int *__restrict__ nrow, int *__restrict__ tstart,
+                                                         int *__restrict__ tbase, int *__restrict__ nrange,
+                                                         int *__restrict__ btotal,
+                                                         const BuildState *__restrict__ bs) {
   const int b = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave;
-  if (b >= nbrick) return;  // the whole wavefront
+  if (b >= nbrick || bs->err) return;  // the whole wavefront
+  if (nrow[b] == 0) {
+    if (lane == 0) {
+      nrange[b] = 0;
+      btotal[b] = 0;
+    }
+    return;
+  }
   const Replica &Rp = B.reps[B.brep[b]];
   const BrickBox X = brick_box(b, Rp);
   const int nc = X.n[0] * X.n[1] * X.n[2];
@@ -157,19 +151,36 @@ __global__ __launch_bounds__(kBlock) void k_brick_ranges(Bricks B, CellTables T,
     tb[kRangesPerCell * nc] = base;
     nrange[b] = kRangesPerCell * nc;
     btotal[b] = base;
-    total_d[b] = (double)base;
   }
 }
+
+// First gather-list entry of each brick; the construction stops when there are
+// more entries than room.
+struct ScanGather {
+  const int *btotal;
+  long long *gbase;
+  int nbrick;
+  long long cap;
+  BuildState *bs;
+  __device__ __forceinline__ long long in(long long b) const { return btotal[b]; }
+  __device__ __forceinline__ void out(long long b, long long x, long long) const { gbase[b] = x; }
+  __device__ __forceinline__ void total(long long t) const {
+    gbase[nbrick] = t;
+    bs->gtotal = t;
+    if (t > cap) atomicOr(&bs->err, kErrGatherCap);
+  }
+};
 
 // Gather list of each brick: glist[gbase[b] + u] = index (owned, or pn + ghost)
 // of staged entry u, so the force kernels stage with one indexed load per
 // entry.  One workgroup per brick.
 __global__ void k_brick_glist(int rstride, const int *__restrict__ tstart, const int *__restrict__ tbase,
                               const int *__restrict__ nrange, const long long *__restrict__ gbase,
-                              int *__restrict__ glist) {
+                              int *__restrict__ glist, const BuildState *__restrict__ bs) {
   __shared__ int tb[kRangesPerCell * kMaxBrickCells + 1];
   const int b = blockIdx.x;
   const int R = nrange[b];
+  if (bs->err || R == 0) return;
   const int *tbg = tbase + (long long)b * (rstride + 1);
   const int *ts = tstart + (long long)b * rstride;
   for (int r = threadIdx.x; r <= R; r += blockDim.x) tb[r] = tbg[r];
@@ -189,7 +200,6 @@ __global__ void k_brick_glist(int rstride, const int *__restrict__ tstart, const
 
 // ---- search --------------------------------------------------------------
 constexpr int kMaxRanges = kRangesPerCell * kMaxBrickCells;
-constexpr int kErrSearchCap = 16;  // a row has more candidates than its bitmask holds
 
 // cell offset code of a partner cell relative to the row's cell (each -1..1)
 __device__ __forceinline__ uint8_t offset_code(int ox, int oy, int oz) {
@@ -234,16 +244,6 @@ __device__ __forceinline__ double4 img_of(double4 q, uint32_t e, const double *L
   q.y += img_shift((s >> 2) & 3u, L[1]);
   q.z += img_shift(s >> 4, L[2]);
   return q;
-}
-
-// The image gather list of a built list: every entry of the gather list
-// (owned, or pn + ghost) as its owner's index and shift.
-__global__ void k_image_glist(const int *__restrict__ glist, long long n, int pn, const int *__restrict__ gsrc,
-                              const int *__restrict__ gcode, uint32_t *__restrict__ gimg) {
-  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int j = glist[k];
-  gimg[k] = j < pn ? img_entry(j, 13) : img_entry(gsrc[j - pn], ghost_shift(gcode[j - pn]));
 }
 
 // Positions of T * kStageBatch consecutive staged entries (one per thread and
@@ -370,7 +370,8 @@ __global__ __launch_bounds__(kWave *W) void k_search_brick(const double4 *__rest
   __shared__ int tb[kMaxRanges + 1];
   constexpr int T = kWave * W;
   const int b = blockIdx.x;
-  if (st.nrow[b] == 0) return;  // a brick of ghost-layer cells only
+  // the one bit this kernel sets is left out: every thread decides alike
+  if (st.nrow[b] == 0 || (*err & ~kErrSearchCap)) return;  // a brick of ghost-layer cells only
   const int R = load_tb<T>(st, b, tb);
   __syncthreads();
   const int total = tb[R];
@@ -525,7 +526,7 @@ __global__ __launch_bounds__(kWave *W) void k_search_cells(const double4 *__rest
   __shared__ int cell_next;  // the next cell a wavefront takes
   constexpr int T = kWave * W;
   const int b = blockIdx.x;
-  if (st.nrow[b] == 0) return;  // a brick without rows
+  if (st.nrow[b] == 0 || (*err & ~kErrSearchCap)) return;  // a brick without rows, or a construction that stopped
   const int R = load_tb<T>(st, b, tb);
   if (threadIdx.x == 0) cell_next = W;
   __syncthreads();
@@ -630,94 +631,213 @@ constexpr int kSortBins = kBlock;  // lengths >= kSortBins - 1 share the last bi
 // close together in the staged array, and the pair kernels' LDS gathers
 // conflict less (the FP64 kick of 4M particles at rho = 0.5 takes 6% less
 // time than with exact lengths).  With sort == 0 the rows keep their cell
-// order (rowsrc and rowinv are the identity).  One workgroup of kBlock
-// threads per brick.
-__global__ __launch_bounds__(kBlock) void k_brick_row_order(const int *__restrict__ row_len,
-                                                            const int *__restrict__ row0,
-                                                            const int *__restrict__ nrow,
-                                                            int *__restrict__ rowsrc, int *__restrict__ rowinv,
-                                                            int sort) {
+// order (rowsrc and rowinv are the identity).
+//
+// The same workgroup then moves the brick's particles into that order (from
+// `in` to `out`, which are the same arrays when sort == 0 and nothing moves),
+// takes PairList::Init's snapshot of them (old, pairlist.cc:11-23), and gives
+// each of its slices its length: the longest row of its 64, rounded up to a
+// multiple of kSliceRound so the force loop runs whole batches.  bsum: the
+// list entries of the brick.  One workgroup of kBlock threads per brick.
+struct RowArrays {
+  OwnedArrays a;
+  int *row_len;
+};
+
+__global__ __launch_bounds__(kBlock) void k_order_rows(const int *__restrict__ row0, const int *__restrict__ nrow,
+                                                       const int *__restrict__ vslice0, int *__restrict__ rowsrc,
+                                                       int *__restrict__ rowinv, int sort, RowArrays in,
+                                                       RowArrays out, double4 *__restrict__ old,
+                                                       int *__restrict__ slen, long long *__restrict__ bsum,
+                                                       const BuildState *__restrict__ bs) {
+  constexpr int kWaves = kBlock / kWave;
   __shared__ int start[kSortBins];
   __shared__ int scan[kSortBins];
-  __shared__ int bins[kBlock];
+  __shared__ int wcount[kWaves][kSortBins];
+  __shared__ long long wsum[kWaves];
   const int b = blockIdx.x;
-  const int r0 = row0[b], n = nrow[b];
-  const int t = threadIdx.x;
+  if (bs->err) return;
+  const int r0 = row0[b], n = nrow[b], vs0 = vslice0[b];
+  const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+  if (n == 0) {
+    if (t == 0) bsum[b] = 0;
+    return;
+  }
   if (!sort) {
     for (int v = t; v < n; v += kBlock) {
       rowsrc[r0 + v] = r0 + v;
       rowinv[r0 + v] = r0 + v;
     }
-    return;
-  }
-  start[t] = 0;
-  __syncthreads();
-  // bin of a row: longest rows first, lengths taken in steps of `sort`
-  for (int v = t; v < n; v += kBlock)
-    atomicAdd(&start[kSortBins - 1 - min((row_len[r0 + v] + sort - 1) / sort, kSortBins - 1)], 1);
-  __syncthreads();
-  // exclusive scan of the bin counts (Hillis-Steele over kSortBins == kBlock)
-  int x = start[t];
-  scan[t] = x;
-  __syncthreads();
-  for (int o = 1; o < kSortBins; o <<= 1) {
-    const int y = t >= o ? scan[t - o] : 0;
+  } else {
+    start[t] = 0;
     __syncthreads();
-    scan[t] += y;
+    // bin of a row: longest rows first, lengths taken in steps of `sort`
+    for (int v = t; v < n; v += kBlock)
+      atomicAdd(&start[kSortBins - 1 - min((in.row_len[r0 + v] + sort - 1) / sort, kSortBins - 1)], 1);
     __syncthreads();
-  }
-  start[t] = scan[t] - x;
-  __syncthreads();
-  for (int c0 = 0; c0 < n; c0 += kBlock) {
-    const int v = c0 + t;
-    const int bin = v < n ? kSortBins - 1 - min((row_len[r0 + v] + sort - 1) / sort, kSortBins - 1) : -1;
-    bins[t] = bin;
+    // exclusive scan of the bin counts (Hillis-Steele over kSortBins == kBlock)
+    const int x = start[t];
+    scan[t] = x;
     __syncthreads();
-    if (v < n) {
-      int rank = 0;
-      for (int k = 0; k < t; k++) rank += bins[k] == bin ? 1 : 0;
-      const int p = r0 + start[bin] + rank;
-      rowsrc[p] = r0 + v;
-      rowinv[r0 + v] = p;
+    for (int o = 1; o < kSortBins; o <<= 1) {
+      const int y = t >= o ? scan[t - o] : 0;
+      __syncthreads();
+      scan[t] += y;
+      __syncthreads();
     }
+    start[t] = scan[t] - x;
     __syncthreads();
-    if (v < n) atomicAdd(&start[bin], 1);
-    __syncthreads();
+    // kBlock rows at a time: a row's place among those of its bin from the
+    // ballots of its wavefront (a round per bin the wavefront holds) and the
+    // counts of the wavefronts before it
+    for (int c0 = 0; c0 < n; c0 += kBlock) {
+      const int v = c0 + t;
+      const int bin = v < n ? kSortBins - 1 - min((in.row_len[r0 + v] + sort - 1) / sort, kSortBins - 1) : -1;
+      for (int w = 0; w < kWaves; w++) wcount[w][t] = 0;
+      __syncthreads();
+      int rank = 0;
+      unsigned long long todo = __ballot(bin >= 0);
+      while (todo) {
+        const int lead = __ffsll((long long)todo) - 1;
+        const int lb = __shfl(bin, lead, kWave);
+        const unsigned long long same = __ballot(bin == lb);
+        if (bin == lb) rank = __popcll(same & ((1ull << lane) - 1ull));
+        if (lane == lead) wcount[wv][lb] = __popcll(same);
+        todo &= ~same;
+      }
+      __syncthreads();
+      if (bin >= 0) {
+        for (int w = 0; w < wv; w++) rank += wcount[w][bin];
+        const int p = r0 + start[bin] + rank;
+        rowsrc[p] = r0 + v;
+        rowinv[r0 + v] = p;
+      }
+      __syncthreads();
+      for (int w = 0; w < kWaves; w++) start[t] += wcount[w][t];
+      __syncthreads();
+    }
+  }
+  __syncthreads();  // rowsrc of the brick
+  long long sum = 0;
+  for (int sl = wv; sl * kWave < n; sl += kWaves) {
+    const int v = sl * kWave + lane;
+    int len = 0;
+    if (v < n) {
+      const int k = r0 + v, i = rowsrc[k];
+      len = in.row_len[i];
+      const double4 q = in.a.pos[i];
+      old[k] = q;
+      if (sort) {
+        out.a.pos[k] = q;
+        out.a.mom[k] = in.a.mom[i];
+        out.a.id[k] = in.a.id[i];
+        out.a.cell[k] = in.a.cell[i];
+        out.a.rep[k] = in.a.rep[i];
+        out.row_len[k] = len;
+      }
+      sum += len;
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) len = max(len, __shfl_xor(len, o, kWave));
+    if (lane == 0) slen[vs0 + sl] = (len + kSliceRound - 1) / kSliceRound * kSliceRound;
+  }
+  for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+  if (lane == 0) wsum[wv] = sum;
+  __syncthreads();
+  if (t == 0) {
+    long long m = 0;
+    for (int w = 0; w < kWaves; w++) m += wsum[w];
+    bsum[b] = m;
   }
 }
 
-__global__ void k_gather_int(const int *__restrict__ perm, int n, const int *__restrict__ in, int *__restrict__ out) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) out[k] = in[perm[k]];
-}
-
-// new indices of owned particles (entries >= pn are ghosts and stay)
-__global__ void k_remap_owned(int *__restrict__ idx, long long n, int pn, const int *__restrict__ rowinv) {
-  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int j = idx[k];
-  if (j < pn) idx[k] = rowinv[j];
-}
-
-// slice length = longest row of its 64 rows, rounded up to a multiple of
-// kSliceRound so the force loop runs whole batches; slots = 64 * length.
-// The largest slice length goes to partial (per workgroup).
-__global__ void k_slice_len(const int *__restrict__ row_len, const int *__restrict__ slice_brick,
-                            const int *__restrict__ vslice0, const int *__restrict__ row0,
-                            const int *__restrict__ nrow, int nslice, int *__restrict__ slen,
-                            long long *__restrict__ slots, double *__restrict__ partial) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  int m = 0;
-  if (s < nslice) {
-    const int b = slice_brick[s];
-    const int v0 = (s - vslice0[b]) * kWave;
-    const int v1 = min(nrow[b], v0 + kWave);
-    for (int v = v0; v < v1; v++) m = max(m, row_len[row0[b] + v]);
-    m = (m + kSliceRound - 1) / kSliceRound * kSliceRound;
-    slen[s] = m;
-    slots[s] = (long long)m * kWave;
+// First slot of each slice (64 times its length); the construction stops when
+// there are more slots than room.
+struct ScanSlots {
+  const int *slen;
+  long long *sbase;
+  long long cap;
+  BuildState *bs;
+  __device__ __forceinline__ long long in(long long s) const { return s < bs->nslice ? (long long)slen[s] * kWave : 0; }
+  __device__ __forceinline__ void out(long long s, long long x, long long) const {
+    if (s < bs->nslice) sbase[s] = x;
   }
-  block_max_to_partial((double)m, partial, blockIdx.x);
+  __device__ __forceinline__ void total(long long t) const {
+    bs->slots = t;
+    if (t > cap) atomicOr(&bs->err, kErrSlotCap);
+  }
+};
+
+// What points at owned particles follows them into their rows' order: the
+// ghosts' sources (gsrc_in to gsrc; those of a unit index other units and are
+// remapped once every unit has ordered its rows), the gather list, and, for a
+// domain, the image gather list (gimg) from both.  The ghosts themselves keep
+// their places: their positions and cells go to the arrays the rows went to
+// (when they moved), and into PairList::Init's snapshot.
+__global__ void k_remap(const int *__restrict__ rowinv, int pn, const int *__restrict__ gsrc_in,
+                        int *__restrict__ gsrc, const int *__restrict__ gcode, int *__restrict__ glist,
+                        uint32_t *__restrict__ gimg, const double4 *__restrict__ pos_in,
+                        double4 *__restrict__ pos_out, const int *__restrict__ cell_in, int *__restrict__ cell_out,
+                        double4 *__restrict__ old, const BuildState *__restrict__ bs) {
+  if (bs->err & kErrBeforeRows) return;
+  const long long ng = bs->ng, gt = bs->gtotal, stride = (long long)gridDim.x * blockDim.x;
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  for (long long k = t; k < ng; k += stride) {
+    const int j = gsrc_in[k];
+    gsrc[k] = gimg ? rowinv[j] : j;
+    const double4 q = pos_in[pn + k];
+    old[pn + k] = q;
+    if (pos_out != pos_in) {
+      pos_out[pn + k] = q;
+      cell_out[pn + k] = cell_in[pn + k];
+    }
+  }
+  for (long long k = t; k < gt; k += stride) {
+    const int j = glist[k];
+    if (j < pn) {
+      const int i = rowinv[j];
+      glist[k] = i;
+      if (gimg) gimg[k] = img_entry(i, 13);
+    } else if (gimg) {
+      gimg[k] = img_entry(rowinv[gsrc_in[j - pn]], ghost_shift(gcode[j - pn]));
+    }
+  }
+}
+
+// The end of a construction: its counts, with the list entries and the largest
+// neighbourhood over its bricks, to the host's pinned copy.  One workgroup.
+constexpr int kPublishThreads = 1024;
+
+__global__ __launch_bounds__(kPublishThreads) void k_publish(const BuildState *__restrict__ bs,
+                                                             const int *__restrict__ btotal,
+                                                             const long long *__restrict__ bsum, int nbrick,
+                                                             BuildState *__restrict__ host) {
+  __shared__ long long ws[kPublishThreads / kWave];
+  __shared__ int wm[kPublishThreads / kWave];
+  long long sum = 0;
+  int top = 0;
+  for (int b = threadIdx.x; b < nbrick; b += kPublishThreads) {
+    top = max(top, btotal[b]);
+    if (bsum) sum += bsum[b];
+  }
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o, kWave);
+    top = max(top, __shfl_xor(top, o, kWave));
+  }
+  if (threadIdx.x % kWave == 0) {
+    ws[threadIdx.x / kWave] = sum;
+    wm[threadIdx.x / kWave] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    BuildState S = *bs;
+    S.entries = 0;
+    S.max_staged = 0;
+    for (int w = 0; w < kPublishThreads / kWave; w++) {
+      S.entries += ws[w];
+      S.max_staged = max(S.max_staged, wm[w]);
+    }
+    *host = S;
+  }
 }
 
 constexpr int kEmitWaves = 4;  // wavefronts per brick workgroup of k_emit_brick
@@ -772,7 +892,7 @@ __global__ __launch_bounds__(kWave *W) void k_emit_brick(const int *__restrict__
   __shared__ int tb[kMaxRanges + 1];
   constexpr int T = kWave * W;
   const int b = blockIdx.x;
-  if (st.nrow[b] == 0) return;  // a brick without rows
+  if (st.nrow[b] == 0 || (*err & ~kErrCapacity)) return;  // a brick without rows, or a construction that stopped
   const int R = load_tb<T>(st, b, tb);
   __syncthreads();
   const unsigned total = (unsigned)tb[R];

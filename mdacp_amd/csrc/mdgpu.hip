@@ -185,6 +185,7 @@ struct mdgpu_domain {
 
   // counts and capacities
   int pn = 0, ng = 0, tn = 0;
+  int ng_last = 0;  // ghosts of the last construction
   int cap = 0, gcap = 0;
   int nslice = 0, slice_cap = 0, max_staged = 0;
   long long nbr_slots = 0, nbr_entries = 0, nbr_cap = 0;
@@ -201,11 +202,11 @@ struct mdgpu_domain {
   int *id = nullptr, *id_alt = nullptr, *cell = nullptr, *cell_alt = nullptr;
   int *gsrc = nullptr, *gcode = nullptr;
   int *c_ocount = nullptr, *c_ostart = nullptr, *c_gcount = nullptr, *c_gstart = nullptr;
-  int *count_r = nullptr, *start_r = nullptr;
+  int *start_r = nullptr;
   double *org = nullptr;  // origins of the cell columns, x then y then z
   // bricks
-  int *rank = nullptr, *brick_of_cell = nullptr, *brick_rank0 = nullptr;
-  int *row0 = nullptr, *nrow = nullptr, *nsl = nullptr, *vslice0 = nullptr, *slice_brick = nullptr;
+  int *cell_order = nullptr, *brick_rank0 = nullptr;  // cells in storage order; each brick's first there
+  int *row0 = nullptr, *nrow = nullptr, *vslice0 = nullptr;
   int *tstart = nullptr, *tbase = nullptr, *nrange = nullptr, *btotal = nullptr;
   long long *gbase = nullptr;  // [nbrick + 1] first gather-list entry of each brick
   int *glist = nullptr;        // staged entry -> particle index, brick by brick
@@ -225,7 +226,7 @@ struct mdgpu_domain {
   double inner_budget = 0.0;   // what is left of prune_delta for particle motion
   double step_vmax = 0.0;      // max |p| at this step's expiry test (all replicas)
   int prunes = 0;
-  long long *sbase = nullptr, *slots64 = nullptr;
+  long long *sbase = nullptr;
   int *slen = nullptr, *row_len = nullptr;
   // build scratch
   int *rowsrc = nullptr, *rowinv = nullptr;  // row order inside bricks: new -> old, old -> new
@@ -233,12 +234,17 @@ struct mdgpu_domain {
   uint32_t *mask = nullptr;  // candidate bitmask per row, mcap words
   size_t mask_cap = 0;
   int mcap = 32;
-  double *spart = nullptr;  // per-workgroup maxima of slice lengths
-  int *slot = nullptr, *perm = nullptr, *nimg = nullptr, *goff = nullptr;
-  int *perm_in = nullptr;  // binned items grouped by cell, before the in-cell order
+  long long *bsum = nullptr;  // list entries per brick
+  int *slot = nullptr, *nimg = nullptr, *goff = nullptr, *row_len_alt = nullptr;
   int *t_gsrc = nullptr, *t_gcode = nullptr, *t_gcell = nullptr;
-  long long *key = nullptr, *scan_scratch = nullptr;
-  long long scan_scratch_n = 0;
+  unsigned long long *key = nullptr;  // binned items grouped by cell: their sort keys
+  // single-launch scans (scan.hpp)
+  unsigned long long *scan_status = nullptr;
+  unsigned *scan_ticket = nullptr, scan_base = 0, scan_epoch = 0;
+  long long scan_cap = 0;  // workgroups
+  BuildState *bs = nullptr, *h_bs = nullptr;  // a construction's counts, and their pinned copy
+  int staged_guess = 0;    // largest neighbourhood of the last construction with these bricks (0: none)
+  bool rows_swapped = false;  // the construction in flight has swapped the owned arrays for the row order
   double *xfer = nullptr;  // 3 doubles per particle: host buffers in the boundary's layout
   size_t xfer_cap = 0;
   double *disp = nullptr, *partial = nullptr, *maxpart = nullptr;
@@ -433,14 +439,13 @@ int set_geometry(mdgpu_domain *d) {
   CHK(dalloc(d, &d->c_ostart, d->ncell));
   CHK(dalloc(d, &d->c_gcount, d->ncell));
   CHK(dalloc(d, &d->c_gstart, d->ncell));
-  CHK(dalloc(d, &d->count_r, d->ncell + 1));
   CHK(dalloc(d, &d->start_r, d->ncell + 1));
   CHK(dalloc(d, &d->org, org.size()));
   HIPCHK(d, hipMemcpy(d->org, org.data(), org.size() * sizeof(double), hipMemcpyHostToDevice));
   // bricks z-major inside each replica, cells z, y, x inside each brick; then
   // the replica's lower ghost-layer cells, which belong to no brick (no owned
   // particle bins there: k_wrap_bin refuses one)
-  std::vector<int> rank(d->ncell), boc(d->ncell, -1), rank0(d->nbrick + 1), brep(d->nbrick);
+  std::vector<int> order(d->ncell), boc(d->ncell, -1), rank0(d->nbrick + 1), brep(d->nbrick);
   int rk = 0;
   for (int r = 0; r < d->nrep; r++) {
     const Replica &R = d->rh[r];
@@ -454,28 +459,26 @@ int set_geometry(mdgpu_domain *d) {
             for (int y = 1 + by * R.bd[1]; y < std::min(R.m[1], 1 + (by + 1) * R.bd[1]); y++)
               for (int x = 1 + bx * R.bd[0]; x < std::min(R.m[0], 1 + (bx + 1) * R.bd[0]); x++) {
                 const int c = R.cell0 + (z * R.m[1] + y) * R.m[0] + x;
-                rank[c] = rk++;
+                order[rk++] = c;
                 boc[c] = b;
               }
         }
     for (int z = 0; z < R.m[2]; z++)
       for (int y = 0; y < R.m[1]; y++)
         for (int x = 0; x < R.m[0]; x++)
-          if (x == 0 || y == 0 || z == 0) rank[R.cell0 + (z * R.m[1] + y) * R.m[0] + x] = rk++;
+          if (x == 0 || y == 0 || z == 0) order[rk++] = R.cell0 + (z * R.m[1] + y) * R.m[0] + x;
   }
   rank0[d->nbrick] = rk;
   d->h_brick_of_cell = boc;
-  CHK(dalloc(d, &d->rank, d->ncell));
-  CHK(dalloc(d, &d->brick_of_cell, d->ncell));
+  CHK(dalloc(d, &d->cell_order, d->ncell));
   CHK(dalloc(d, &d->brick_rank0, d->nbrick + 1));
   CHK(dalloc(d, &d->brep, d->nbrick));
-  HIPCHK(d, hipMemcpy(d->rank, rank.data(), rank.size() * sizeof(int), hipMemcpyHostToDevice));
-  HIPCHK(d, hipMemcpy(d->brick_of_cell, boc.data(), boc.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIPCHK(d, hipMemcpy(d->cell_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(d, hipMemcpy(d->brick_rank0, rank0.data(), rank0.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(d, hipMemcpy(d->brep, brep.data(), brep.size() * sizeof(int), hipMemcpyHostToDevice));
   CHK(dalloc(d, &d->row0, d->nbrick));
   CHK(dalloc(d, &d->nrow, d->nbrick));
-  CHK(dalloc(d, &d->nsl, d->nbrick));
+  CHK(dalloc(d, &d->bsum, d->nbrick));
   CHK(dalloc(d, &d->vslice0, d->nbrick));
   CHK(dalloc(d, &d->nrange, d->nbrick));
   CHK(dalloc(d, &d->bpart, d->nbrick));
@@ -486,6 +489,7 @@ int set_geometry(mdgpu_domain *d) {
   CHK(dalloc(d, &d->tbase, (size_t)d->nbrick * (kRangesPerCell * d->rmax + 1)));
   CHK(upload_replicas(d));
   d->initialized = false;
+  d->staged_guess = 0;
   invalidate(d);
   return MDGPU_OK;
 }
@@ -526,12 +530,11 @@ int ensure_owned(mdgpu_domain *d, int need) {
   CHK(dalloc(d, &d->mom_alt, nc));
   CHK(dalloc(d, &d->id_alt, nc));
   CHK(dalloc(d, &d->slot, tc_new));
-  CHK(dalloc(d, &d->perm, tc_new));
-  CHK(dalloc(d, &d->perm_in, tc_new));
   CHK(dalloc(d, &d->key, tc_new));
   CHK(dalloc(d, &d->nimg, nc));
   CHK(dalloc(d, &d->goff, nc));
   CHK(dalloc(d, &d->row_len, nc));
+  CHK(dalloc(d, &d->row_len_alt, nc));
   CHK(dalloc(d, &d->rowsrc, nc));
   CHK(dalloc(d, &d->rowinv, nc));
   d->cap = nc;
@@ -563,8 +566,6 @@ int ensure_ghosts(mdgpu_domain *d, int need) {
   CHK(dalloc(d, &d->disp, tc_new));
   CHK(dalloc(d, &d->maxpart, nblk((long long)tc_new, kWave)));
   CHK(dalloc(d, &d->slot, tc_new));
-  CHK(dalloc(d, &d->perm, tc_new));
-  CHK(dalloc(d, &d->perm_in, tc_new));
   CHK(dalloc(d, &d->key, tc_new));
   CHK(dalloc(d, &d->gsrc, ngc));
   CHK(dalloc(d, &d->gcode, ngc));
@@ -577,12 +578,25 @@ int ensure_ghosts(mdgpu_domain *d, int need) {
   return MDGPU_OK;
 }
 
-int ensure_scan(mdgpu_domain *d, long long n) {
-  const long long need = scan_scratch_size(n);
-  if (d->scan_scratch && need <= d->scan_scratch_n) return MDGPU_OK;
-  d->scan_scratch_n = 0;  // dalloc frees the old buffer first; a failed allocation leaves none
-  CHK(dalloc(d, &d->scan_scratch, (size_t)need));
-  d->scan_scratch_n = need;
+// An exclusive scan of n items by functor f (scan.hpp), nothing when *skip is set.
+template <class F>
+int scan(mdgpu_domain *d, const F &f, long long n, const int *skip = nullptr) {
+  const long long nb = std::max(1ll, (n + kScanItems - 1) / kScanItems);
+  if (nb > d->scan_cap) {
+    d->scan_cap = 0;
+    const long long c = nb + nb / 4 + 64;
+    CHK(dalloc(d, &d->scan_status, (size_t)c));
+    d->scan_cap = c;
+    d->scan_epoch = 0;
+  }
+  if (d->scan_epoch == 0 || d->scan_epoch + 1 == kScanEpochs) {
+    HIPCHK(d, hipMemsetAsync(d->scan_status, 0, (size_t)d->scan_cap * sizeof(unsigned long long), d->stream));
+    d->scan_epoch = 0;
+  }
+  const ScanCtx c{d->scan_status, d->scan_ticket, d->scan_base, ++d->scan_epoch};
+  hipLaunchKernelGGL((k_scan<F>), dim3((unsigned)nb), dim3(kScanThreads), 0, d->stream, f, n, c, skip);
+  CHK(check_launch(d, "scan"));
+  d->scan_base += (unsigned)nb;  // the places this launch's workgroups take
   return MDGPU_OK;
 }
 
@@ -594,10 +608,8 @@ int ensure_partial(mdgpu_domain *d, int nb) {
   return MDGPU_OK;
 }
 
-int read_err_flags(mdgpu_domain *d) {
-  HIPCHK(d, hipMemcpyAsync(d->h_i32, d->i32, sizeof(int) * 4, hipMemcpyDeviceToHost, d->stream));
-  CHK(sync(d));
-  const int e = d->h_i32[0];
+// The error that a construction's kernels report (kErr bits).
+int build_error(mdgpu_domain *d, int e) {
   if (e & kErrInvalidPosition) {
     d->err = "Invalid position";
     return MDGPU_ERR_INVALID_POSITION;
@@ -610,7 +622,7 @@ int read_err_flags(mdgpu_domain *d) {
     d->err = "internal: a listed partner lies outside its brick's staged ranges";
     return MDGPU_ERR_HIP;
   }
-  if (e & (kErrCapacity | kErrSearchCap)) {
+  if (e & kErrCapacity) {
     d->err = "pair list capacity";
     return MDGPU_ERR_CAPACITY;
   }
@@ -633,30 +645,6 @@ int read_max(mdgpu_domain *d, int k, double *v) {
   return MDGPU_OK;
 }
 
-// Order n binned items (cellv[], slot[] from atomics, counts[] per cell):
-// starts[] over cells (in brick rank order when `ranked`), perm[] = new order,
-// members of a cell by (key, input index), or input index when key is null
-// (k_rank_in_cell).
-int cell_sort(mdgpu_domain *d, const int *cellv, int n, int *counts, int *starts, bool ranked,
-              const int *key) {
-  hipStream_t st = d->stream;
-  CHK(ensure_scan(d, d->ncell));
-  if (ranked) {
-    hipLaunchKernelGGL(k_rank_counts, dim3(nblk(d->ncell)), dim3(kBlock), 0, st, counts, d->rank, d->ncell,
-                       d->count_r);
-    exclusive_scan<int, int>(d->count_r, d->start_r, d->ncell, d->scan_scratch, nullptr, st);
-    hipLaunchKernelGGL(k_unrank_starts, dim3(nblk(d->ncell)), dim3(kBlock), 0, st, d->start_r, d->rank, d->ncell,
-                       starts);
-  } else {
-    exclusive_scan<int, int>(counts, starts, d->ncell, d->scan_scratch, nullptr, st);
-  }
-  hipLaunchKernelGGL(k_scatter_perm, dim3(nblk(n)), dim3(kBlock), 0, st, cellv, d->slot, starts, n, d->perm_in);
-  if (n > 0)
-    hipLaunchKernelGGL(k_rank_in_cell, dim3(nblk(n)), dim3(kBlock), 0, st, d->perm_in, cellv, starts, counts, key, n,
-                       d->perm);
-  return check_launch(d, "cell sort");
-}
-
 template <class K>
 void allow_lds(K kernel, size_t bytes) {
   if (bytes > 64 * 1024)
@@ -674,6 +662,14 @@ int lds_cap_for(const mdgpu_domain *d, int bytes_per_entry, int kb) {
 // per-step trade-off between staged bricks and workgroups per CU).
 constexpr int kSearchLdsKb = 96;
 
+// Room per brick for the search's staging: what the last construction with
+// these bricks needed and a little more (not known: all of the budget).  A
+// brick that needs more reads its candidates from memory.
+int search_lds_cap(const mdgpu_domain *d) {
+  const int budget = std::min(kSearchLdsKb, d->lds_max_kb) * 1024 / (3 * (int)sizeof(double));
+  return d->staged_guess ? std::max(1, std::min(d->staged_guess + d->staged_guess / 16 + 32, budget)) : budget;
+}
+
 SearchTables search_tables(const mdgpu_domain *d) {
   SearchTables t;
   t.tstart = d->tstart;
@@ -685,7 +681,7 @@ SearchTables search_tables(const mdgpu_domain *d) {
   t.nrow = d->nrow;
   t.vslice0 = d->vslice0;
   t.rstride = kRangesPerCell * d->rmax;
-  t.lds_cap = lds_cap_for(d, 3 * sizeof(double), kSearchLdsKb);
+  t.lds_cap = search_lds_cap(d);
   return t;
 }
 
@@ -696,11 +692,11 @@ void launch_search_w(mdgpu_domain *d, const Bricks &B, SearchTables t) {
   if (d->search_cells) {
     allow_lds(k_search_cells<W>, shm);
     hipLaunchKernelGGL(k_search_cells<W>, dim3(d->nbrick), dim3(kWave * W), shm, d->stream, d->pos, B, t, d->S2,
-                       d->mcap, d->row_len, d->mask, d->i32);
+                       d->mcap, d->row_len, d->mask, &d->bs->err);
   } else {
     allow_lds(k_search_brick<W>, shm);
     hipLaunchKernelGGL(k_search_brick<W>, dim3(d->nbrick), dim3(kWave * W), shm, d->stream, d->pos, d->cell, B, t,
-                       d->S2, d->mcap, d->row_len, d->mask, d->i32);
+                       d->S2, d->mcap, d->row_len, d->mask, &d->bs->err);
   }
 }
 
@@ -714,6 +710,25 @@ int launch_search(mdgpu_domain *d, const Bricks &B, const SearchTables &t) {
     default: launch_search_w<16>(d, B, t); break;
   }
   return check_launch(d, "neighbour search");
+}
+
+int grow_glist(mdgpu_domain *d, long long n) {
+  n = std::max(n, 1024ll);
+  d->glist_cap = 0;
+  CHK(dalloc(d, &d->glist, (size_t)n));
+  if (!d->group) CHK(dalloc(d, &d->gimg, (size_t)n));
+  d->glist_cap = n;
+  return MDGPU_OK;
+}
+
+int grow_slots(mdgpu_domain *d, long long n) {
+  // kListTail readable entries past the last slice (the force kernels read ahead)
+  n = std::max(n, 1024ll);
+  d->nbr_cap = 0;
+  CHK(dalloc(d, &d->nbr, (size_t)(n + kListTail)));
+  CHK(dalloc(d, &d->nbr_in, (size_t)(n + kListTail)));
+  d->nbr_cap = n;
+  return MDGPU_OK;
 }
 
 // Room for a code per slot of the list and of the inner list.
@@ -733,10 +748,10 @@ int launch_emit(mdgpu_domain *d, const Bricks &B, const SearchTables &t) {
   if (codes) {
     CHK(ensure_codes(d));
     hipLaunchKernelGGL((k_emit_brick<kEmitWaves, true>), dim3(d->nbrick), dim3(kWave * kEmitWaves), 0, d->stream,
-                       d->cell, B, t, d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, d->ncode, d->i32);
+                       d->cell, B, t, d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, d->ncode, &d->bs->err);
   } else {
     hipLaunchKernelGGL((k_emit_brick<kEmitWaves, false>), dim3(d->nbrick), dim3(kWave * kEmitWaves), 0, d->stream,
-                       d->cell, B, t, d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, nullptr, d->i32);
+                       d->cell, B, t, d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, nullptr, &d->bs->err);
   }
   d->list_coded = codes;
   return check_launch(d, "neighbour list emit");
@@ -750,54 +765,6 @@ int launch_emit(mdgpu_domain *d, const Bricks &B, const SearchTables &t) {
 int recode_list(mdgpu_domain *d) {
   if (!rel_frame(d) || d->list_coded || !d->initialized || d->pn == 0 || d->nbr_slots == 0) return MDGPU_OK;
   return launch_emit(d, bricks_of(d), search_tables(d));
-}
-
-// The image gather list of the fused step (a unit's images come from other
-// units' particles: its steps refresh the halo).
-int image_glist(mdgpu_domain *d) {
-  if (d->group || d->gtotal == 0) return MDGPU_OK;
-  hipLaunchKernelGGL(k_image_glist, dim3(nblk(d->gtotal)), dim3(kBlock), 0, d->stream, d->glist, d->gtotal, d->pn,
-                     d->gsrc, d->gcode, d->gimg);
-  return check_launch(d, "image gather list");
-}
-
-// Rows of each brick by decreasing list length: permute the owned particles
-// (positions, momenta, ids, cells, row lengths) and remap the indices that
-// point at them (gather lists, ghost sources).  Ghosts keep their places.
-// With row_sort 0 the rows stay in cell order (rowsrc is the identity) and
-// nothing moves: a unit's owned particles keep the indices other units'
-// ghosts refer to.
-int order_rows(mdgpu_domain *d) {
-  hipStream_t st = d->stream;
-  const int pn = d->pn, ng = d->ng;
-  hipLaunchKernelGGL(k_brick_row_order, dim3(d->nbrick), dim3(kBlock), 0, st, d->row_len, d->row0, d->nrow,
-                     d->rowsrc, d->rowinv, d->row_sort);
-  if (d->row_sort == 0) {
-    CHK(image_glist(d));
-    return check_launch(d, "row order");
-  }
-  hipLaunchKernelGGL(k_gather_owned, dim3(nblk(pn)), dim3(kBlock), 0, st, d->rowsrc, pn, d->pos, d->mom, d->id,
-                     d->cell, d->rep, d->pos_tmp, d->mom_alt, d->id_alt, d->cell_alt, d->rep_alt);
-  hipLaunchKernelGGL(k_gather_int, dim3(nblk(pn)), dim3(kBlock), 0, st, d->rowsrc, pn, d->row_len, d->nimg);
-  if (ng > 0) {
-    HIPCHK(d, hipMemcpyAsync(d->pos_tmp + pn, d->pos + pn, ng * sizeof(double4), hipMemcpyDeviceToDevice, st));
-    HIPCHK(d, hipMemcpyAsync(d->cell_alt + pn, d->cell + pn, ng * sizeof(int), hipMemcpyDeviceToDevice, st));
-    // a unit's ghost sources index other units' rows: remapped once every
-    // unit of the group has ordered its own (remap_unit_ghosts)
-    if (!d->group)
-      hipLaunchKernelGGL(k_remap_owned, dim3(nblk(ng)), dim3(kBlock), 0, st, d->gsrc, (long long)ng, pn, d->rowinv);
-  }
-  if (d->gtotal > 0)
-    hipLaunchKernelGGL(k_remap_owned, dim3(nblk(d->gtotal)), dim3(kBlock), 0, st, d->glist, d->gtotal, pn,
-                       d->rowinv);
-  std::swap(d->pos, d->pos_tmp);
-  std::swap(d->mom, d->mom_alt);
-  std::swap(d->id, d->id_alt);
-  std::swap(d->cell, d->cell_alt);
-  std::swap(d->rep, d->rep_alt);
-  std::swap(d->row_len, d->nimg);
-  CHK(image_glist(d));
-  return check_launch(d, "row order");
 }
 
 // Cells per brick for a box of density rho (cubic bricks): the largest edge
@@ -915,9 +882,32 @@ int auto_bricks(mdgpu_domain *d) {
   return MDGPU_OK;
 }
 
-// Bin the owned particles (after the periodic wrap of each replica's box when
-// `wrap`) and put them in brick order, each cell's members by particle id.
-int bin_owned(mdgpu_domain *d, int wrap) {
+void swap_owned(mdgpu_domain *d) {
+  std::swap(d->pos, d->pos_tmp);
+  std::swap(d->mom, d->mom_alt);
+  std::swap(d->id, d->id_alt);
+  std::swap(d->cell, d->cell_alt);
+  std::swap(d->rep, d->rep_alt);
+}
+
+// The row order's arrays: the owned ones and the rows' list lengths.
+void swap_rows(mdgpu_domain *d) {
+  swap_owned(d);
+  std::swap(d->row_len, d->row_len_alt);
+}
+
+int begin_build(mdgpu_domain *d) {
+  hipLaunchKernelGGL(k_build_begin, dim3(nblk(d->ncell)), dim3(kBlock), 0, d->stream, d->bs, d->c_ocount, d->c_gcount,
+                     d->ncell);
+  return check_launch(d, "construction");
+}
+
+// Queue the binning of the owned particles (after the periodic wrap of each
+// replica's box when `wrap`) and their brick order, each cell's members by
+// particle id; with `images`, each particle's number of ghost images too.
+// Follows begin_build; on a position outside the box (kErrInvalidPosition) the
+// particles stay where they were and the caller swaps the arrays back.
+int queue_bin(mdgpu_domain *d, int wrap, bool images) {
   hipStream_t st = d->stream;
   invalidate(d);  // particles are reordered and wrapped
   const int pn = d->pn;
@@ -925,189 +915,219 @@ int bin_owned(mdgpu_domain *d, int wrap) {
   d->tn = pn;
   d->initialized = false;
   d->ghosts_ready = false;
-  HIPCHK(d, hipMemsetAsync(d->c_ocount, 0, sizeof(int) * d->ncell, st));
-  if (pn > 0) {
+  if (pn > 0)
     hipLaunchKernelGGL(k_wrap_bin, dim3(nblk(pn)), dim3(kBlock), 0, st, d->pos, pn, d->rep, d->reps, d->cell,
-                       d->slot, d->c_ocount, d->i32, wrap);
-  }
-  CHK(read_err_flags(d));
-  CHK(cell_sort(d, d->cell, pn, d->c_ocount, d->c_ostart, true, d->id));
+                       d->slot, d->c_ocount, &d->bs->err, wrap);
+  CHK(scan(d, ScanCells{d->c_ocount, d->cell_order, d->c_ostart, d->start_r}, d->ncell));
   if (pn > 0) {
-    hipLaunchKernelGGL(k_gather_owned, dim3(nblk(pn)), dim3(kBlock), 0, st, d->perm, pn, d->pos, d->mom, d->id,
-                       d->cell, d->rep, d->pos_tmp, d->mom_alt, d->id_alt, d->cell_alt, d->rep_alt);
-    std::swap(d->pos, d->pos_tmp);
-    std::swap(d->mom, d->mom_alt);
-    std::swap(d->id, d->id_alt);
-    std::swap(d->cell, d->cell_alt);
-    std::swap(d->rep, d->rep_alt);
+    hipLaunchKernelGGL(k_scatter_keys, dim3(nblk(pn)), dim3(kBlock), 0, st, d->cell, d->slot, d->c_ostart, pn, d->id,
+                       d->key, d->bs);
+    hipLaunchKernelGGL(k_sort_owned, dim3(nblk(pn)), dim3(kBlock), 0, st, d->key, d->c_ostart, d->c_ocount, pn,
+                       OwnedArrays{d->pos, d->mom, d->id, d->cell, d->rep},
+                       OwnedArrays{d->pos_tmp, d->mom_alt, d->id_alt, d->cell_alt, d->rep_alt},
+                       images ? d->nimg : nullptr, d->reps, d->SL, d->bs);
+    swap_owned(d);
+  }
+  return check_launch(d, "binning");
+}
+
+// Blocks for a launch over the ghosts, whose number only the device knows yet
+// (its loop strides over the rest): by the last construction's number, or the
+// room for them before the first.
+unsigned ghost_blocks(const mdgpu_domain *d) {
+  const int n = d->ng_last ? d->ng_last + d->ng_last / 8 : d->gcap;
+  return nblk(std::max(1024, std::min(n, d->gcap)));
+}
+
+// Queue the ghost images of a periodic domain or of every replica of an
+// ensemble (FindBorderParticles / SendBorderParticlesSub x 6), cell-sorted
+// after the owned particles (k_sort_owned counted them).
+int queue_images(mdgpu_domain *d) {
+  hipStream_t st = d->stream;
+  const int pn = d->pn;
+  if (pn > 0) {
+    CHK(scan(d, ScanImages{d->nimg, d->goff, d->bs, d->gcap}, pn, &d->bs->err));
+    // pos_tmp[0..ng) holds the unsorted images
+    hipLaunchKernelGGL(k_emit_images, dim3(nblk(pn)), dim3(kBlock), 0, st, d->pos, pn, d->rep, d->reps, d->SL,
+                       d->goff, d->bs, GhostArrays{d->t_gsrc, d->t_gcode, d->pos_tmp, d->t_gcell, d->slot, d->c_gcount});
+  }
+  CHK(scan(d, ScanArray<int, int>{d->c_gcount, d->c_gstart, nullptr}, d->ncell));
+  if (pn > 0) {
+    hipLaunchKernelGGL(k_scatter_keys, dim3(ghost_blocks(d)), dim3(kBlock), 0, st, d->t_gcell, d->slot, d->c_gstart,
+                       -1, nullptr, d->key, d->bs);
+    hipLaunchKernelGGL(k_sort_ghosts, dim3(ghost_blocks(d)), dim3(kBlock), 0, st, d->key, d->c_gstart, d->c_gcount,
+                       pn, d->t_gsrc, d->t_gcode, d->pos_tmp, d->t_gcell, d->gsrc, d->gcode, nullptr, d->pos, d->cell,
+                       d->bs);
+    if (d->nrep > 1)
+      hipLaunchKernelGGL(k_replica_ghosts, dim3(nblk(d->nrep)), dim3(kBlock), 0, st, d->goff, d->reps, d->nrep, d->bs,
+                         d->grng);
+  }
+  return check_launch(d, "ghost images");
+}
+
+// Queue the bricks' rows, slices and staged ranges.
+int queue_bricks(mdgpu_domain *d) {
+  CHK(scan(d, ScanBricks{d->brick_rank0, d->start_r, d->ncell, d->pn, d->row0, d->nrow, d->vslice0, d->bs}, d->nbrick));
+  hipLaunchKernelGGL(k_brick_ranges, dim3(nblk((long long)d->nbrick * kWave)), dim3(kBlock), 0, d->stream,
+                     bricks_of(d), CellTables{d->c_ostart, d->c_ocount, d->c_gstart, d->c_gcount}, d->nbrick, d->pn,
+                     d->nrow, d->tstart, d->tbase, d->nrange, d->btotal, d->bs);
+  return scan(d, ScanGather{d->btotal, d->gbase, d->nbrick, d->glist_cap, d->bs}, d->nbrick, &d->bs->err);
+}
+
+int queue_glist(mdgpu_domain *d) {
+  hipLaunchKernelGGL(k_brick_glist, dim3(d->nbrick), dim3(kBlock), 0, d->stream, kRangesPerCell * d->rmax, d->tstart,
+                     d->tbase, d->nrange, d->gbase, d->glist, d->bs);
+  return check_launch(d, "gather lists");
+}
+
+// Queue the rows' order inside their bricks (by decreasing list length) and
+// what follows from it: the owned particles moved, the slices' lengths and
+// first slots, the indices that point at owned particles, PairList::Init's
+// snapshot.  Ghosts keep their places.  With row_sort 0 the rows stay in cell
+// order and nothing moves.
+int queue_rows(mdgpu_domain *d) {
+  hipStream_t st = d->stream;
+  const RowArrays in{{d->pos, d->mom, d->id, d->cell, d->rep}, d->row_len};
+  const RowArrays out{{d->pos_tmp, d->mom_alt, d->id_alt, d->cell_alt, d->rep_alt}, d->row_len_alt};
+  hipLaunchKernelGGL(k_order_rows, dim3(d->nbrick), dim3(kBlock), 0, st, d->row0, d->nrow, d->vslice0, d->rowsrc,
+                     d->rowinv, d->row_sort, in, d->row_sort ? out : in, d->pos_old, d->slen, d->bsum, d->bs);
+  CHK(scan(d, ScanSlots{d->slen, d->sbase, d->nbr_cap, d->bs}, (long long)d->pn / kWave + d->nbrick, &d->bs->err));
+  const double4 *pos_in = d->pos;
+  const int *cell_in = d->cell;
+  if (d->row_sort) swap_rows(d);
+  d->rows_swapped = d->row_sort != 0;
+  const long long work = std::max<long long>(ghost_blocks(d) * (long long)kBlock, d->gtotal + d->gtotal / 16);
+  hipLaunchKernelGGL(k_remap, dim3(nblk(std::max(1ll << 14, work))), dim3(kBlock), 0, st, d->rowinv, d->pn, d->gsrc,
+                     d->t_gsrc, d->gcode, d->glist, d->group ? nullptr : d->gimg, pos_in, d->pos, cell_in, d->cell,
+                     d->pos_old, d->bs);
+  std::swap(d->gsrc, d->t_gsrc);
+  return check_launch(d, "row order");
+}
+
+// Room for what a construction will need, before it runs: masks for every row,
+// slices for the rows there are, and, the first time, gather-list entries and
+// list slots by the mean density (later ones have the last construction's and
+// an eighth more).
+int ensure_build(mdgpu_domain *d) {
+  const long long sl = (long long)d->pn / kWave + d->nbrick + 1;
+  if (sl > d->slice_cap) {
+    const int sc = (int)(sl + sl / 8 + 64);
+    d->slice_cap = 0;
+    CHK(dalloc(d, &d->slen, sc));
+    CHK(dalloc(d, &d->slen_in, sc));
+    CHK(dalloc(d, &d->sbase, sc));
+    d->slice_cap = sc;
+  }
+  const size_t need = (size_t)d->pn * d->mcap;
+  if (!d->mask || need > d->mask_cap) {
+    d->mask_cap = 0;
+    CHK(dalloc(d, &d->mask, need + need / 8));
+    d->mask_cap = need + need / 8;
+  }
+  double entries = 0.0, slots = 0.0;
+  for (int r = 0; r < d->nrep; r++) {
+    const Replica &R = d->rh[r];
+    const double pn = d->nrep == 1 ? d->pn : R.pn, rho = pn / (R.L[0] * R.L[1] * R.L[2]);
+    entries += rho * R.w[0] * R.w[1] * R.w[2] * R.nb[0] * R.nb[1] * R.nb[2] *
+               ((R.bd[0] + 2) * (R.bd[1] + 2) * (R.bd[2] + 2));
+    slots += pn * (rho * (4.0 / 3.0) * M_PI * d->SL * d->SL * d->SL * 1.25 + 16.0);
+  }
+  if (d->glist_cap == 0) CHK(grow_glist(d, (long long)(1.1 * entries)));
+  if (d->nbr_cap == 0) CHK(grow_slots(d, (long long)slots));
+  if (d->staged_guess == 0 && d->nrep == 1 && d->pn > 0) {
+    // new bricks: the mean neighbourhood and a sixth more
+    const Replica &R = d->rh[0];
+    d->staged_guess = (int)std::min(65534.0, 1.16 * (d->pn / (R.L[0] * R.L[1] * R.L[2])) * R.w[0] * R.w[1] * R.w[2] *
+                                                 ((R.bd[0] + 2) * (R.bd[1] + 2) * (R.bd[2] + 2)));
   }
   return MDGPU_OK;
 }
 
-// The ghost images of a periodic domain or of every replica of an ensemble
-// (FindBorderParticles / SendBorderParticlesSub x 6), cell-sorted after the
-// owned particles.
-int place_images(mdgpu_domain *d) {
-  hipStream_t st = d->stream;
-  const int pn = d->pn;
-  CHK(ensure_scan(d, std::max(pn, d->ncell)));
-  long long ngl = 0;
-  if (pn > 0) {
-    hipLaunchKernelGGL(k_count_images, dim3(nblk(pn)), dim3(kBlock), 0, st, d->pos, pn, d->rep, d->reps, d->SL,
-                       d->nimg);
-    exclusive_scan<int, int>(d->nimg, d->goff, pn, d->scan_scratch, d->i64, st);
-    CHK(read_total(d, &ngl));
+// The stages of a construction after the binning, in the order they are queued.
+enum BuildStage { kStageImages, kStageBricks, kStageGlist, kStageSearch, kStageEmit };
+
+int queue_from(mdgpu_domain *d, BuildStage from) {
+  if (from <= kStageImages) CHK(queue_images(d));
+  if (from <= kStageBricks) CHK(queue_bricks(d));
+  if (from <= kStageGlist) CHK(queue_glist(d));
+  const bool rows = d->pn > 0;
+  if (rows && from <= kStageSearch) {
+    CHK(launch_search(d, bricks_of(d), search_tables(d)));
+    CHK(queue_rows(d));
   }
-  if (ngl + pn + 1 > kMaxParticles) {
-    d->err = "particle capacity exceeded (owned + ghosts)";
-    return MDGPU_ERR_CAPACITY;
-  }
-  const int ng = (int)ngl;
-  CHK(ensure_ghosts(d, ng));
-  HIPCHK(d, hipMemsetAsync(d->c_gcount, 0, sizeof(int) * d->ncell, st));
-  if (ng > 0) {
-    // pos_tmp[0..ng) holds the unsorted images
-    hipLaunchKernelGGL(k_emit_images, dim3(nblk(pn)), dim3(kBlock), 0, st, d->pos, pn, d->rep, d->reps, d->SL,
-                       d->goff, ng, d->t_gsrc, d->t_gcode, d->pos_tmp, d->t_gcell, d->slot, d->c_gcount);
-    CHK(check_launch(d, "emit images"));
-    CHK(cell_sort(d, d->t_gcell, ng, d->c_gcount, d->c_gstart, false, nullptr));
-    hipLaunchKernelGGL(k_gather_ghosts, dim3(nblk(ng)), dim3(kBlock), 0, st, d->perm, ng, pn, d->t_gsrc,
-                       d->t_gcode, d->pos_tmp, d->t_gcell, d->gsrc, d->gcode, d->pos, d->cell);
-  } else {
-    exclusive_scan<int, int>(d->c_gcount, d->c_gstart, d->ncell, d->scan_scratch, nullptr, st);
-  }
-  d->ng = ng;
-  d->tn = pn + ng;
-  if (d->nrep > 1 && pn > 0)
-    hipLaunchKernelGGL(k_replica_ghosts, dim3(nblk(d->nrep)), dim3(kBlock), 0, st, d->goff, d->reps, d->nrep, ng,
-                       d->grng);
-  d->ghosts_ready = true;
-  return check_launch(d, "ghost images");
+  if (rows) CHK(launch_emit(d, bricks_of(d), search_tables(d)));
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kPublishThreads), 0, d->stream, d->bs, d->btotal, rows ? d->bsum : nullptr,
+                     d->nbrick, d->h_bs);
+  return check_launch(d, "construction");
 }
 
-// Bricks, the neighbour list and the PairList::Init snapshot for the owned
-// particles and ghosts in place (bin_owned, then place_images or a unit's
-// ghost placement).
-int build_lists(mdgpu_domain *d) {
-  hipStream_t st = d->stream;
+// Queue a construction from stage `from` on and wait for it once; where it
+// stopped for want of room, make it and queue the rest again.
+int finish_build(mdgpu_domain *d, BuildStage from) {
   const int pn = d->pn;
-  HIPCHK(d, hipMemsetAsync(d->i32, 0, sizeof(int) * 4, st));
-  // 4. bricks: rows, slices, staged ranges
-  const Bricks B = bricks_of(d);
-  const CellTables T{d->c_ostart, d->c_ocount, d->c_gstart, d->c_gcount};
-  hipLaunchKernelGGL(k_brick_rows, dim3(nblk(d->nbrick)), dim3(kBlock), 0, st, d->brick_rank0, d->start_r,
-                     d->nbrick, d->ncell, pn, d->row0, d->nrow, d->nsl);
-  CHK(ensure_scan(d, d->nbrick));
-  exclusive_scan<int, int>(d->nsl, d->vslice0, d->nbrick, d->scan_scratch, d->i64, st);
-  long long nsl_total = 0;
-  CHK(read_total(d, &nsl_total));
-  d->nslice = (int)nsl_total;
-  if (d->nslice + 1 > d->slice_cap) {
-    const int sc = d->nslice + d->nslice / 4 + 64;
-    CHK(dalloc(d, &d->slen, sc));
-    CHK(dalloc(d, &d->slen_in, sc));
-    CHK(dalloc(d, &d->sbase, sc));
-    CHK(dalloc(d, &d->slots64, sc));
-    CHK(dalloc(d, &d->slice_brick, sc));
-    CHK(dalloc(d, &d->spart, nblk(sc)));
-    d->slice_cap = sc;
-  }
-  hipLaunchKernelGGL(k_slice_brick, dim3(nblk(d->nbrick)), dim3(kBlock), 0, st, d->vslice0, d->nsl, d->nbrick,
-                     d->slice_brick);
-  hipLaunchKernelGGL(k_brick_ranges, dim3(nblk((long long)d->nbrick * kWave)), dim3(kBlock), 0, st, B, T,
-                     d->nbrick, pn, d->tstart, d->tbase, d->nrange, d->btotal, d->bpart);
-  hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(kBlock), 0, st, d->bpart, d->nbrick, d->u64 + 2);
-  // gather lists: gbase = exclusive scan of the staged counts, gbase[nbrick] = total;
-  // the largest neighbourhood and the total are read after one wait
-  exclusive_scan<int, long long>(d->btotal, d->gbase, d->nbrick, d->scan_scratch, d->i64, st);
-  HIPCHK(d, hipMemcpyAsync(d->gbase + d->nbrick, d->i64, sizeof(long long), hipMemcpyDeviceToDevice, st));
-  HIPCHK(d, hipMemcpyAsync(d->h_u64 + 2, d->u64 + 2, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-  long long gtotal = 0;
-  CHK(read_total(d, &gtotal));
-  double mstaged = 0.0;
-  std::memcpy(&mstaged, d->h_u64 + 2, sizeof(double));
-  d->max_staged = (int)mstaged;
-  if (d->max_staged > 65534) {
-    d->err = "a brick's neighbourhood exceeds 16-bit indexing (extreme local density): use smaller bricks";
-    return MDGPU_ERR_CAPACITY;
-  }
-  d->gtotal = gtotal;
-  if (gtotal > d->glist_cap) {
-    const long long gc = gtotal + gtotal / 8 + 1024;
-    d->glist_cap = 0;
-    CHK(dalloc(d, &d->glist, (size_t)gc));
-    if (!d->group) CHK(dalloc(d, &d->gimg, (size_t)gc));
-    d->glist_cap = gc;
-  }
-  hipLaunchKernelGGL(k_brick_glist, dim3(d->nbrick), dim3(kBlock), 0, st, kRangesPerCell * d->rmax, d->tstart,
-                     d->tbase, d->nrange, d->gbase, d->glist);
-  // 5. MeshList::MakeList: full neighbour list in sliced-ELL layout
-  long long slots = 0;
-  int scap = 0;
-  const SearchTables STb = search_tables(d);
-  if (pn > 0) {
-    // candidate masks: retried with room for more candidates if a row overflows
-    for (;;) {
-      const size_t need = (size_t)pn * d->mcap;
-      if (!d->mask || need > d->mask_cap) {
-        d->mask_cap = 0;
-        CHK(dalloc(d, &d->mask, need + need / 8));
-        d->mask_cap = need + need / 8;
+  CHK(ensure_build(d));
+  d->rows_swapped = false;
+  for (;;) {
+    CHK(queue_from(d, from));
+    CHK(sync(d));
+    const BuildState S = *d->h_bs;
+    if ((S.err & kErrBeforeRows) && from <= kStageSearch && pn > 0) {
+      if (d->rows_swapped) swap_rows(d);  // nothing moved
+      std::swap(d->gsrc, d->t_gsrc);
+      d->rows_swapped = false;
+    }
+    if (S.err & kErrInvalidPosition) {
+      if (from == kStageImages && pn > 0) swap_owned(d);  // k_sort_owned did not run
+      return build_error(d, S.err);
+    }
+    if (S.err & kErrGhostCap) {
+      if (S.ng + pn + 1 > kMaxParticles) {
+        d->err = "particle capacity exceeded (owned + ghosts)";
+        return MDGPU_ERR_CAPACITY;
       }
-      HIPCHK(d, hipMemsetAsync(d->i32, 0, sizeof(int), st));
-      CHK(launch_search(d, B, STb));
-      HIPCHK(d, hipMemcpyAsync(d->h_i32, d->i32, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
-      CHK(sync(d));
-      if (!(d->h_i32[0] & kErrSearchCap)) break;
+      CHK(ensure_ghosts(d, (int)S.ng));
+      from = kStageImages;
+    } else if (S.err & kErrGatherCap) {
+      CHK(grow_glist(d, S.gtotal + S.gtotal / 8 + 1024));
+      from = kStageBricks;
+    } else if (S.err & kErrSearchCap) {
       if (d->mcap >= (1 << 16)) {
         d->err = "a row has too many neighbour candidates";
         return MDGPU_ERR_CAPACITY;
       }
       d->mcap *= 2;
+      CHK(ensure_build(d));
+      from = kStageSearch;
+    } else if (S.err & kErrSlotCap) {
+      CHK(grow_slots(d, S.slots + S.slots / 8 + 1024));
+      from = kStageEmit;
+    } else {
+      CHK(build_error(d, S.err));
+      break;
     }
-    CHK(order_rows(d));
-    // scratch for both scans before either is queued (a reallocation frees
-    // the buffer a queued scan would use)
-    CHK(ensure_scan(d, std::max<long long>(pn, d->nslice)));
-    // number of listed (row, partner) entries, for accounting: copied now,
-    // read after the next wait
-    exclusive_scan<int, long long>(d->row_len, d->key, pn, d->scan_scratch, d->i64, st);
-    HIPCHK(d, hipMemcpyAsync(d->h_i64 + 1, d->i64, sizeof(long long), hipMemcpyDeviceToHost, st));
-    hipLaunchKernelGGL(k_slice_len, dim3(nblk(d->nslice)), dim3(kBlock), 0, st, d->row_len, d->slice_brick,
-                       d->vslice0, d->row0, d->nrow, d->nslice, d->slen, d->slots64, d->spart);
-    hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(kBlock), 0, st, d->spart, (int)nblk(d->nslice), d->u64 + 3);
-    exclusive_scan<long long, long long>(d->slots64, d->sbase, d->nslice, d->scan_scratch, d->i64, st);
-    // the slots and the longest slice after one wait
-    HIPCHK(d, hipMemcpyAsync(d->h_u64 + 3, d->u64 + 3, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-    CHK(read_total(d, &slots));
-    d->nbr_entries = d->h_i64[1];
-    double smax = 0.0;
-    std::memcpy(&smax, d->h_u64 + 3, sizeof(double));
-    scap = (int)smax;
-  } else {
-    d->nbr_entries = 0;
+    HIPCHK(d, hipMemsetAsync(&d->bs->err, 0, sizeof(int), d->stream));
   }
-  if (slots > d->nbr_cap) {
-    // kListTail readable entries past the last slice (the force kernels read ahead)
-    const long long nc = slots + slots / 8 + 1024;
-    CHK(dalloc(d, &d->nbr, (size_t)(nc + kListTail)));
-    CHK(dalloc(d, &d->nbr_in, (size_t)(nc + kListTail)));
-    d->nbr_cap = nc;
+  const BuildState &S = *d->h_bs;
+  d->max_staged = S.max_staged;
+  if (d->max_staged > 65534) {
+    d->err = "a brick's neighbourhood exceeds 16-bit indexing (extreme local density): use smaller bricks";
+    return MDGPU_ERR_CAPACITY;
   }
-  d->nbr_slots = slots;
-  if (pn > 0 && scap > 0) CHK(launch_emit(d, B, STb));
-  else d->list_coded = false;  // no slots to code
-  CHK(check_launch(d, "neighbour list"));
-  // PairList::Init: snapshot of owned + ghost positions (pairlist.cc:11-23)
-  if (d->tn > 0)
-    hipLaunchKernelGGL(k_copy_pos, dim3(nblk(d->tn)), dim3(kBlock), 0, st, d->pos, d->pos_old, d->tn);
-  CHK(read_err_flags(d));
+  d->staged_guess = std::max(1, d->max_staged);
+  d->ng = d->ng_last = (int)S.ng;
+  d->tn = pn + d->ng;
+  d->nslice = S.nslice;
+  d->gtotal = S.gtotal;
+  d->nbr_slots = pn > 0 ? S.slots : 0;
+  d->nbr_entries = pn > 0 ? S.entries : 0;
+  if (d->nbr_slots == 0) d->list_coded = false;  // no slots to code
+  d->ghosts_ready = true;
   d->initialized = true;
   d->buffer_length = d->margin;
   d->lifetime = 0;
-  for (ReplicaState &S : d->rst) {
-    S.buffer_length = d->margin;
-    S.lifetime = 0;
+  for (ReplicaState &S2 : d->rst) {
+    S2.buffer_length = d->margin;
+    S2.lifetime = 0;
   }
   d->vmax_valid = false;
   d->since_build = 0;
@@ -1127,13 +1147,23 @@ int make_pair_list(mdgpu_domain *d) {
                "(mdgpu_group_make_pair_list, or the mdgpu_unit_* sequence)";
       return MDGPU_ERR_ARGUMENT;
     }
-    return build_lists(d);
+    return finish_build(d, kStageBricks);
   }
   CHK(auto_bricks(d));
-  HIPCHK(d, hipMemsetAsync(d->i32, 0, sizeof(int) * 4, d->stream));
-  CHK(bin_owned(d, 1));
-  CHK(place_images(d));
-  return build_lists(d);
+  if (d->ng_last == 0 && d->pn > 0) {
+    // the first construction: room for the images of a uniform density
+    double g = 0.0;
+    for (int r = 0; r < d->nrep; r++) {
+      const Replica &R = d->rh[r];
+      const double pn = d->nrep == 1 ? d->pn : R.pn;
+      g += pn * ((1.0 + 2.0 * d->SL / R.L[0]) * (1.0 + 2.0 * d->SL / R.L[1]) * (1.0 + 2.0 * d->SL / R.L[2]) - 1.0);
+    }
+    const double most = (double)(kMaxParticles - 1 - d->cap);
+    CHK(ensure_ghosts(d, (int)std::min(1.1 * g, most)));
+  }
+  CHK(begin_build(d));
+  CHK(queue_bin(d, 1, true));
+  return finish_build(d, kStageImages);
 }
 
 // max |p|^2 of a single domain; after a fused step it is the one the step's
@@ -2153,7 +2183,7 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
     mdgpu_destroy(d);
     return r;
   }
-  if ((r = dalloc(d, &d->u64, 4)) || (r = dalloc(d, &d->i64, 4)) || (r = dalloc(d, &d->i32, 4)) ||
+  if ((r = dalloc(d, &d->bs, 1)) || (r = dalloc(d, &d->scan_ticket, 1)) || (r = dalloc(d, &d->u64, 4)) || (r = dalloc(d, &d->i64, 4)) || (r = dalloc(d, &d->i32, 4)) ||
       (r = dalloc(d, &d->d3, 4)) || (r = dalloc(d, &d->cand, (size_t)d->check_list_length + 1))) {
     mdgpu_destroy(d);
     return r;
@@ -2163,7 +2193,8 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
     mdgpu_destroy(d);
     return r ? r : MDGPU_ERR_HIP;
   }
-  if (hipHostMalloc((void **)&d->h_u64, 4 * sizeof(unsigned long long)) != hipSuccess ||
+  if (hipHostMalloc((void **)&d->h_bs, sizeof(BuildState)) != hipSuccess ||
+      hipHostMalloc((void **)&d->h_u64, 4 * sizeof(unsigned long long)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_i64, 4 * sizeof(long long)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_i32, 4 * sizeof(int)) != hipSuccess ||
       hipHostMalloc((void **)&d->h_d3, 4 * sizeof(double)) != hipSuccess) {
@@ -2172,6 +2203,8 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
   }
   std::memset(d->h_rr, 0, nrep * sizeof(RunRep));
   (void)hipMemset(d->rr, 0, nrep * sizeof(RunRep));
+  (void)hipMemset(d->bs, 0, sizeof(BuildState));
+  (void)hipMemset(d->scan_ticket, 0, sizeof(unsigned));
   (void)hipMemset(d->i32, 0, 4 * sizeof(int));
   (void)hipMemset(d->u64, 0, 4 * sizeof(unsigned long long));
   (void)hipMemset(d->clock, 0, sizeof(unsigned long long));
@@ -2206,10 +2239,9 @@ int unit_send(mdgpu_domain *d, int dir, int *nsend) {
   d->st_n = 0;
   if (pn > 0) {
     const int a = dir >> 1;
-    CHK(ensure_scan(d, pn));
     hipLaunchKernelGGL(k_leave_flags, dim3(nblk(pn)), dim3(kBlock), 0, st, d->pos, pn, dir, d->rs[a], d->re[a],
                        d->nimg);
-    exclusive_scan<int, int>(d->nimg, d->goff, pn, d->scan_scratch, d->i64, st);
+    CHK(scan(d, ScanArray<int, int>{d->nimg, d->goff, d->i64}, pn));
     long long ns = 0;
     CHK(read_total(d, &ns));
     if (ns > d->st_cap) {
@@ -2265,11 +2297,15 @@ int unit_receive(mdgpu_domain *d, mdgpu_domain *src) {
 int unit_adjust(mdgpu_domain *d) {
   hipStream_t st = d->stream;
   CHK(auto_bricks(d));
-  HIPCHK(d, hipMemsetAsync(d->i32, 0, sizeof(int) * 4, st));
+  CHK(begin_build(d));
   if (d->pn > 0)
     hipLaunchKernelGGL(k_unit_wrap, dim3(nblk(d->pn)), dim3(kBlock), 0, st, d->pos, d->pn, d->L[0], d->L[1],
-                       d->L[2], d->i32);
-  return bin_owned(d, 0);
+                       d->L[2], &d->bs->err);
+  CHK(queue_bin(d, 0, false));
+  HIPCHK(d, hipMemcpyAsync(d->h_bs, d->bs, sizeof(BuildState), hipMemcpyDeviceToHost, st));
+  CHK(sync(d));
+  if ((d->h_bs->err & kErrInvalidPosition) && d->pn > 0) swap_owned(d);  // k_sort_owned did not run
+  return build_error(d, d->h_bs->err);
 }
 
 // The unit's ghosts: what MDManager's six FindBorderParticles /
@@ -2317,13 +2353,14 @@ int unit_ghosts(mdgpu_domain *d) {
     d->ucap = c;
   }
   HIPCHK(d, hipMemcpyAsync(d->src_tab, d->h_src_tab, nsrc * sizeof(SrcUnit), hipMemcpyHostToDevice, st));
-  CHK(ensure_scan(d, std::max<long long>(total, d->ncell)));
   long long ngl = 0;
   if (total > 0) {
     hipLaunchKernelGGL(k_unit_count, dim3(nblk(total)), dim3(kBlock), 0, st, d->src_tab, nsrc, (int)total,
                        d->unit_slot, d->SL, d->ucnt);
-    exclusive_scan<int, int>(d->ucnt, d->uoff, (int)total, d->scan_scratch, d->i64, st);
-    CHK(read_total(d, &ngl));
+    CHK(scan(d, ScanArray<int, int>{d->ucnt, d->uoff, &d->bs->ng}, total));
+    HIPCHK(d, hipMemcpyAsync(d->h_bs, d->bs, sizeof(BuildState), hipMemcpyDeviceToHost, st));
+    CHK(sync(d));
+    ngl = d->h_bs->ng;
   }
   if (ngl + pn + 1 > kMaxParticles) {
     d->err = "particle capacity exceeded (owned + ghosts)";
@@ -2337,20 +2374,23 @@ int unit_ghosts(mdgpu_domain *d) {
     d->h_src_tab[d->unit_slot].pos = d->pos;
     HIPCHK(d, hipMemcpyAsync(d->src_tab, d->h_src_tab, nsrc * sizeof(SrcUnit), hipMemcpyHostToDevice, st));
   }
-  HIPCHK(d, hipMemsetAsync(d->c_gcount, 0, sizeof(int) * d->ncell, st));
+  HIPCHK(d, hipMemsetAsync(d->c_gcount, 0, sizeof(int) * d->ncell, st));  // placed twice: counted twice
   if (ng > 0) {
     // pos_tmp[0..ng) holds the unsorted images
     hipLaunchKernelGGL(k_unit_emit, dim3(nblk(total)), dim3(kBlock), 0, st, d->src_tab, nsrc, (int)total,
                        d->unit_slot, d->SL, d->uoff, ng, g->L[0], g->L[1], g->L[2], d->reps, d->t_gsrc, d->t_gcode,
                        d->pos_tmp, d->t_gcell, d->slot, d->c_gcount);
     CHK(check_launch(d, "unit ghosts"));
-    CHK(cell_sort(d, d->t_gcell, ng, d->c_gcount, d->c_gstart, false, nullptr));
-    hipLaunchKernelGGL(k_gather_unit_ghosts, dim3(nblk(ng)), dim3(kBlock), 0, st, d->perm, ng, pn, d->t_gsrc,
-                       d->t_gcode, d->pos_tmp, d->t_gcell, d->gsrc, d->gcode, d->gunit, d->pos, d->cell);
-  } else {
-    exclusive_scan<int, int>(d->c_gcount, d->c_gstart, d->ncell, d->scan_scratch, nullptr, st);
   }
-  d->ng = ng;
+  CHK(scan(d, ScanArray<int, int>{d->c_gcount, d->c_gstart, nullptr}, d->ncell));
+  if (ng > 0) {
+    hipLaunchKernelGGL(k_scatter_keys, dim3(nblk(ng)), dim3(kBlock), 0, st, d->t_gcell, d->slot, d->c_gstart, ng,
+                       nullptr, d->key, d->bs);
+    hipLaunchKernelGGL(k_sort_ghosts, dim3(nblk(ng)), dim3(kBlock), 0, st, d->key, d->c_gstart, d->c_gcount, pn,
+                       d->t_gsrc, d->t_gcode, d->pos_tmp, d->t_gcell, d->gsrc, d->gcode, d->gunit, d->pos, d->cell,
+                       d->bs);
+  }
+  d->ng = d->ng_last = ng;
   d->tn = pn + ng;
   d->ghosts_ready = true;
   d->ghost_epoch = g->epoch;
@@ -3049,17 +3089,17 @@ int mdgpu_destroy(mdgpu_domain *d) {
   if (d->stream) (void)hipStreamSynchronize(d->stream);
   void *bufs[] = {d->pos,     d->pos_tmp,     d->pos_next,    d->rel_next,  d->pos_old,     d->mom,       d->mom_alt,  d->rel,
                   d->rel_tmp, d->id,          d->id_alt,      d->cell,      d->cell_alt, d->gsrc,
-                  d->gcode,   d->c_ocount,    d->c_ostart,    d->c_gcount,  d->c_gstart, d->count_r,
-                  d->start_r, d->org,         d->rank,        d->brick_of_cell, d->brick_rank0, d->row0,
-                  d->nrow,    d->nsl,         d->vslice0,     d->slice_brick, d->tstart,  d->tbase,
-                  d->nrange,  d->btotal,      d->gbase,       d->glist,     d->mask,     d->spart,
-                  d->nbr,     d->ncode,       d->sbase,       d->slots64,   d->slen,     d->row_len,
-                  d->rowsrc,  d->rowinv,      d->slot,        d->perm,      d->nimg,     d->goff,
-                  d->t_gsrc,  d->t_gcode,     d->t_gcell,     d->key,       d->scan_scratch, d->disp,
+                  d->gcode,   d->c_ocount,    d->c_ostart,    d->c_gcount,  d->c_gstart, d->bsum,
+                  d->start_r, d->org,         d->cell_order,  d->brick_rank0, d->row0,
+                  d->nrow,    d->bs,          d->vslice0,     d->scan_status, d->tstart,  d->tbase,
+                  d->nrange,  d->btotal,      d->gbase,       d->glist,     d->mask,     d->scan_ticket,
+                  d->nbr,     d->ncode,       d->sbase,       d->slen,     d->row_len,
+                  d->rowsrc,  d->rowinv,      d->slot,        d->row_len_alt, d->nimg,     d->goff,
+                  d->t_gsrc,  d->t_gcode,     d->t_gcell,     d->key,       d->disp,
                   d->partial, d->maxpart,     d->bpart,       d->cand,      d->u64,      d->i64,
                   d->i32,     d->d3,          d->reps,        d->brep,      d->rep,      d->rep_alt,
                   d->grng,    d->rep_v2,      d->rep_out,     d->which,     d->rep_exp,  d->clock,
-                  d->perm_in, d->nbr_in,      d->ncode_in,    d->slen_in,   d->chk_dmax, d->chk_cnt,
+                  d->nbr_in,      d->ncode_in,    d->slen_in,   d->chk_dmax, d->chk_cnt,
                   d->chk_cand, d->gate,       d->gimg,       d->rr,          d->run_cand,  d->dpart,     d->xfer,     d->gunit,
                   d->st_pos,  d->st_mom,      d->st_id,       d->src_tab,   d->ucnt,     d->uoff,
                   d->rep_factor};
@@ -3071,6 +3111,7 @@ int mdgpu_destroy(mdgpu_domain *d) {
                   (void *)d->h_gate, (void *)d->h_rr, (void *)d->h_rep_factor,
                   (void *)d->h_chk_dmax})
     if (h) (void)hipHostFree(h);
+  if (d->h_bs) (void)hipHostFree(d->h_bs);
   if (d->h_u64) (void)hipHostFree(d->h_u64);
   if (d->h_i64) (void)hipHostFree(d->h_i64);
   if (d->h_i32) (void)hipHostFree(d->h_i32);

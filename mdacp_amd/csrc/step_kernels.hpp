@@ -370,10 +370,6 @@ __global__ void k_candidate_pairs(const double4 *__restrict__ pos, const double4
   if (dr2 < CL2) atomicOr(flag, 1);
 }
 
-__global__ void k_copy_pos(const double4 *__restrict__ a, double4 *__restrict__ b, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = a[i];
-}
 
 __global__ void k_scale_pos(double4 *__restrict__ pos, int pn, double alpha) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -906,11 +902,12 @@ __global__ void k_zero_check(unsigned long long *__restrict__ dmax, int *__restr
 
 // Ghost ranges of each replica after a construction: replica r's images are
 // [goff[p0], goff[p0 + pn]) (goff = exclusive scan of the image counts over
-// the replica-major owned order; total = the number of images).
+// the replica-major owned order; bs->ng = the number of images).
 __global__ void k_replica_ghosts(const int *__restrict__ goff, const Replica *__restrict__ reps, int nrep,
-                                 int total, int2 *__restrict__ grng) {
+                                 const BuildState *__restrict__ bs, int2 *__restrict__ grng) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nrep) return;
+  if (r >= nrep || bs->err) return;
+  const int total = (int)bs->ng;
   const Replica &R = reps[r];
   const int a = R.pn > 0 ? goff[R.p0] : 0;
   int e = total;
