@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kPublishThreads) void k_publish(const BuildState *_
   }
 }
 
-constexpr int kEmitWaves = 4;  // wavefronts per brick workgroup of k_emit_brick
+constexpr int kEmitFewBricks = 4;  // bricks per CU below which k_emit_brick runs 16 wavefronts per brick, not 4
 
 // A row's walk through its candidate mask during the emit: the current
 // 64-bit mask word (bits already taken cleared) and the next one, loaded ahead;

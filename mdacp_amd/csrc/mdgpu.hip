@@ -741,18 +741,25 @@ int ensure_codes(mdgpu_domain *d) {
   return MDGPU_OK;
 }
 
-// one wavefront per 64-row slice, four per brick workgroup; with codes for
-// the cell-frame mixed kick only (recode_list gives them to a built list)
+template <int W>
+void launch_emit_w(mdgpu_domain *d, const Bricks &B, const SearchTables &t, bool codes) {
+  if (codes)
+    hipLaunchKernelGGL((k_emit_brick<W, true>), dim3(d->nbrick), dim3(kWave * W), 0, d->stream, d->cell, B, t,
+                       d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, d->ncode, &d->bs->err);
+  else
+    hipLaunchKernelGGL((k_emit_brick<W, false>), dim3(d->nbrick), dim3(kWave * W), 0, d->stream, d->cell, B, t,
+                       d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, nullptr, &d->bs->err);
+}
+
+// One wavefront per 64-row slice, four per brick workgroup, or sixteen where
+// the bricks do not fill the CUs several times: a wavefront's slices, about 30
+// us each alone, then run side by side.  With codes for the cell-frame mixed
+// kick only (recode_list gives them to a built list).
 int launch_emit(mdgpu_domain *d, const Bricks &B, const SearchTables &t) {
   const bool codes = rel_frame(d);
-  if (codes) {
-    CHK(ensure_codes(d));
-    hipLaunchKernelGGL((k_emit_brick<kEmitWaves, true>), dim3(d->nbrick), dim3(kWave * kEmitWaves), 0, d->stream,
-                       d->cell, B, t, d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, d->ncode, &d->bs->err);
-  } else {
-    hipLaunchKernelGGL((k_emit_brick<kEmitWaves, false>), dim3(d->nbrick), dim3(kWave * kEmitWaves), 0, d->stream,
-                       d->cell, B, t, d->rowsrc, d->mask, d->mcap, d->sbase, d->slen, d->nbr, nullptr, &d->bs->err);
-  }
+  if (codes) CHK(ensure_codes(d));
+  if (d->nbrick < kEmitFewBricks * d->num_cu) launch_emit_w<16>(d, B, t, codes);
+  else launch_emit_w<4>(d, B, t, codes);
   d->list_coded = codes;
   return check_launch(d, "neighbour list emit");
 }
