@@ -3157,54 +3157,6 @@ int mdgpu_set_precision(mdgpu_domain *d, int precision) {
   return recode_list(d);
 }
 
-int mdgpu_add_particles(mdgpu_domain *d, int n, const double *q, const double *p, const int *type) {
-  if (!d || n < 0 || (n > 0 && !q)) return MDGPU_ERR_ARGUMENT;
-  if (d->nrep > 1) {
-    d->err = "an ensemble's particles are set when it is created";
-    return MDGPU_ERR_ARGUMENT;
-  }
-  invalidate(d);  // the next fused step recomputes its first half drift
-  std::vector<double4> hq, hp;
-  std::vector<int> hid;
-  hq.reserve(n);
-  for (int i = 0; i < n; i++) {
-    const double *x = q + 3 * (size_t)i;
-    // MDRect::IsInside (mdrect.h:35-38)
-    if (!(d->rs[0] <= x[0] && x[0] < d->re[0] && d->rs[1] <= x[1] && x[1] < d->re[1] && d->rs[2] <= x[2] &&
-          x[2] < d->re[2]))
-      continue;
-    hq.push_back(make_double4(x[0], x[1], x[2], 0.0));
-    hp.push_back(p ? make_double4(p[3 * (size_t)i], p[3 * (size_t)i + 1], p[3 * (size_t)i + 2], 0.0)
-                   : make_double4(0.0, 0.0, 0.0, 0.0));
-    hid.push_back(type ? type[i] : 0);
-  }
-  const int add = (int)hq.size();
-  if (add == 0) return MDGPU_OK;
-  CHK(ensure_owned(d, d->pn + add));
-  // ghosts of an earlier build are dropped (Variables::AddParticle sets total = owned)
-  HIPCHK(d, hipMemcpyAsync(d->pos + d->pn, hq.data(), add * sizeof(double4), hipMemcpyHostToDevice, d->stream));
-  HIPCHK(d, hipMemcpyAsync(d->mom + d->pn, hp.data(), add * sizeof(double4), hipMemcpyHostToDevice, d->stream));
-  HIPCHK(d, hipMemcpyAsync(d->id + d->pn, hid.data(), add * sizeof(int), hipMemcpyHostToDevice, d->stream));
-  HIPCHK(d, hipMemsetAsync(d->rep + d->pn, 0, add * sizeof(int), d->stream));
-  CHK(sync(d));
-  d->pn += add;
-  d->tn = d->pn;
-  d->ng = 0;
-  d->ghosts_ready = false;
-  CHK(upload_replicas(d));
-  d->vmax_valid = false;
-  // indices of the old list are stale: the next step rebuilds
-  d->initialized = false;
-  return MDGPU_OK;
-}
-
-int mdgpu_particle_number(const mdgpu_domain *d, int *pn, int *tn) {
-  if (!d) return MDGPU_ERR_ARGUMENT;
-  if (pn) *pn = d->pn;
-  if (tn) *tn = d->tn;
-  return MDGPU_OK;
-}
-
 // The owned particles' x, y, z (of q or p) between the device's 32-byte
 // entries and a caller's array of 3 doubles per particle: packed or unpacked
 // on the device in `xfer`, so that one copy moves exactly the caller's bytes
@@ -3228,6 +3180,66 @@ int copy_in3(mdgpu_domain *d, const double *src, int n, double4 *dst) {
   CHK(ensure_xfer(d, 3 * (size_t)n));
   HIPCHK(d, hipMemcpyAsync(d->xfer, src, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, d->stream));
   hipLaunchKernelGGL(k_unpack3, dim3(nblk(n)), dim3(kBlock), 0, d->stream, d->xfer, n, dst);
+  return MDGPU_OK;
+}
+
+int mdgpu_add_particles(mdgpu_domain *d, int n, const double *q, const double *p, const int *type) {
+  if (!d || n < 0 || (n > 0 && !q)) return MDGPU_ERR_ARGUMENT;
+  if (d->nrep > 1) {
+    d->err = "an ensemble's particles are set when it is created";
+    return MDGPU_ERR_ARGUMENT;
+  }
+  invalidate(d);  // the next fused step recomputes its first half drift
+  // MDRect::IsInside (mdrect.h:35-38)
+  auto inside = [&](const double *x) {
+    return (d->rs[0] <= x[0]) & (x[0] < d->re[0]) & (d->rs[1] <= x[1]) & (x[1] < d->re[1]) & (d->rs[2] <= x[2]) &
+           (x[2] < d->re[2]);
+  };
+  int add = 0;
+  for (int i = 0; i < n; i++) add += inside(q + 3 * (size_t)i);
+  if (add == 0) return MDGPU_OK;
+  // the caller's arrays as they are when every particle is inside, else those
+  // that are (a domain: all of them; a unit: its own)
+  std::vector<double> hq, hp;
+  std::vector<int> hid;
+  if (add < n) {
+    hq.reserve(3 * (size_t)add);
+    for (int i = 0; i < n; i++) {
+      const size_t o = 3 * (size_t)i;
+      if (!inside(q + o)) continue;
+      hq.insert(hq.end(), q + o, q + o + 3);
+      if (p) hp.insert(hp.end(), p + o, p + o + 3);
+      if (type) hid.push_back(type[i]);
+    }
+    q = hq.data();
+    if (p) p = hp.data();
+    if (type) type = hid.data();
+  }
+  CHK(ensure_owned(d, d->pn + add));
+  // ghosts of an earlier build are dropped (Variables::AddParticle sets total = owned)
+  CHK(copy_in3(d, q, add, d->pos + d->pn));
+  if (p) CHK(copy_in3(d, p, add, d->mom + d->pn));
+  else HIPCHK(d, hipMemsetAsync(d->mom + d->pn, 0, add * sizeof(double4), d->stream));
+  if (type) HIPCHK(d, hipMemcpyAsync(d->id + d->pn, type, add * sizeof(int), hipMemcpyHostToDevice, d->stream));
+  else HIPCHK(d, hipMemsetAsync(d->id + d->pn, 0, add * sizeof(int), d->stream));
+  HIPCHK(d, hipMemsetAsync(d->rep + d->pn, 0, add * sizeof(int), d->stream));
+  CHK(check_launch(d, "copy from host"));
+  CHK(sync(d));
+  d->pn += add;
+  d->tn = d->pn;
+  d->ng = 0;
+  d->ghosts_ready = false;
+  CHK(upload_replicas(d));
+  d->vmax_valid = false;
+  // indices of the old list are stale: the next step rebuilds
+  d->initialized = false;
+  return MDGPU_OK;
+}
+
+int mdgpu_particle_number(const mdgpu_domain *d, int *pn, int *tn) {
+  if (!d) return MDGPU_ERR_ARGUMENT;
+  if (pn) *pn = d->pn;
+  if (tn) *tn = d->tn;
   return MDGPU_OK;
 }
 
@@ -3682,16 +3694,10 @@ int mdgpu_compute_kick(mdgpu_domain *d, double *dp) {
   HIPCHK(d, hipMemcpyAsync(d->mom_alt, d->mom, n * sizeof(double4), hipMemcpyDeviceToDevice, d->stream));
   HIPCHK(d, hipMemsetAsync(d->mom, 0, n * sizeof(double4), d->stream));
   CHK(force_in_place(d));
-  std::vector<double4> hp(n);
-  HIPCHK(d, hipMemcpyAsync(hp.data(), d->mom, n * sizeof(double4), hipMemcpyDeviceToHost, d->stream));
+  CHK(copy_out3(d, d->mom, n, dp));
   HIPCHK(d, hipMemcpyAsync(d->mom, d->mom_alt, n * sizeof(double4), hipMemcpyDeviceToDevice, d->stream));
-  CHK(sync(d));
-  for (int i = 0; i < n; i++) {
-    dp[3 * (size_t)i] = hp[i].x;
-    dp[3 * (size_t)i + 1] = hp[i].y;
-    dp[3 * (size_t)i + 2] = hp[i].z;
-  }
-  return MDGPU_OK;
+  CHK(check_launch(d, "copy to host"));
+  return sync(d);
 }
 
 int mdgpu_enable_timing(mdgpu_domain *d, int on) {
