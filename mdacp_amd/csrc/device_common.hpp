@@ -159,6 +159,10 @@ struct RunRep {
   int lifetime;
   int measured;   // the step in progress (or the last one) takes displacements
   int ncand;      // candidates found (more than the room for them: not all kept)
+  // Nose-Hoover
+  double zeta;    // Variables::Zeta
+  double factor;  // the step's momentum factor, exp(-dt/2 zeta)
+  double T, aim;  // temperature after the last step, its target
 };
 
 // A candidate of the displacement test: its position at the construction (w:
@@ -170,6 +174,7 @@ struct RunCand {
 // Where a run's kick puts what a measured step takes (rr == nullptr: nothing).
 struct RunMeasure {
   RunRep *rr;
+  double *kpart;       // per brick: kinetic energy (Nose-Hoover; else nullptr)
   const double4 *old;  // positions at the construction, owned particles
   double *dpart;       // per brick: largest squared displacement
   RunCand *cand;       // cap per replica
@@ -194,6 +199,18 @@ __device__ __forceinline__ double3 image_of(double4 q, int code, const double *L
   const double dy = sy > 0 ? L[1] : (sy < 0 ? -L[1] : 0.0);
   const double dz = sz > 0 ? L[2] : (sz < 0 ? -L[2] : 0.0);
   return make_double3(q.x + dx, q.y + dy, q.z + dz);
+}
+
+// Sum over the workgroup in a fixed order, in thread 0.  Every thread calls it.
+__device__ __forceinline__ double block_sum_first(double v) {
+  __shared__ double ws[16];  // up to 1024 threads
+  v = wave_sum(v);
+  if ((threadIdx.x % kWave) == 0) ws[threadIdx.x / kWave] = v;
+  __syncthreads();
+  double t = 0.0;
+  if (threadIdx.x == 0)
+    for (int k = 0; k < (int)(blockDim.x / kWave); k++) t += ws[k];
+  return t;
 }
 
 // The face tests of the halo (strict, mdrect.cc:24-47) for a position of a

@@ -31,6 +31,8 @@ enum Epilogue {
   kKickOnly = 0,      // p += kick                       (CalculateForce)
   kKickDrift = 1,     // p += kick; q_out = q + p*dt2    (CalculateForce + UpdatePositionHalf)
   kKickLangevin = 2,  // p += kick; Langevin update      (CalculateLangevin)
+  kKickNoseHoover = 3,  // p = (p f + kick) f; q_out = q + p*dt2, f the step's factor
+                        // (HeatbathMomenta, CalculateForce, HeatbathMomenta, UpdatePositionHalf)
 };
 
 struct BrickList {
@@ -430,6 +432,24 @@ __device__ __forceinline__ RowExtra row_extra(int i, int epilogue, const int *__
   return x;
 }
 
+// The momentum after the kick a; Nose-Hoover: scaled by f before and after.
+__device__ __forceinline__ void kick_row(double4 &p, const double3 a, int epilogue, double f) {
+  if (epilogue == kKickNoseHoover) {
+    p.x = (p.x * f + a.x) * f;
+    p.y = (p.y * f + a.y) * f;
+    p.z = (p.z * f + a.z) * f;
+  } else {
+    p.x += a.x;
+    p.y += a.y;
+    p.z += a.z;
+  }
+}
+
+// The Nose-Hoover factor of replica r in this step of a run.
+__device__ __forceinline__ double step_factor(const StepClock &sc, int r, int epilogue) {
+  return epilogue == kKickNoseHoover ? sc.meas.rr[r].factor : 1.0;
+}
+
 __device__ __forceinline__ double finish_row(int i, double4 p, const double4 qi, double4 *__restrict__ mom,
                                              double4 *__restrict__ pos_out, int epilogue, double dt2,
                                              const LangevinConsts &lc, const RowExtra &x, const NextDrift &nd,
@@ -437,7 +457,7 @@ __device__ __forceinline__ double finish_row(int i, double4 p, const double4 qi,
   if (epilogue == kKickLangevin) langevin_update(p, lc, (uint32_t)x.id);
   mom[i] = p;
   double4 q = qi;
-  if (epilogue == kKickDrift) {
+  if (epilogue == kKickDrift || epilogue == kKickNoseHoover) {
     q.x += p.x * dt2;
     q.y += p.y * dt2;
     q.z += p.z * dt2;
@@ -485,7 +505,7 @@ __device__ __forceinline__ void measure_brick(int b, int r, int row0, int nrow, 
     const int i = row0 + v;
     const double4 o = M.old[i], qh = src[i];
     double4 q = qh;
-    if (epilogue == kKickDrift) {
+    if (epilogue != kKickLangevin) {
       const double4 p = mom[i];
       q.x += p.x * dt2;
       q.y += p.y * dt2;
@@ -507,6 +527,23 @@ __device__ __forceinline__ void measure_brick(int b, int r, int row0, int nrow, 
   block_max_to_partial(dm, M.dpart, b);
 }
 
+// The brick's kinetic energy after the kick (KineticEnergyObserver's terms,
+// observer.cc:5-15), its rows in a fixed order, for a Nose-Hoover step's
+// temperature.  A pass of its own: the slices go to whichever wavefront is
+// free, so a sum along them would depend on timing.  Every thread calls it.
+template <int T>
+__device__ __forceinline__ void kinetic_brick(int b, int row0, int nrow, const double4 *mom, double *kpart) {
+  if (kpart == nullptr) return;
+  __syncthreads();  // the brick's momenta are written
+  double ke = 0.0;
+  for (int v = threadIdx.x; v < nrow; v += T) {
+    const double4 p = mom[row0 + v];
+    ke += 0.5 * p.x * p.x + 0.5 * p.y * p.y + 0.5 * p.z * p.z;
+  }
+  ke = block_sum_first(ke);
+  if (threadIdx.x == 0) kpart[b] = ke;
+}
+
 // FP64 kick: one workgroup per brick, wavefronts over the brick's slices;
 // U groups of list indices in flight ahead of the group computed.
 // The FP64 kick of brick b by the calling workgroup (the body of
@@ -522,10 +559,14 @@ __device__ __forceinline__ void brick_kick_fp64(const int b, const double4 *__re
   constexpr int T = kWave * W;
   const Replica &Rp = bl.reps[bl.brep[b]];
   const LangevinConsts lc = langevin_consts(Rp, sc.dt, step_of(sc));
+  const double nhf = step_factor(sc, bl.brep[b], epilogue);
   const int nrow = bl.nrow[b], row0 = bl.row0[b], vs0 = bl.vslice0[b];
   if (nrow == 0) {  // a brick without rows: nothing to stage
     if (vpart) block_max_to_partial(0.0, vpart, b);
-    if (sc.meas.rr != nullptr && threadIdx.x == 0) sc.meas.dpart[b] = 0.0;
+    if (sc.meas.rr != nullptr && threadIdx.x == 0) {
+      sc.meas.dpart[b] = 0.0;
+      if (sc.meas.kpart != nullptr) sc.meas.kpart[b] = 0.0;
+    }
     return;
   }
   const long long g0 = bl.gbase[b];
@@ -552,14 +593,13 @@ __device__ __forceinline__ void brick_kick_fp64(const int b, const double4 *__re
     const double3 a = staged ? row_kick_fp64<true, U>(sg, lane, len, qi, lds64, G, fc)
                              : row_kick_fp64<false, U>(sg, lane, len, qi, lds64, G, fc);
     if (ok) {
-      p.x += a.x;
-      p.y += a.y;
-      p.z += a.z;
+      kick_row(p, a, epilogue, nhf);
       vmax = fmax(vmax, finish_row(i, p, qi, mom, pos_out, epilogue, fc.dt2, lc, x, nd, Rp));
     }
   }
   if (vpart) block_max_to_partial(vmax, vpart, b);
   measure_brick<T>(b, bl.brep[b], row0, nrow, src, mom, epilogue, fc.dt2, Rp, sc.meas);
+  kinetic_brick<T>(b, row0, nrow, mom, sc.meas.kpart);
 }
 
 // At most 128 registers with up to two groups ahead: four wavefronts per SIMD,
@@ -761,6 +801,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
       if (nrow > 0) {
         const Replica &Rp = bl.reps[bl.brep[b]];
         const LangevinConsts lc = langevin_consts(Rp, sc.dt, step_of(sc));
+  const double nhf = step_factor(sc, bl.brep[b], epilogue);
         const int row0 = bl.row0[b], vs0 = bl.vslice0[b];
         const long long g0 = bl.gbase[b];
         const int total = (int)(bl.gbase[b + 1] - g0);
@@ -781,9 +822,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
                                    : row_kick_fp64<false, U>(slice_groups(bl.nbr, bl.sbase[s]), lane, len, qi,
                                                              nullptr, Gb, fc);
           if (ok) {
-            p.x += a.x;
-            p.y += a.y;
-            p.z += a.z;
+            kick_row(p, a, epilogue, nhf);
             vmax = fmax(vmax, finish_row(i, p, qi, mom, pos_out, epilogue, fc.dt2, lc, x, nd, Rp));
           }
         }
@@ -803,6 +842,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
                                       bl.reps[bl.brep[b]], sc.meas);
       else if (threadIdx.x == 0)
         sc.meas.dpart[b] = 0.0;
+      kinetic_brick<kWave *(W + P)>(b, bl.row0[b], bl.nrow[b], mom, sc.meas.kpart);
     }
   }
 }
@@ -826,6 +866,7 @@ __global__ __launch_bounds__(kWave *W) void k_force_brick_mixed(
   const int b = blockIdx.x;
   const Replica &Rp = bl.reps[bl.brep[b]];
   const LangevinConsts lc = langevin_consts(Rp, sc.dt, step_of(sc));
+  const double nhf = step_factor(sc, bl.brep[b], epilogue);
   if (threadIdx.x < 64) {
     const int c = threadIdx.x;
     const int ox = (c & 3) - 1, oy = ((c >> 2) & 3) - 1, oz = ((c >> 4) & 3) - 1;
@@ -835,7 +876,10 @@ __global__ __launch_bounds__(kWave *W) void k_force_brick_mixed(
   const int nrow = bl.nrow[b], row0 = bl.row0[b], vs0 = bl.vslice0[b];
   if (nrow == 0) {  // a brick without rows: nothing to stage
     if (vpart) block_max_to_partial(0.0, vpart, b);
-    if (sc.meas.rr != nullptr && threadIdx.x == 0) sc.meas.dpart[b] = 0.0;
+    if (sc.meas.rr != nullptr && threadIdx.x == 0) {
+      sc.meas.dpart[b] = 0.0;
+      if (sc.meas.kpart != nullptr) sc.meas.kpart[b] = 0.0;
+    }
     return;
   }
   const long long g0 = bl.gbase[b];
@@ -882,14 +926,13 @@ __global__ __launch_bounds__(kWave *W) void k_force_brick_mixed(
       double4 p = mom[i];
       const double4 qi = pos[i];
       const RowExtra x = row_extra(i, epilogue, id, nd);
-      p.x += a.x;
-      p.y += a.y;
-      p.z += a.z;
+      kick_row(p, a, epilogue, nhf);
       vmax = fmax(vmax, finish_row(i, p, qi, mom, pos_out, epilogue, dt2, lc, x, nd, Rp));
     }
   }
   if (vpart) block_max_to_partial(vmax, vpart, b);
   measure_brick<T>(b, bl.brep[b], row0, nrow, pos, mom, epilogue, dt2, Rp, sc.meas);
+  kinetic_brick<T>(b, row0, nrow, mom, sc.meas.kpart);
 }
 
 // Mixed-precision kick in a brick-centred FP32 frame: the workgroup stages its
@@ -913,10 +956,14 @@ __device__ __forceinline__ void brick_kick_mixed_brick(const int b, const double
   constexpr int T = kWave * W;
   const Replica &Rp = bl.reps[bl.brep[b]];
   const LangevinConsts lc = langevin_consts(Rp, sc.dt, step_of(sc));
+  const double nhf = step_factor(sc, bl.brep[b], epilogue);
   const int nrow = bl.nrow[b], row0 = bl.row0[b], vs0 = bl.vslice0[b];
   if (nrow == 0) {  // a brick without rows: nothing to stage
     if (vpart) block_max_to_partial(0.0, vpart, b);
-    if (sc.meas.rr != nullptr && threadIdx.x == 0) sc.meas.dpart[b] = 0.0;
+    if (sc.meas.rr != nullptr && threadIdx.x == 0) {
+      sc.meas.dpart[b] = 0.0;
+      if (sc.meas.kpart != nullptr) sc.meas.kpart[b] = 0.0;
+    }
     return;
   }
   const BrickBox X = brick_box(b, Rp);
@@ -964,14 +1011,13 @@ __device__ __forceinline__ void brick_kick_mixed_brick(const int b, const double
       double4 p = mom[i];
       const double4 qi = src[i];
       const RowExtra x = row_extra(i, epilogue, id, nd);
-      p.x += a.x;
-      p.y += a.y;
-      p.z += a.z;
+      kick_row(p, a, epilogue, nhf);
       vmax = fmax(vmax, finish_row(i, p, qi, mom, pos_out, epilogue, dt2, lc, x, nd, Rp));
     }
   }
   if (vpart) block_max_to_partial(vmax, vpart, b);
   measure_brick<T>(b, bl.brep[b], row0, nrow, src, mom, epilogue, dt2, Rp, sc.meas);
+  kinetic_brick<T>(b, row0, nrow, mom, sc.meas.kpart);
 }
 
 template <int W, int U, int kSum>

@@ -166,6 +166,7 @@ struct mdgpu_domain {
   RunCand *run_cand = nullptr;                 // candidates of the runs' displacement tests
   int run_cap = 1;                             // ... kept per replica
   double *dpart = nullptr;                     // one maximum displacement per brick workgroup
+  double *kpart = nullptr;                     // one kinetic energy per brick workgroup (Nose-Hoover)
   bool run_halted = false;  // the last run stopped at a step that the host decides
   bool run_keep = false;    // what the last run's last step measured still holds
   int since_build = 0;      // run steps since the last construction
@@ -483,6 +484,7 @@ int set_geometry(mdgpu_domain *d) {
   CHK(dalloc(d, &d->nrange, d->nbrick));
   CHK(dalloc(d, &d->bpart, d->nbrick));
   CHK(dalloc(d, &d->dpart, d->nbrick));
+  CHK(dalloc(d, &d->kpart, d->nbrick));
   CHK(dalloc(d, &d->btotal, d->nbrick));
   CHK(dalloc(d, &d->gbase, d->nbrick + 1));
   CHK(dalloc(d, &d->tstart, (size_t)d->nbrick * kRangesPerCell * d->rmax));
@@ -1530,6 +1532,8 @@ RunRules run_rules(const mdgpu_domain *d) {
   U.SL2 = d->SL * d->SL;
   U.CL2 = d->CL2;
   U.check = d->disp_check;
+  U.bath = d->thermostat == MDGPU_NOSEHOOVER;
+  U.tau = d->tau;
   U.list_cap = d->check_list_length;
   U.cap = d->run_cap;
   U.single = d->nrep == 1;
@@ -1550,7 +1554,8 @@ int launch_force(mdgpu_domain *d, const double4 *src, const float4 *rel, double4
   const ForceConsts fc = fconsts(d);
   const ForceConstsF f32 = fconsts32(d);
   RunMeasure meas{};
-  if (gated) meas = RunMeasure{d->rr, d->pos_old, d->dpart, d->run_cand, d->run_cap, d->SL};
+  const bool bath = d->thermostat == MDGPU_NOSEHOOVER;
+  if (gated) meas = RunMeasure{d->rr, bath ? d->kpart : nullptr, d->pos_old, d->dpart, d->run_cand, d->run_cap, d->SL};
   const StepClock sc{d->dt, d->step, clock, gated ? d->gate : nullptr, meas};
   double *vb = want_vmax ? d->bpart : nullptr;
   const int ev0 = d->force_launches * 2;
@@ -1571,9 +1576,10 @@ int launch_force(mdgpu_domain *d, const double4 *src, const float4 *rel, double4
     // the next step's validity test from them
     const bool own = d->nrep > kTailReplicas;
     if (own)
-      hipLaunchKernelGGL(k_run_max, dim3(d->nrep), dim3(kBlock), 0, st, d->gate, d->bpart, d->dpart, d->reps, d->rr);
+      hipLaunchKernelGGL(k_run_max, dim3(d->nrep), dim3(kBlock), 0, st, d->gate, d->bpart, d->dpart,
+                         bath ? d->kpart : nullptr, d->reps, d->rr);
     hipLaunchKernelGGL(k_run_tail, dim3(1), dim3(kTailThreads), 0, st, d->gate, own ? nullptr : d->bpart, d->dpart,
-                       d->rr, d->nrep, run_rules(d), d->run_cand, d->reps, d->grng, d->ng, d->clock, d->h_gate,
+                       d->kpart, d->rr, d->nrep, run_rules(d), d->run_cand, d->reps, d->grng, d->ng, d->clock, d->h_gate,
                        d->h_rr);
   } else if (want_vmax) {
     hipLaunchKernelGGL(k_replica_max, dim3(d->nrep), dim3(kBlock), 0, st, d->bpart, d->reps, d->rep_v2, clock);
@@ -1723,6 +1729,9 @@ int final_positions(mdgpu_domain *d, const double4 *qh, const double4 *qh2 = nul
   return check_launch(d, "final positions");
 }
 
+// Whether the steps read the inner list (Nose-Hoover steps read the full one).
+bool inner_steps(const mdgpu_domain *d) { return d->prune_delta > 0.0 && d->thermostat != MDGPU_NOSEHOOVER; }
+
 // The fused step's launches.  gated: a step of a run, whose launches do nothing
 // once the run has halted, and which leaves the halo refresh out where the
 // kick takes the images from their owners (run_gated writes the ghosts once
@@ -1741,14 +1750,16 @@ int enqueue_fused(mdgpu_domain *d, unsigned long long *clock, bool prune = false
   }
   CHK(check_launch(d, "refresh"));
   if (prune) CHK(launch_prune(d));
-  const int epi = d->thermostat == MDGPU_LANGEVIN ? kKickLangevin : kKickDrift;
+  const int epi = d->thermostat == MDGPU_LANGEVIN     ? kKickLangevin
+                  : d->thermostat == MDGPU_NOSEHOOVER ? kKickNoseHoover
+                                                      : kKickDrift;
   const NextDrift nd{d->pos_next, mixed ? d->rel_next : nullptr, d->cell, d->org};
   // a run's steps leave the final owned positions out (run_gated writes them
   // after the run); a timed step does too and writes them after its timed kick,
   // so that the events time the kernel the runs launch
   const bool timed = d->timing && clock == nullptr && !gated;
   CHK(launch_force(d, d->pos_tmp, d->rel_tmp, gated || timed ? nullptr : d->pos, epi, true, nd, clock,
-                   d->prune_delta > 0.0, gated));
+                   inner_steps(d), gated));
   if (timed && d->pn > 0) CHK(final_positions(d, d->pos_tmp));
   return MDGPU_OK;
 }
@@ -1911,11 +1922,11 @@ int calculate_step(mdgpu_domain *d) {
   return MDGPU_OK;
 }
 
-// Whether steps may be queued without waiting for the host: fused NVE or
-// Langevin steps (replayed from graphs or launched), no inner list.
-bool can_run(const mdgpu_domain *d) {
-  return d->run_ahead > 0 && !d->timing && d->thermostat != MDGPU_NOSEHOOVER && !(d->prune_delta > 0.0) && d->pn > 0;
-}
+// Whether steps may be queued without waiting for the host: fused steps
+// (replayed from graphs or launched) on the full list.
+bool can_run(const mdgpu_domain *d) { return d->run_ahead > 0 && !d->timing && !inner_steps(d) && d->pn > 0; }
+
+double &zeta_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->zeta : d->rst[r].zeta; }
 
 double &budget_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->buffer_length : d->rst[r].buffer_length; }
 int &lifetime_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->lifetime : d->rst[r].lifetime; }
@@ -1975,11 +1986,27 @@ int run_steps(mdgpu_domain *d, int limit, int *done) {
     S.budget = budget_of(d, r);
     S.lifetime = lifetime_of(d, r);
     S.v2 = d->vmax_valid ? d->h_rep_v2[r] : 0.0;
+    S.zeta = zeta_of(d, r);
+    S.aim = R == 1 ? d->T_aim : d->rst[r].T;
     if (!approved) S.measured = 0;
+  }
+  // a Nose-Hoover step starts from the temperature the last one ended with:
+  // the last run's, or summed here
+  double *ke = nullptr;
+  if (d->thermostat == MDGPU_NOSEHOOVER && !keep) {
+    if (R == 1) {
+      const unsigned nb = nblk(d->pn);
+      CHK(ensure_partial(d, (int)nb));
+      hipLaunchKernelGGL(k_kinetic, dim3(nb), dim3(kBlock), 0, st, d->mom, d->pn, d->partial);
+      hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kBlock), 0, st, d->partial, (int)nb, 1, d->rep_out);
+    } else {
+      hipLaunchKernelGGL(k_replica_kinetic, dim3(R), dim3(kBlock), 0, st, d->mom, d->reps, d->rep_out);
+    }
+    ke = d->rep_out;
   }
   d->h_gate->done = -1;
   hipLaunchKernelGGL(k_run_begin, dim3(1), dim3(kTailThreads), 0, st, d->gate, k, d->rr, d->h_rr, R, run_rules(d),
-                     d->run_cand, d->reps, d->grng, d->ng, approved ? 1 : 0, keep ? 1 : 0, d->clock,
+                     d->run_cand, d->reps, d->grng, d->ng, approved ? 1 : 0, keep ? 1 : 0, ke, d->clock,
                      (unsigned long long)d->step, d->h_gate);
   const double4 *qh = d->pos_tmp, *qh2 = d->pos_next;
   for (int j = 0; j < k; j++) {
@@ -2004,6 +2031,7 @@ int run_steps(mdgpu_domain *d, int limit, int *done) {
       budget_of(d, r) = d->h_rr[r].budget;
       lifetime_of(d, r) = d->h_rr[r].lifetime;
       d->h_rep_v2[r] = d->h_rr[r].v2;
+      if (d->thermostat == MDGPU_NOSEHOOVER) zeta_of(d, r) = d->h_rr[r].zeta;
     }
   d->run_halted = d->h_gate->halted != 0;
   d->run_keep = !d->run_halted;
@@ -3107,7 +3135,7 @@ int mdgpu_destroy(mdgpu_domain *d) {
                   d->i32,     d->d3,          d->reps,        d->brep,      d->rep,      d->rep_alt,
                   d->grng,    d->rep_v2,      d->rep_out,     d->which,     d->rep_exp,  d->clock,
                   d->nbr_in,      d->ncode_in,    d->slen_in,   d->chk_dmax, d->chk_cnt,
-                  d->chk_cand, d->gate,       d->gimg,       d->rr,          d->run_cand,  d->dpart,     d->xfer,     d->gunit,
+                  d->chk_cand, d->gate,       d->gimg,       d->rr,          d->run_cand,  d->dpart,     d->kpart,     d->xfer,     d->gunit,
                   d->st_pos,  d->st_mom,      d->st_id,       d->src_tab,   d->ucnt,     d->uoff,
                   d->rep_factor};
   for (StepGraph &g : d->graphs) drop_graph(g);

@@ -430,6 +430,17 @@ __device__ __forceinline__ double replica_part_max(const double *__restrict__ pa
   return fmax(fmax(m0, m1), fmax(m2, m3));
 }
 
+// Sum of a replica's per-brick values by the T lanes `t`: each lane's in a
+// fixed order.
+__device__ __forceinline__ double replica_part_sum(const double *__restrict__ part, int b0, int nb, int t, int T) {
+  double s = 0.0;
+  for (int k = t; k < nb; k += T) s += part[b0 + k];
+  return s;
+}
+
+// MDManager::Temperature (mdmanager.cc:390-397) from the kinetic energy.
+__device__ __forceinline__ double run_temperature(double ke, const Replica &R) { return (ke / (double)R.pn) / 1.5; }
+
 // out[r] = max of part over each replica's bricks, one workgroup per replica.
 // clock (optional) is the step counter of the fused step; it advances by one
 // here.
@@ -448,12 +459,18 @@ __global__ __launch_bounds__(kBlock) void k_replica_max(const double *__restrict
 // replica (k_run_tail's first part, for kTailReplicas replicas and more).
 __global__ __launch_bounds__(kBlock) void k_run_max(const RunGate *__restrict__ gate, const double *__restrict__ part,
                                                     const double *__restrict__ dpart,
+                                                    const double *__restrict__ kpart,
                                                     const Replica *__restrict__ reps, RunRep *__restrict__ rr) {
   if (run_halted(gate)) return;
   const int r = blockIdx.x;
   const Replica &R = reps[r];
   const double m = block_max_all(replica_part_max(part, R.brick0, replica_bricks(R), threadIdx.x, kBlock));
   if (threadIdx.x == 0) rr[r].v2 = m;
+  if (kpart != nullptr) {
+    const double ke = block_sum_first(replica_part_sum(kpart, R.brick0, replica_bricks(R), threadIdx.x, kBlock));
+    if (threadIdx.x == 0) rr[r].T = run_temperature(ke, R);
+    __syncthreads();
+  }
   if (!rr[r].measured) return;
   __syncthreads();
   const double dm = block_max_all(replica_part_max(dpart, R.brick0, replica_bricks(R), threadIdx.x, kBlock));
@@ -464,6 +481,8 @@ __global__ __launch_bounds__(kBlock) void k_run_max(const RunGate *__restrict__ 
 struct RunRules {
   double dt, margin, SL2, CL2;
   int check;       // the displacement check (MDGPU_OPT_DISPLACEMENT_CHECK)
+  int bath;        // Nose-Hoover
+  double tau;      // ... its time constant
   int list_cap;    // CheckListLength
   int cap;         // room for candidates per replica
   int single;      // one replica
@@ -533,6 +552,13 @@ __device__ __forceinline__ void run_put_cand(RunShared &sh, int at, const RunCan
   sh.c[3][at] = C.now.x;
   sh.c[4][at] = C.now.y;
   sh.c[5][at] = C.now.z;
+}
+
+// ForceCalculator::HeatbathZeta (fcalculator.cc:744-749) with the temperature
+// after the last step.
+__device__ __forceinline__ double run_heatbath(const RunRep &S, const RunRules &U) {
+  const double t1 = (S.T - S.aim) / (U.tau * U.tau);
+  return S.zeta + t1 * (U.dt * 0.5);
 }
 
 // PairList::IsPairListExpired (pairlist.cc:26-45) for the next step of a run,
@@ -634,6 +660,13 @@ __device__ __forceinline__ bool run_gate(RunRep *rr, int nrep, const RunRules &U
     S.cthr = bound ? U.margin - reach : 1.0e200;
     S.measured = !(S.budget > 4.5 * v * U.dt);
     S.ncand = 0;
+    // Nose-Hoover: the step starts with a HeatbathZeta at the temperature the
+    // last one ended with, and scales the momenta by this factor (HeatbathMomenta,
+    // fcalculator.cc:752-762)
+    if (U.bath) {
+      S.zeta = run_heatbath(S, U);
+      S.factor = exp(-(U.dt * 0.5) * S.zeta);
+    }
     rr[r] = S;
   }
   return true;
@@ -643,18 +676,24 @@ __device__ __forceinline__ bool run_gate(RunRep *rr, int nrep, const RunRules &U
 // from the host's copies (pinned memory, read here), the step counter, and the
 // first step's validity test (run_gate), unless the host has decided that step
 // (`approved`).  keep: the displacements that the last run's last step
-// measured still hold.  host: where the outcome goes when the run ends here.
+// measured still hold.  ke (Nose-Hoover, when the last run's temperature does
+// not hold): each replica's kinetic energy.  host: where the outcome goes when
+// the run ends here.
 __global__ __launch_bounds__(kTailThreads) void k_run_begin(RunGate *gate, int left, RunRep *rr,
                                                             const RunRep *__restrict__ from, int nrep, RunRules U,
                                                             const RunCand *cand, const Replica *__restrict__ reps,
                                                             const int2 *__restrict__ grng, int ng, int approved,
-                                                            int keep, unsigned long long *clock,
-                                                            unsigned long long step, RunGate *host) {
+                                                            int keep, const double *__restrict__ ke,
+                                                            unsigned long long *clock, unsigned long long step,
+                                                            RunGate *host) {
   __shared__ RunShared sh;
   for (int r = threadIdx.x; r < nrep; r += kTailThreads) {
     rr[r].budget = from[r].budget;
     rr[r].v2 = from[r].v2;
     rr[r].lifetime = from[r].lifetime;
+    rr[r].zeta = from[r].zeta;
+    rr[r].aim = from[r].aim;
+    if (ke != nullptr) rr[r].T = run_temperature(ke[r], reps[r]);
     if (!keep) {  // the displacements the host has checked, if it has
       rr[r].measured = from[r].measured;
       rr[r].dmax2 = from[r].dmax2;
@@ -684,7 +723,8 @@ __global__ __launch_bounds__(kTailThreads) void k_run_begin(RunGate *gate, int l
 constexpr int kTailReplicas = 128;
 
 __global__ __launch_bounds__(kTailThreads) void k_run_tail(RunGate *gate, const double *__restrict__ part,
-                                                           const double *__restrict__ dpart, RunRep *rr, int nrep,
+                                                           const double *__restrict__ dpart,
+                                                           const double *__restrict__ kpart, RunRep *rr, int nrep,
                                                            RunRules U, const RunCand *cand,
                                                            const Replica *__restrict__ reps,
                                                            const int2 *__restrict__ grng, int ng,
@@ -703,19 +743,29 @@ __global__ __launch_bounds__(kTailThreads) void k_run_tail(RunGate *gate, const 
       const double dm = block_max_all<kTailThreads>(replica_part_max(dpart, b0, nb, threadIdx.x, kTailThreads));
       if (threadIdx.x == 0) rr[0].dmax2 = dm;
     }
+    if (U.bath) {
+      const double ke = block_sum_first(replica_part_sum(kpart, b0, nb, threadIdx.x, kTailThreads));
+      if (threadIdx.x == 0) rr[0].T = run_temperature(ke, reps[0]);
+    }
   } else {
     for (int r = threadIdx.x / kWave; r < nrep; r += kTailThreads / kWave) {
       const int b0 = reps[r].brick0, nb = replica_bricks(reps[r]);
       const double m = wave_max(replica_part_max(part, b0, nb, threadIdx.x % kWave, kWave));
       const double dm =
           rr[r].measured ? wave_max(replica_part_max(dpart, b0, nb, threadIdx.x % kWave, kWave)) : 0.0;
+      const double ke = U.bath ? wave_sum(replica_part_sum(kpart, b0, nb, threadIdx.x % kWave, kWave)) : 0.0;
       if (threadIdx.x % kWave == 0) {
         rr[r].v2 = m;
         if (rr[r].measured) rr[r].dmax2 = dm;
+        if (U.bath) rr[r].T = run_temperature(ke, reps[r]);
       }
     }
   }
   __syncthreads();
+  if (U.bath) {  // the HeatbathZeta that ends a Nose-Hoover step
+    for (int r = threadIdx.x; r < nrep; r += kTailThreads) rr[r].zeta = run_heatbath(rr[r], U);
+    __syncthreads();
+  }
   const bool go = left == 0 || run_gate(rr, nrep, U, cand, reps, grng, ng, false, sh);
   if (threadIdx.x == 0) {
     const RunGate G{go ? 0 : 1, done, left};

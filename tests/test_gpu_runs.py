@@ -87,3 +87,33 @@ def test_runs_of_a_domain_match_single_steps(cap):
     assert a.time() == b.time()
     for d in ds:
         d.close()
+
+
+@pytest.mark.parametrize("name", ["six", "one", "many"])
+def test_nose_hoover_runs_follow_single_steps(name):
+    """Nose-Hoover in runs: the temperatures and zetas stay on the device, summed brick by brick
+    instead of in index order, so the two agree to rounding, which 60 steps amplify (1e-10)."""
+    c = CASES[name]
+    print("case: Nose-Hoover", name, flush=True)
+    (boxes, counts, q, p, ids), T = replicas(c["n"], c["k_of"], c["rho_of"])
+    es = []
+    for ahead in (64, 0):
+        e = mdgpu.Ensemble(boxes, counts, q, p, ids, T=T, thermostat=mdgpu.NOSEHOOVER, dt=0.005)
+        e.set_option(mdgpu.OPT_RUN_AHEAD, ahead)
+        if c["n"] == 1:
+            e.set_thermostat(mdgpu.NOSEHOOVER, T=1.3, tau=0.2)
+        es.append(e)
+    a, b = es
+    ra = rb = 0
+    for chunk in (1, 40, 2, 17):
+        ra += a.calculate(chunk)
+        rb += b.calculate(chunk)
+        assert ra == rb, (chunk, ra, rb)
+    assert ra >= 1, ra
+    za, zb = a.replica_zetas(), b.replica_zetas()
+    assert np.abs(za - zb).max() < 1e-10 and np.abs(zb).max() > 1e-3
+    (qa, pa, ta), (qb, pb, tb) = a.particles(), b.particles()
+    assert np.array_equal(ta, tb)
+    assert np.abs(qa - qb).max() < 1e-10 and np.abs(pa - pb).max() < 1e-10
+    for e in es:
+        e.close()
