@@ -13,6 +13,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "mdgpu.h"
@@ -243,6 +244,7 @@ struct mdgpu_domain {
   unsigned long long *scan_status = nullptr;
   unsigned *scan_ticket = nullptr, scan_base = 0, scan_epoch = 0;
   long long scan_cap = 0;  // workgroups
+  char *pinned = nullptr;  // the allocation that holds all pinned mirrors (h_...)
   BuildState *bs = nullptr, *h_bs = nullptr;  // a construction's counts, and their pinned copy
   int staged_guess = 0;    // largest neighbourhood of the last construction with these bricks (0: none)
   bool rows_swapped = false;  // the construction in flight has swapped the owned arrays for the row order
@@ -578,6 +580,32 @@ int ensure_ghosts(mdgpu_domain *d, int need) {
   d->gcap = ngc;
   invalidate(d);
   return MDGPU_OK;
+}
+
+// Ghost images of n particles (an ensemble: its replicas') at uniform density,
+// and a tenth more.
+double expected_images(const mdgpu_domain *d, int n) {
+  double g = 0.0;
+  for (int r = 0; r < d->nrep; r++) {
+    const Replica &R = d->rh[r];
+    const double pn = d->nrep == 1 ? n : R.pn;
+    g += pn * ((1.0 + 2.0 * d->SL / R.L[0]) * (1.0 + 2.0 * d->SL / R.L[1]) * (1.0 + 2.0 * d->SL / R.L[2]) - 1.0);
+  }
+  return std::min(1.1 * g, (double)(kMaxParticles - 2 - std::max(n, d->cap)));
+}
+
+// A new domain's first arrays: the ghosts' before the owned ones', so that the
+// arrays of both are made once.
+int reserve(mdgpu_domain *d, int owned, int ghosts) {
+  const int ngc = std::max(1024, std::min(ghosts, kMaxParticles - 1 - owned));
+  CHK(dalloc(d, &d->gsrc, ngc));
+  CHK(dalloc(d, &d->gcode, ngc));
+  CHK(dalloc(d, &d->gunit, ngc));
+  CHK(dalloc(d, &d->t_gsrc, ngc));
+  CHK(dalloc(d, &d->t_gcode, ngc));
+  CHK(dalloc(d, &d->t_gcell, ngc));
+  d->gcap = ngc;
+  return ensure_owned(d, owned);
 }
 
 // An exclusive scan of n items by functor f (scan.hpp), nothing when *skip is set.
@@ -1159,17 +1187,7 @@ int make_pair_list(mdgpu_domain *d) {
     return finish_build(d, kStageBricks);
   }
   CHK(auto_bricks(d));
-  if (d->ng_last == 0 && d->pn > 0) {
-    // the first construction: room for the images of a uniform density
-    double g = 0.0;
-    for (int r = 0; r < d->nrep; r++) {
-      const Replica &R = d->rh[r];
-      const double pn = d->nrep == 1 ? d->pn : R.pn;
-      g += pn * ((1.0 + 2.0 * d->SL / R.L[0]) * (1.0 + 2.0 * d->SL / R.L[1]) * (1.0 + 2.0 * d->SL / R.L[2]) - 1.0);
-    }
-    const double most = (double)(kMaxParticles - 1 - d->cap);
-    CHK(ensure_ghosts(d, (int)std::min(1.1 * g, most)));
-  }
+  if (d->ng_last == 0 && d->pn > 0) CHK(ensure_ghosts(d, (int)expected_images(d, d->pn)));  // the first construction
   CHK(begin_build(d));
   CHK(queue_bin(d, 1, true));
   return finish_build(d, kStageImages);
@@ -2201,42 +2219,55 @@ int create_domain(const mdgpu_params *prm, int nrep, const mdgpu_replica *rl, co
     mdgpu_destroy(d);
     return r;
   }
-  if (hipHostMalloc((void **)&d->h_rep_v2, nrep * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_rep_out, 3 * nrep * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_which, nrep * sizeof(int)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_rep_exp, nrep * sizeof(int)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_gate, sizeof(RunGate)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_rr, nrep * sizeof(RunRep)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_rep_factor, nrep * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_chk_dmax, nrep * sizeof(unsigned long long)) != hipSuccess) {
+  // the pinned mirrors, in one allocation
+  size_t pinned = 0;
+  auto place = [&](auto *&p, size_t n, char *base) {
+    if (base) p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + pinned);
+    pinned += (n * sizeof(*p) + 63) / 64 * 64;
+  };
+  auto place_all = [&](char *base) {
+    pinned = 0;
+    place(d->h_rep_v2, nrep, base);
+    place(d->h_rep_out, 3 * (size_t)nrep, base);
+    place(d->h_which, nrep, base);
+    place(d->h_rep_exp, nrep, base);
+    place(d->h_gate, 1, base);
+    place(d->h_rr, nrep, base);
+    place(d->h_rep_factor, nrep, base);
+    place(d->h_chk_dmax, nrep, base);
+    place(d->h_bs, 1, base);
+    place(d->h_u64, 4, base);
+    place(d->h_i64, 4, base);
+    place(d->h_i32, 4, base);
+    place(d->h_d3, 4, base);
+    if (unit) place(d->h_src_tab, kMaxUnits, base);
+  };
+  place_all(nullptr);
+  if (hipHostMalloc((void **)&d->pinned, pinned) != hipSuccess) {
     mdgpu_destroy(d);
     return MDGPU_ERR_HIP;
   }
+  place_all(d->pinned);
+  std::memset(d->pinned, 0, pinned);
   const int cap0 = rl ? (int)std::min<long long>(p0, kMaxParticles) : prm->capacity;
-  if ((r = set_geometry(d)) != MDGPU_OK || (r = ensure_owned(d, std::max(cap0, 1024))) != MDGPU_OK ||
-      (r = ensure_ghosts(d, std::max(1024, cap0 / 4))) != MDGPU_OK) {
+  if (!rl && !unit && cap0 > 0) {
+    // a domain told how many particles to expect takes its bricks for them
+    // now; its first construction takes them for those it then has
+    auto_brick(d, cap0 / (d->L[0] * d->L[1] * d->L[2]), d->L, brick_budget(d), d->bd, kDomainFill);
+    for (int k = 0; k < 3; k++) d->rh[0].bd[k] = d->bd[k];
+  }
+  if ((r = set_geometry(d)) != MDGPU_OK ||
+      (r = reserve(d, std::max(cap0, 1024), unit ? cap0 / 4 : (int)expected_images(d, cap0))) != MDGPU_OK) {
     mdgpu_destroy(d);
     return r;
   }
-  if ((r = dalloc(d, &d->bs, 1)) || (r = dalloc(d, &d->scan_ticket, 1)) || (r = dalloc(d, &d->u64, 4)) || (r = dalloc(d, &d->i64, 4)) || (r = dalloc(d, &d->i32, 4)) ||
-      (r = dalloc(d, &d->d3, 4)) || (r = dalloc(d, &d->cand, (size_t)d->check_list_length + 1))) {
+  if ((r = dalloc(d, &d->bs, 1)) || (r = dalloc(d, &d->scan_ticket, 1)) || (r = dalloc(d, &d->u64, 4)) ||
+      (r = dalloc(d, &d->i64, 4)) || (r = dalloc(d, &d->i32, 4)) || (r = dalloc(d, &d->d3, 4)) ||
+      (r = dalloc(d, &d->cand, (size_t)d->check_list_length + 1)) ||
+      (unit && (r = dalloc(d, &d->src_tab, kMaxUnits)) != MDGPU_OK)) {
     mdgpu_destroy(d);
     return r;
   }
-  if (unit && ((r = dalloc(d, &d->src_tab, kMaxUnits)) != MDGPU_OK ||
-               hipHostMalloc((void **)&d->h_src_tab, kMaxUnits * sizeof(SrcUnit)) != hipSuccess)) {
-    mdgpu_destroy(d);
-    return r ? r : MDGPU_ERR_HIP;
-  }
-  if (hipHostMalloc((void **)&d->h_bs, sizeof(BuildState)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_u64, 4 * sizeof(unsigned long long)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_i64, 4 * sizeof(long long)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_i32, 4 * sizeof(int)) != hipSuccess ||
-      hipHostMalloc((void **)&d->h_d3, 4 * sizeof(double)) != hipSuccess) {
-    mdgpu_destroy(d);
-    return MDGPU_ERR_HIP;
-  }
-  std::memset(d->h_rr, 0, nrep * sizeof(RunRep));
   (void)hipMemset(d->rr, 0, nrep * sizeof(RunRep));
   (void)hipMemset(d->bs, 0, sizeof(BuildState));
   (void)hipMemset(d->scan_ticket, 0, sizeof(unsigned));
@@ -3142,16 +3173,7 @@ int mdgpu_destroy(mdgpu_domain *d) {
   for (StepGraph &g : d->gated) drop_graph(g);
   for (void *b : bufs)
     if (b) (void)hipFree(b);
-  for (void *h : {(void *)d->h_rep_v2, (void *)d->h_rep_out, (void *)d->h_which, (void *)d->h_rep_exp,
-                  (void *)d->h_gate, (void *)d->h_rr, (void *)d->h_rep_factor,
-                  (void *)d->h_chk_dmax})
-    if (h) (void)hipHostFree(h);
-  if (d->h_bs) (void)hipHostFree(d->h_bs);
-  if (d->h_u64) (void)hipHostFree(d->h_u64);
-  if (d->h_i64) (void)hipHostFree(d->h_i64);
-  if (d->h_i32) (void)hipHostFree(d->h_i32);
-  if (d->h_d3) (void)hipHostFree(d->h_d3);
-  if (d->h_src_tab) (void)hipHostFree(d->h_src_tab);
+  if (d->pinned) (void)hipHostFree(d->pinned);
   for (hipEvent_t e : d->ev) (void)hipEventDestroy(e);
   if (d->stream && d->own_stream) (void)hipStreamDestroy(d->stream);
   if (d->group) {
