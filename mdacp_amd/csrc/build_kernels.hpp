@@ -491,10 +491,35 @@ __global__ void k_group_drift(GroupDrift G, double dt2) {
   G.pos[u][i] = q;
 }
 
+// The first half drift of the units' owned particles into tmp, the start of a
+// run of fused steps.
+struct GroupStart {
+  const double4 *pos[kMaxUnits];
+  const double4 *mom[kMaxUnits];
+  double4 *tmp[kMaxUnits];
+  int base[kMaxUnits + 1];
+  int n;
+};
+
+__global__ void k_group_start(GroupStart G, double dt2, RunGate *__restrict__ gate) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t == 0) *gate = RunGate{0, 0, 0};
+  if (t >= G.base[G.n]) return;
+  const int u = group_unit_of(G.base, G.n, t);
+  const int i = t - G.base[u];
+  double4 q = G.pos[u][i];
+  const double4 p = G.mom[u][i];
+  q.x += p.x * dt2;
+  q.y += p.y * dt2;
+  q.z += p.z * dt2;
+  G.tmp[u][i] = q;
+}
+
 // The ghosts of every unit from their sources' current positions (k_unit_refresh
-// for the whole group).
+// for the whole group); in a run (gate), from the half-drifted ones in src.
 struct GroupHalo {
   double4 *pos[kMaxUnits];
+  const double4 *src[kMaxUnits];
   const int *gsrc[kMaxUnits];
   const int *gcode[kMaxUnits];
   const int *gunit[kMaxUnits];
@@ -503,13 +528,14 @@ struct GroupHalo {
   int n;
 };
 
-__global__ void k_group_refresh(GroupHalo G, double Lx, double Ly, double Lz) {
+__global__ void k_group_refresh(GroupHalo G, double Lx, double Ly, double Lz, const RunGate *__restrict__ gate) {
+  if (run_halted(gate)) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= G.base[G.n]) return;
   const int u = group_unit_of(G.base, G.n, t);
   const int k = t - G.base[u];
   const double L[3] = {Lx, Ly, Lz};
-  const double3 y = image_of(G.pos[G.gunit[u][k]][G.gsrc[u][k]], G.gcode[u][k], L);
+  const double3 y = image_of(G.src[G.gunit[u][k]][G.gsrc[u][k]], G.gcode[u][k], L);
   G.pos[u][G.pn[u] + k] = make_double4(y.x, y.y, y.z, 0.0);
 }
 

@@ -617,13 +617,15 @@ __global__ __launch_bounds__(kWave *W, U <= 2 ? 4 : 1) void k_force_brick_fp64(c
 
 // The units of a process grid, kicked in one launch: unit u's bricks are the
 // launch's workgroups [brick0 of u, brick0 of u + 1), each doing what the
-// unit's own kick does (CalculateForce in place, no epilogue), on the unit's
-// own arrays.  One launch of all the units' bricks fills the CUs where one
+// unit's own kick does (CalculateForce in place, or the kick of a fused step),
+// on the unit's own arrays.  One launch of all the units' bricks fills the CUs where one
 // launch per unit ends each unit with a partial round of workgroups.  The
 // table travels in the kernel arguments (1 KB for kMaxKickUnits units).
 struct UnitKick {
-  const double4 *src;  // positions, owned then ghosts (kicked in place: no position output)
+  const double4 *src;  // owned positions (the ghosts': bl.ghost)
   double4 *mom;
+  double4 *pos_out;    // a step of a run: the positions at its end (else nullptr: kicked in place)
+  double4 *next;       //                  the next step's first half drift
   BrickList bl;
   int brick0;          // the unit's first workgroup in the launch
 };
@@ -640,12 +642,16 @@ __device__ __forceinline__ int group_kick_unit(const UnitKicks &uk, int b) {
   return u;
 }
 
+// Registers as in k_force_brick_fp64.
 template <int W, int U>
-__global__ __launch_bounds__(kWave *W) void k_force_group_fp64(UnitKicks uk, ForceConsts fc, StepClock sc) {
+__global__ __launch_bounds__(kWave *W, U <= 2 ? 4 : 1) void k_force_group_fp64(UnitKicks uk, ForceConsts fc,
+                                                                              int epilogue, StepClock sc,
+                                                                              double *__restrict__ vpart) {
+  if (run_halted(sc.gate)) return;
   const int b = blockIdx.x;
   const UnitKick &k = uk.u[group_kick_unit(uk, b)];
-  brick_kick_fp64<W, U>(b - k.brick0, k.src, k.mom, nullptr, k.bl, fc, kKickOnly, sc, nullptr, nullptr,
-                        NextDrift{nullptr, nullptr, nullptr, nullptr});
+  brick_kick_fp64<W, U>(b - k.brick0, k.src, k.mom, k.pos_out, k.bl, fc, epilogue, sc, nullptr,
+                        vpart ? vpart + k.brick0 : nullptr, NextDrift{k.next, nullptr, nullptr, nullptr});
 }
 
 // ---------------------------------------------------------------------------
@@ -1033,11 +1039,14 @@ __global__ __launch_bounds__(kWave *W) void k_force_brick_mixed_brick(
 // precision in the brick-centred frame.
 template <int W, int U, int kSum>
 __global__ __launch_bounds__(kWave *W) void k_force_group_mixed_brick(UnitKicks uk, ForceConstsF fc, double dt2,
-                                                                     StepClock sc) {
+                                                                     int epilogue, StepClock sc,
+                                                                     double *__restrict__ vpart) {
+  if (run_halted(sc.gate)) return;
   const int b = blockIdx.x;
   const UnitKick &k = uk.u[group_kick_unit(uk, b)];
-  brick_kick_mixed_brick<W, U, kSum>(b - k.brick0, k.src, k.mom, nullptr, k.bl, fc, dt2, kKickOnly, sc, nullptr,
-                                     nullptr, NextDrift{nullptr, nullptr, nullptr, nullptr});
+  brick_kick_mixed_brick<W, U, kSum>(b - k.brick0, k.src, k.mom, k.pos_out, k.bl, fc, dt2, epilogue, sc, nullptr,
+                                     vpart ? vpart + k.brick0 : nullptr,
+                                     NextDrift{k.next, nullptr, nullptr, nullptr});
 }
 
 // Dynamic pruning of the pair list (no counterpart in the reference: it

@@ -74,6 +74,7 @@ struct UnitGroup {
   double *part = nullptr;
   size_t part_n = 0;
   unsigned long long *vmax2 = nullptr, *h_vmax2 = nullptr;
+  GroupRun *run = nullptr, *h_run = nullptr;  // a run of the group's steps, and its pinned outcome
 };
 }  // namespace
 
@@ -2619,6 +2620,18 @@ int group_make_pair_list(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us)
   return MDGPU_OK;
 }
 
+// Room for n per-block maxima of the group.
+int ensure_group_part(mdgpu_domain *d, size_t n) {
+  UnitGroup *g = d->group;
+  if (n <= g->part_n) return MDGPU_OK;
+  if (g->part) (void)hipFree(g->part);
+  g->part = nullptr;
+  g->part_n = 0;
+  HIPCHK(d, hipMalloc((void **)&g->part, n * 2 * sizeof(double)));
+  g->part_n = n * 2;
+  return MDGPU_OK;
+}
+
 // MDManager::IsPairListExpired (mdmanager.cc:369-377): every unit's
 // PairList::IsPairListExpired (pairlist.cc:26-65, is_expired), OR'ed.  The
 // units share a stream, so their maxima of |p| are reduced together and read
@@ -2656,13 +2669,7 @@ int group_expired(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, bool *
     }
     G.bbase[ns] = nb;
     G.n = ns;
-    if ((size_t)nb > g->part_n) {
-      if (g->part) (void)hipFree(g->part);
-      g->part = nullptr;
-      g->part_n = 0;
-      HIPCHK(d, hipMalloc((void **)&g->part, (size_t)nb * 2 * sizeof(double)));
-      g->part_n = (size_t)nb * 2;
-    }
+    CHK(ensure_group_part(d, (size_t)nb));
     if (!g->vmax2) {
       HIPCHK(d, hipMalloc((void **)&g->vmax2, kMaxUnits * sizeof(unsigned long long)));
       HIPCHK(d, hipHostMalloc((void **)&g->h_vmax2, kMaxUnits * sizeof(unsigned long long)));
@@ -2736,17 +2743,17 @@ int group_drift(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us) {
   return check_launch(d, "group drift");
 }
 
-// MDManager::SendBorderParticles for every unit in one launch (each unit's
-// ghost sources remapped first where its construction left that pending).
-int group_refresh(mdgpu_domain *d) {
+// MDManager::SendBorderParticles for every unit in one launch: its table (each
+// unit's ghost sources remapped first where its construction left that pending).
+int group_halo(mdgpu_domain *d, GroupHalo &G) {
   UnitGroup *g = d->group;
   std::lock_guard<std::mutex> lock(g->mu);
   const int ns = (int)g->units.size();
-  GroupHalo G{};
   int t = 0;
   for (int w = 0; w < ns; w++) {
     mdgpu_domain *W = g->units[w];
     G.pos[w] = W ? W->pos : nullptr;
+    G.src[w] = G.pos[w];
     G.base[w] = t;
     if (!W || W->ng == 0) continue;
     if (W->ghost_epoch != g->epoch) {
@@ -2763,9 +2770,20 @@ int group_refresh(mdgpu_domain *d) {
   }
   G.base[ns] = t;
   G.n = ns;
-  if (t > 0)
-    hipLaunchKernelGGL(k_group_refresh, dim3(nblk(t)), dim3(kBlock), 0, d->stream, G, g->L[0], g->L[1], g->L[2]);
+  return MDGPU_OK;
+}
+
+int launch_group_refresh(mdgpu_domain *d, const GroupHalo &G, const RunGate *gate) {
+  const double *L = d->group->L;
+  const int t = G.base[G.n];
+  if (t > 0) hipLaunchKernelGGL(k_group_refresh, dim3(nblk(t)), dim3(kBlock), 0, d->stream, G, L[0], L[1], L[2], gate);
   return check_launch(d, "group halo");
+}
+
+int group_refresh(mdgpu_domain *d) {
+  GroupHalo G{};
+  CHK(group_halo(d, G));
+  return launch_group_refresh(d, G, nullptr);
 }
 
 // Temperature over the whole group (MDManager::Temperature, mdmanager.cc:390-397).
@@ -2796,31 +2814,45 @@ int group_temperature(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, do
 // with the launch shape of the unit stepping the group; else one launch per
 // unit.  The units' results are those of their own launches bit for bit: each
 // workgroup does what the unit's own kick does to that brick.
+//
+// A fused step's kick (epilogue kKickDrift) also writes the positions at its
+// end, the next first half drift and the bricks' max |p|^2 (vpart).
+struct GroupKick {
+  UnitKicks uk{};
+  int nb = 0;      // bricks of all units
+  size_t shm = 0;  // LDS of the launch
+  int epilogue = kKickOnly;
+  const RunGate *gate = nullptr;
+  double *vpart = nullptr;
+};
+
 template <int W, int U>
-void launch_group_kick(mdgpu_domain *d, const UnitKicks &uk, int nb, size_t shm) {
-  const StepClock sc{d->dt, d->step, nullptr, nullptr, RunMeasure{}};
+void launch_group_kick(mdgpu_domain *d, const GroupKick &k) {
+  const StepClock sc{d->dt, d->step, nullptr, k.gate, RunMeasure{}};
+  const dim3 grid(k.nb), block(kWave * W);
   if (d->precision == MDGPU_FP64) {
-    allow_lds(k_force_group_fp64<W, U>, shm);
-    hipLaunchKernelGGL((k_force_group_fp64<W, U>), dim3(nb), dim3(kWave * W), shm, d->stream, uk, fconsts(d), sc);
+    allow_lds(k_force_group_fp64<W, U>, k.shm);
+    hipLaunchKernelGGL((k_force_group_fp64<W, U>), grid, block, k.shm, d->stream, k.uk, fconsts(d), k.epilogue, sc,
+                       k.vpart);
     return;
   }
   const ForceConstsF f32 = fconsts32(d);
   const double dt2 = d->dt * 0.5;
   switch (d->kahan) {
     case kSumPlain:
-      allow_lds(k_force_group_mixed_brick<W, U, kSumPlain>, shm);
-      hipLaunchKernelGGL((k_force_group_mixed_brick<W, U, kSumPlain>), dim3(nb), dim3(kWave * W), shm, d->stream, uk,
-                         f32, dt2, sc);
+      allow_lds(k_force_group_mixed_brick<W, U, kSumPlain>, k.shm);
+      hipLaunchKernelGGL((k_force_group_mixed_brick<W, U, kSumPlain>), grid, block, k.shm, d->stream, k.uk, f32, dt2,
+                         k.epilogue, sc, k.vpart);
       break;
     case kSumKahan:
-      allow_lds(k_force_group_mixed_brick<W, U, kSumKahan>, shm);
-      hipLaunchKernelGGL((k_force_group_mixed_brick<W, U, kSumKahan>), dim3(nb), dim3(kWave * W), shm, d->stream, uk,
-                         f32, dt2, sc);
+      allow_lds(k_force_group_mixed_brick<W, U, kSumKahan>, k.shm);
+      hipLaunchKernelGGL((k_force_group_mixed_brick<W, U, kSumKahan>), grid, block, k.shm, d->stream, k.uk, f32, dt2,
+                         k.epilogue, sc, k.vpart);
       break;
     default:
-      allow_lds(k_force_group_mixed_brick<W, U, kSumGroup64>, shm);
-      hipLaunchKernelGGL((k_force_group_mixed_brick<W, U, kSumGroup64>), dim3(nb), dim3(kWave * W), shm, d->stream,
-                         uk, f32, dt2, sc);
+      allow_lds(k_force_group_mixed_brick<W, U, kSumGroup64>, k.shm);
+      hipLaunchKernelGGL((k_force_group_mixed_brick<W, U, kSumGroup64>), grid, block, k.shm, d->stream, k.uk, f32,
+                         dt2, k.epilogue, sc, k.vpart);
       break;
   }
 }
@@ -2833,56 +2865,157 @@ void launch_group_kick(mdgpu_domain *d, const UnitKicks &uk, int nb, size_t shm)
 int group_unroll(const mdgpu_domain *d) { return d->unroll ? d->unroll : 8; }
 
 template <int W>
-void launch_group_kick_w(mdgpu_domain *d, const UnitKicks &uk, int nb, size_t shm) {
-  if (group_unroll(d) == 32) launch_group_kick<W, 4>(d, uk, nb, shm);
-  else if (group_unroll(d) == 16) launch_group_kick<W, 2>(d, uk, nb, shm);
-  else launch_group_kick<W, 1>(d, uk, nb, shm);
+void launch_group_kick_w(mdgpu_domain *d, const GroupKick &k) {
+  if (group_unroll(d) == 32) launch_group_kick<W, 4>(d, k);
+  else if (group_unroll(d) == 16) launch_group_kick<W, 2>(d, k);
+  else launch_group_kick<W, 1>(d, k);
 }
 
-int group_force(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us) {
+// Whether one launch kicks all the units' bricks.
+bool group_batched(const mdgpu_domain *d, const std::vector<mdgpu_domain *> &us) {
   bool batch = (d->precision == MDGPU_FP64 || (d->precision == MDGPU_MIXED && d->mixed_frame == 1)) &&
                !d->pipeline && us.size() <= (size_t)kMaxKickUnits;
-  for (mdgpu_domain *u : us)
+  for (const mdgpu_domain *u : us)
     batch = batch && u->precision == d->precision && u->mixed_frame == d->mixed_frame && u->kahan == d->kahan &&
             u->dt == d->dt && u->CL2 == d->CL2 && u->C2 == d->C2 && u->step == d->step;
-  if (!batch) {
-    for (mdgpu_domain *u : us) CHK(force_in_place(u));
-    return MDGPU_OK;
-  }
+  return batch;
+}
+
+GroupKick group_kick(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us) {
   const int bytes = d->precision == MDGPU_FP64 ? 3 * (int)sizeof(double) : (int)sizeof(float4);
-  UnitKicks uk{};
-  uk.n = (int)us.size();
-  int nb = 0;
-  size_t shm = 0;
+  GroupKick g;
+  g.uk.n = (int)us.size();
   for (size_t k = 0; k < us.size(); k++) {
     mdgpu_domain *u = us[k];
     invalidate(u);
     u->vmax_valid = false;
-    UnitKick &e = uk.u[k];
+    UnitKick &e = g.uk.u[k];
     e.src = u->pos;
     e.mom = u->mom;
     e.bl = brick_list(u, bytes);
-    e.brick0 = nb;
+    e.brick0 = g.nb;
     if (u->pn > 0) {
-      nb += u->nbrick;
-      shm = std::max(shm, (size_t)e.bl.lds_cap * bytes);
+      g.nb += u->nbrick;
+      g.shm = std::max(g.shm, (size_t)e.bl.lds_cap * bytes);
     }
   }
-  if (nb == 0) return MDGPU_OK;
+  return g;
+}
+
+int launch_group_force(mdgpu_domain *d, const GroupKick &k) {
+  if (k.nb == 0) return MDGPU_OK;
   const int ev0 = d->force_launches * 2;
   const bool ev = d->timing && ev0 + 1 < (int)d->ev.size();
   if (ev) HIPCHK(d, hipEventRecord(d->ev[ev0], d->stream));
   switch (d->waves) {
-    case 2: launch_group_kick_w<2>(d, uk, nb, shm); break;
-    case 8: launch_group_kick_w<8>(d, uk, nb, shm); break;
-    case 16: launch_group_kick_w<16>(d, uk, nb, shm); break;
-    default: launch_group_kick_w<4>(d, uk, nb, shm); break;
+    case 2: launch_group_kick_w<2>(d, k); break;
+    case 8: launch_group_kick_w<8>(d, k); break;
+    case 16: launch_group_kick_w<16>(d, k); break;
+    default: launch_group_kick_w<4>(d, k); break;
   }
   if (ev) {
     HIPCHK(d, hipEventRecord(d->ev[ev0 + 1], d->stream));
     d->force_launches++;
   }
   return check_launch(d, "group force");
+}
+
+int group_force(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us) {
+  if (!group_batched(d, us)) {
+    for (mdgpu_domain *u : us) CHK(force_in_place(u));
+    return MDGPU_OK;
+  }
+  return launch_group_force(d, group_kick(d, us));
+}
+
+// The steps a run of the group may take before a unit's budget is spent (each
+// unit has one, and its max |p| from the test of the run's first step): a few
+// more are queued, which do nothing if it is.
+constexpr int kGroupRunMost = 64;
+int group_run_length(const mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, int most) {
+  double n = std::min(most, kGroupRunMost);
+  for (const mdgpu_domain *u : us) {
+    if (!(u->buffer_length > 0.0)) return 1;  // tested on every step
+    const bool known = u->step_vmax > 0.0;  // not before the first test
+    n = std::min(n, known ? u->buffer_length / (2.0 * u->step_vmax * d->dt) + 2.0 : 8.0);
+  }
+  return std::max(1, (int)n);
+}
+
+// Up to `most` NVE steps of the group, queued without the host in between, the
+// first one's expiry test behind them: each step is the halo from the
+// half-drifted positions, the kick with both half drifts in its epilogue, and
+// the units' budgets (k_group_tail), which end the run before a step that the
+// host has to test.  2x2x2 units of 500k particles: 76 us a step against 155
+// with the drifts and maxima in launches of their own (10 us each for the
+// drifts, 10 for the maxima) and a wait per step.
+int group_run(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, int most, int *taken) {
+  UnitGroup *g = d->group;
+  if (!g->run) {
+    HIPCHK(d, hipMalloc((void **)&g->run, sizeof(GroupRun)));
+    HIPCHK(d, hipHostMalloc((void **)&g->h_run, sizeof(GroupRun)));
+  }
+  GroupHalo H{};
+  CHK(group_halo(d, H));
+  GroupKick K = group_kick(d, us);
+  CHK(ensure_group_part(d, (size_t)K.nb + 1));
+  K.epilogue = kKickDrift;
+  K.gate = &g->run->gate;
+  K.vpart = g->part;
+  GroupStart S{};
+  GroupBudgets B{};
+  const int ns = (int)g->units.size();
+  int t = 0;
+  for (int w = 0; w < ns; w++) {
+    mdgpu_domain *W = g->units[w];
+    S.base[w] = t;
+    if (!W) continue;
+    S.pos[w] = W->pos;
+    S.mom[w] = W->mom;
+    S.tmp[w] = W->pos_tmp;
+    t += W->pn;
+  }
+  S.base[ns] = t;
+  S.n = ns;
+  B.n = (int)us.size();
+  for (int k = 0; k < B.n; k++) {
+    B.budget[k] = us[k]->buffer_length;
+    B.margin[k] = us[k]->margin;
+    B.brick0[k] = K.uk.u[k].brick0;
+    K.uk.u[k].pos_out = us[k]->pos;
+  }
+  B.brick0[B.n] = K.nb;
+  const int n = group_run_length(d, us, most), launches0 = d->force_launches;
+  g->h_run->gate.done = -1;
+  hipLaunchKernelGGL(k_group_start, dim3(nblk(std::max(t, 1))), dim3(kBlock), 0, d->stream, S, d->dt * 0.5,
+                     &g->run->gate);
+  for (int s = 1; s <= n; s++) {
+    for (int k = 0; k < B.n; k++) {
+      mdgpu_domain *u = us[k];
+      H.src[u->unit_slot] = u->pos_tmp;
+      K.uk.u[k].src = u->pos_tmp;
+      K.uk.u[k].next = u->pos_next;
+      std::swap(u->pos_tmp, u->pos_next);
+    }
+    CHK(launch_group_refresh(d, H, K.gate));
+    CHK(launch_group_force(d, K));
+    hipLaunchKernelGGL(k_group_tail, dim3(1), dim3(kWave * kGroupRunUnits), 0, d->stream, B, d->dt, s, n - s, g->part,
+                       g->run, g->h_run);
+  }
+  CHK(check_launch(d, "group run"));
+  CHK(sync(d));
+  const int done = g->h_run->gate.done;
+  if (done < 1) {
+    d->err = "internal: a run of the group's steps left no outcome";
+    return MDGPU_ERR_HIP;
+  }
+  if (d->timing) d->force_launches = std::min(d->force_launches, launches0 + done);
+  for (int k = 0; k < B.n; k++) {
+    us[k]->buffer_length = g->h_run->budget[k];
+    us[k]->lifetime += done - 1;
+  }
+  *taken = done;
+  return MDGPU_OK;
 }
 
 int group_calculate(mdgpu_domain *d, int nsteps, int *rebuilds) {
@@ -2920,6 +3053,16 @@ int group_calculate(mdgpu_domain *d, int nsteps, int *rebuilds) {
     if (any) {
       if ((r = group_make_pair_list(d, us)) != MDGPU_OK) break;
       count++;
+    }
+    if (d->thermostat == MDGPU_NVE && group_batched(d, us)) {
+      int n = 0;
+      if ((r = group_run(d, us, nsteps - s, &n)) != MDGPU_OK) break;
+      for (mdgpu_domain *u : us) {
+        for (int k = 0; k < n; k++) u->sim_time += u->dt;
+        u->step += n;
+      }
+      s += n - 1;
+      continue;
     }
     if ((r = group_drift(d, us)) != MDGPU_OK || (r = group_refresh(d)) != MDGPU_OK) break;
     if (d->thermostat == MDGPU_NOSEHOOVER) {
@@ -3191,6 +3334,8 @@ int mdgpu_destroy(mdgpu_domain *d) {
       if (g->part) (void)hipFree(g->part);
       if (g->vmax2) (void)hipFree(g->vmax2);
       if (g->h_vmax2) (void)hipHostFree(g->h_vmax2);
+      if (g->run) (void)hipFree(g->run);
+      if (g->h_run) (void)hipHostFree(g->h_run);
       delete g;
     }
   }

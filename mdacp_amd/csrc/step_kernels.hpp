@@ -500,6 +500,58 @@ __device__ __forceinline__ bool run_budget(double v2, double dt, double margin, 
   return true;
 }
 
+// The validity tests of a group of units in a run of steps (PairList::
+// IsPairListExpired of every unit, OR'ed, mdmanager.cc:369-377), after its
+// step `done` of `left`: each unit's max |p|^2 from its bricks' (vpart), one
+// wavefront per unit, and its budget.  Where every unit's budget outlasts the
+// next step they are committed; else the run halts and the host tests that
+// step itself, from the budgets before it.  Not tested after the last step.
+constexpr int kGroupRunUnits = 8;
+struct GroupRun {
+  RunGate gate;
+  double budget[kGroupRunUnits];
+};
+struct GroupBudgets {
+  double budget[kGroupRunUnits], margin[kGroupRunUnits];
+  int brick0[kGroupRunUnits + 1];
+  int n;
+};
+
+__global__ __launch_bounds__(kWave *kGroupRunUnits) void k_group_tail(GroupBudgets G, double dt, int done, int left,
+                                                                      const double *__restrict__ vpart,
+                                                                      GroupRun *__restrict__ run,
+                                                                      GroupRun *__restrict__ out) {
+  __shared__ double nb[kGroupRunUnits];
+  __shared__ int stop;
+  if (run->gate.halted) return;  // uniform
+  const int u = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (threadIdx.x == 0) stop = 0;
+  __syncthreads();
+  if (u < G.n) {
+    double v2 = 0.0;
+    if (left > 0)
+      for (int k = G.brick0[u] + lane; k < G.brick0[u + 1]; k += kWave) v2 = fmax(v2, vpart[k]);
+    v2 = wave_max(v2);
+    if (lane == 0) {
+      const double b0 = done == 1 ? G.budget[u] : run->budget[u];
+      double b = b0;
+      if (left > 0 && !(run_budget(v2, dt, G.margin[u], b) && b > 0.0)) stop = 1;
+      nb[u] = left > 0 ? b : b0;
+    }
+  }
+  __syncthreads();
+  const bool halt = stop != 0;
+  if (lane == 0 && u < G.n) {
+    const double b = !halt ? nb[u] : done == 1 ? G.budget[u] : run->budget[u];
+    run->budget[u] = b;
+    if (halt || left == 0) out->budget[u] = b;
+  }
+  if (threadIdx.x == 0) {
+    run->gate.halted = halt;
+    if (halt || left == 0) out->gate = RunGate{halt, done, left};
+  }
+}
+
 // A list whose displacements were measured after the last step, the largest
 // squared one dmax2, takes a budget again while none has reached half the
 // margin: no entry is then displaced by more than margin - max displacement,

@@ -8,6 +8,7 @@ import pytest
 
 from mdacp_amd import mdgpu
 from mdacp_amd.ensemble import build
+from mdacp_amd.lattice import fcc, initial_velocity
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +118,36 @@ def test_nose_hoover_runs_follow_single_steps(name):
     assert np.abs(qa - qb).max() < 1e-10 and np.abs(pa - pb).max() < 1e-10
     for e in es:
         e.close()
+
+
+@pytest.mark.parametrize("grid", [(1, 1, 1), (2, 1, 2), (2, 2, 2)])
+@pytest.mark.parametrize("precision,check", [(mdgpu.FP64, 1), (mdgpu.FP64, 0), (mdgpu.MIXED, 1)])
+def test_runs_of_a_group_match_single_steps(grid, precision, check):
+    """Runs of a process grid's units (mdgpu_group_calculate) against one step per call, which the
+    host tests: the same constructions, state, images and time."""
+    print("case:", grid, precision, check, flush=True)
+    L = 14.0
+    q = fcc(L, 0.7)
+    p = initial_velocity(len(q), 1.1, seed=4)
+    ids = np.arange(len(q), dtype=np.int32)
+    groups = []
+    for _ in range(2):
+        us = mdgpu.unit_grid(L, grid, dt=0.005, rc=2.5, margin=0.5, capacity=len(q))
+        for u in us:
+            u.add_particles(q, p, ids)
+            u.set_precision(precision)
+            u.set_option(mdgpu.OPT_DISPLACEMENT_CHECK, check)
+        groups.append(us)
+    a, b = groups
+    ra = rb = 0
+    for chunk in (1, 37, 2, 100):
+        ra += a[0].group_calculate(chunk)
+        rb += sum(b[0].group_calculate(1) for _ in range(chunk))
+        assert ra == rb, (chunk, ra, rb)
+        for u, v in zip(a, b):
+            assert u.counts() == v.counts()
+            for x, y in zip(u.particles(), v.particles()):
+                assert np.array_equal(x, y), chunk
+            assert u.observe_raw() == v.observe_raw()  # the images are the last halo's
+            assert u.time() == v.time()
+    assert ra >= 2, ra
