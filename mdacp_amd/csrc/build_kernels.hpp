@@ -560,7 +560,8 @@ __global__ void k_group_max_p2(GroupMomenta G, double *__restrict__ partial) {
   block_max_to_partial(v, partial, b);
 }
 
-__global__ void k_group_reduce_max(GroupMomenta G, const double *__restrict__ partial,
+template <class T>
+__global__ void k_group_reduce_max(T G, const double *__restrict__ partial,
                                    unsigned long long *__restrict__ out) {
   __shared__ double red[kBlock];
   const int u = blockIdx.x;
@@ -573,6 +574,79 @@ __global__ void k_group_reduce_max(GroupMomenta G, const double *__restrict__ pa
     __syncthreads();
   }
   if (threadIdx.x == 0) out[u] = (unsigned long long)__double_as_longlong(red[0]);
+}
+
+// PairList::CheckByDisplacement (pairlist.cc:68-121) of the units whose budget
+// is spent, all of them in each launch (k_displacement, k_candidates and
+// k_candidate_pairs unit by unit otherwise): blocks aligned to units, the
+// maxima by k_group_reduce_max.  A check is launches and a wait: 50 steps of
+// 500k particles in 2x2x2 units, seven checks among them, took 11.5 ms with
+// eight launches, clears and copies per unit and take 10.1 with these four and
+// one copy.
+constexpr int kCheckUnits = 16;      // units per launch
+constexpr int kCheckPairBlocks = 64; // blocks over a unit's candidate pairs
+struct GroupCheck {
+  const double4 *pos[kCheckUnits], *old[kCheckUnits];
+  double *disp[kCheckUnits];
+  int *cand[kCheckUnits];
+  double margin[kCheckUnits], SL2[kCheckUnits], CL2[kCheckUnits];
+  int tn[kCheckUnits], cap[kCheckUnits];
+  int bbase[kCheckUnits + 1];
+  int n;
+};
+struct UnitCheck {  // a unit's outcome
+  int count, flag;
+};
+
+__global__ void k_group_displacement(GroupCheck G, double *__restrict__ partial, UnitCheck *__restrict__ out) {
+  const int b = blockIdx.x;
+  const int u = group_unit_of(G.bbase, G.n, b);
+  const int i = (b - G.bbase[u]) * blockDim.x + threadIdx.x;
+  if (i == 0) out[u] = UnitCheck{0, 0};
+  double v = 0.0;
+  if (i < G.tn[u]) {
+    const double4 o = G.old[u][i], q = G.pos[u][i];
+    const double dx = o.x - q.x, dy = o.y - q.y, dz = o.z - q.z;
+    v = dx * dx + dy * dy + dz * dz;
+    G.disp[u][i] = v;
+  }
+  block_max_to_partial(v, partial, b);
+}
+
+__global__ void k_group_candidates(GroupCheck G, const unsigned long long *__restrict__ dmax,
+                                   UnitCheck *__restrict__ out) {
+  const int b = blockIdx.x;
+  const int u = group_unit_of(G.bbase, G.n, b);
+  const int i = (b - G.bbase[u]) * blockDim.x + threadIdx.x;
+  if (i >= G.tn[u]) return;
+  const double c_distance = G.margin[u] - sqrt(__longlong_as_double((long long)dmax[u]));
+  if (G.disp[u][i] > c_distance * c_distance) {
+    const int k = atomicAdd(&out[u].count, 1);
+    if (k < G.cap[u]) G.cand[u][k] = i;
+  }
+}
+
+__global__ void k_group_candidate_pairs(GroupCheck G, UnitCheck *__restrict__ out) {
+  const int u = blockIdx.x / kCheckPairBlocks;
+  const int l = out[u].count;
+  if (l <= 1 || l >= min(G.tn[u], G.cap[u])) return;
+  const double4 *pos = G.pos[u], *old = G.old[u];
+  const int *list = G.cand[u];
+  const long long total = (long long)l * l;
+  for (long long t = (long long)(blockIdx.x % kCheckPairBlocks) * blockDim.x + threadIdx.x; t < total;
+       t += (long long)kCheckPairBlocks * blockDim.x) {
+    const int a = (int)(t / l), b = (int)(t % l);
+    if (b <= a) continue;
+    const int i1 = list[a], i2 = list[b];
+    const double4 o1 = old[i1], o2 = old[i2];
+    double dx = o1.x - o2.x, dy = o1.y - o2.y, dz = o1.z - o2.z;
+    if (dx * dx + dy * dy + dz * dz < G.SL2[u]) continue;
+    const double4 q1 = pos[i1], q2 = pos[i2];
+    dx = q1.x - q2.x;
+    dy = q1.y - q2.y;
+    dz = q1.z - q2.z;
+    if (dx * dx + dy * dy + dz * dz < G.CL2[u]) atomicOr(&out[u].flag, 1);
+  }
 }
 
 // A unit's ghost sources follow their source units' row orders: the indices

@@ -56,6 +56,11 @@ struct StepGraph {
   long epoch = -1;
 };
 
+struct GroupChecks {  // largest |dq|^2 (bits), candidates and outcome of the units checked together
+  unsigned long long dmax2[kCheckUnits];
+  UnitCheck unit[kCheckUnits];
+};
+
 // The units of one process grid (MDManager's MDUnits of one process,
 // mdmanager.cc:34-45) on one device: they share one stream, so that work
 // each unit queues after MDManager's phase barriers runs after what every
@@ -75,6 +80,7 @@ struct UnitGroup {
   size_t part_n = 0;
   unsigned long long *vmax2 = nullptr, *h_vmax2 = nullptr;
   GroupRun *run = nullptr, *h_run = nullptr;  // a run of the group's steps, and its pinned outcome
+  GroupChecks *check = nullptr, *h_check = nullptr;  // displacement checks, and their pinned outcome
 };
 }  // namespace
 
@@ -2632,6 +2638,52 @@ int ensure_group_part(mdgpu_domain *d, size_t n) {
   return MDGPU_OK;
 }
 
+// The displacement checks of some units (enqueue_displacement_check for all of
+// them, kCheckUnits at a time), each unit's outcome left where
+// displacement_check_result reads it.
+int group_check_displacements(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us) {
+  UnitGroup *g = d->group;
+  if (!g->check) {
+    HIPCHK(d, hipMalloc((void **)&g->check, sizeof(GroupChecks)));
+    HIPCHK(d, hipHostMalloc((void **)&g->h_check, sizeof(GroupChecks)));
+  }
+  for (size_t k0 = 0; k0 < us.size(); k0 += kCheckUnits) {
+    GroupCheck G{};
+    G.n = (int)std::min(us.size() - k0, (size_t)kCheckUnits);
+    for (int k = 0; k < G.n; k++) {
+      const mdgpu_domain *u = us[k0 + k];
+      G.pos[k] = u->pos;
+      G.old[k] = u->pos_old;
+      G.disp[k] = u->disp;
+      G.cand[k] = u->cand;
+      G.margin[k] = u->margin;
+      G.SL2[k] = u->SL * u->SL;
+      G.CL2[k] = u->CL2;
+      G.tn[k] = u->tn;
+      G.cap[k] = u->check_list_length;
+      G.bbase[k + 1] = G.bbase[k] + (int)std::max(1u, nblk(u->tn));
+    }
+    const int nb = G.bbase[G.n];
+    CHK(ensure_group_part(d, (size_t)nb));
+    const dim3 grid(nb), block(kBlock);
+    GroupChecks *c = g->check;
+    hipLaunchKernelGGL(k_group_displacement, grid, block, 0, d->stream, G, g->part, c->unit);
+    hipLaunchKernelGGL(k_group_reduce_max<GroupCheck>, dim3(G.n), block, 0, d->stream, G, g->part, c->dmax2);
+    hipLaunchKernelGGL(k_group_candidates, grid, block, 0, d->stream, G, c->dmax2, c->unit);
+    hipLaunchKernelGGL(k_group_candidate_pairs, dim3(G.n * kCheckPairBlocks), block, 0, d->stream, G, c->unit);
+    CHK(check_launch(d, "group displacement check"));
+    HIPCHK(d, hipMemcpyAsync(g->h_check, c, sizeof(GroupChecks), hipMemcpyDeviceToHost, d->stream));
+    CHK(sync(d));
+    for (int k = 0; k < G.n; k++) {
+      mdgpu_domain *u = us[k0 + k];
+      u->h_u64[1] = g->h_check->dmax2[k];
+      u->h_i32[1] = g->h_check->unit[k].count;
+      u->h_i32[2] = g->h_check->unit[k].flag;
+    }
+  }
+  return MDGPU_OK;
+}
+
 // MDManager::IsPairListExpired (mdmanager.cc:369-377): every unit's
 // PairList::IsPairListExpired (pairlist.cc:26-65, is_expired), OR'ed.  The
 // units share a stream, so their maxima of |p| are reduced together and read
@@ -2675,7 +2727,7 @@ int group_expired(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, bool *
       HIPCHK(d, hipHostMalloc((void **)&g->h_vmax2, kMaxUnits * sizeof(unsigned long long)));
     }
     hipLaunchKernelGGL(k_group_max_p2, dim3(nb), dim3(kBlock), 0, d->stream, G, g->part);
-    hipLaunchKernelGGL(k_group_reduce_max, dim3(ns), dim3(kBlock), 0, d->stream, G, g->part, g->vmax2);
+    hipLaunchKernelGGL(k_group_reduce_max<GroupMomenta>, dim3(ns), dim3(kBlock), 0, d->stream, G, g->part, g->vmax2);
     CHK(check_launch(d, "group max |p|"));
     HIPCHK(d, hipMemcpyAsync(g->h_vmax2, g->vmax2, ns * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                              d->stream));
@@ -2696,7 +2748,7 @@ int group_expired(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, bool *
     }
     u->buffer_length = u->buffer_length - vmax * 2.0 * u->dt;
   }
-  queued = false;
+  std::vector<mdgpu_domain *> checked;
   for (size_t k = 0; k < us.size(); k++) {
     mdgpu_domain *u = us[k];
     if (!u->initialized || !(u->buffer_length < 0.0)) continue;
@@ -2704,12 +2756,10 @@ int group_expired(mdgpu_domain *d, const std::vector<mdgpu_domain *> &us, bool *
       *any = true;
       continue;
     }
-    const int r = enqueue_displacement_check(u);
-    if (r != MDGPU_OK) return group_fail(d, u, r);
     check_of[k] = 1;
-    queued = true;
+    checked.push_back(u);
   }
-  if (queued) CHK(sync(d));
+  if (!checked.empty()) CHK(group_check_displacements(d, checked));
   for (size_t k = 0; k < us.size(); k++) {
     if (!check_of[k]) continue;
     int e = 0;
@@ -3335,6 +3385,8 @@ int mdgpu_destroy(mdgpu_domain *d) {
       if (g->vmax2) (void)hipFree(g->vmax2);
       if (g->h_vmax2) (void)hipHostFree(g->h_vmax2);
       if (g->run) (void)hipFree(g->run);
+      if (g->check) (void)hipFree(g->check);
+      if (g->h_check) (void)hipHostFree(g->h_check);
       if (g->h_run) (void)hipHostFree(g->h_run);
       delete g;
     }

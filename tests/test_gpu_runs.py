@@ -120,13 +120,13 @@ def test_nose_hoover_runs_follow_single_steps(name):
         e.close()
 
 
-@pytest.mark.parametrize("grid", [(1, 1, 1), (2, 1, 2), (2, 2, 2)])
+@pytest.mark.parametrize("grid", [(1, 1, 1), (2, 1, 2), (2, 2, 2), (3, 3, 2)])  # 18: more than one launch checks
 @pytest.mark.parametrize("precision,check", [(mdgpu.FP64, 1), (mdgpu.FP64, 0), (mdgpu.MIXED, 1)])
 def test_runs_of_a_group_match_single_steps(grid, precision, check):
     """Runs of a process grid's units (mdgpu_group_calculate) against one step per call, which the
     host tests: the same constructions, state, images and time."""
     print("case:", grid, precision, check, flush=True)
-    L = 14.0
+    L = 20.0 if max(grid) > 2 else 14.0
     q = fcc(L, 0.7)
     p = initial_velocity(len(q), 1.1, seed=4)
     ids = np.arange(len(q), dtype=np.int32)
