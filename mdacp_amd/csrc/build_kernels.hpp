@@ -331,7 +331,7 @@ __global__ void k_leave_flags(const double4 *__restrict__ pos, int n, int dir, d
 
 // MDUnit::MakeBufferForSendingParticle (mdunit.cc:78-101): the particles that
 // leave go to the send buffer in their order (off = exclusive scan of the
-// flags), the others are compacted in theirs.
+// flags, from any value), the others are compacted in theirs.
 __global__ void k_partition(const int *__restrict__ flag, const int *__restrict__ off, int n,
                             const double4 *__restrict__ pos, const double4 *__restrict__ mom,
                             const int *__restrict__ id, double4 *__restrict__ pos_keep,
@@ -340,7 +340,7 @@ __global__ void k_partition(const int *__restrict__ flag, const int *__restrict_
                             int *__restrict__ id_send) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int o = off[i];
+  const int o = off[i] - off[0];
   if (flag[i]) {
     pos_send[o] = pos[i];
     mom_send[o] = mom[i];
@@ -647,6 +647,48 @@ __global__ void k_group_candidate_pairs(GroupCheck G, UnitCheck *__restrict__ ou
     dz = q1.z - q2.z;
     if (dx * dx + dy * dy + dz * dz < G.CL2[u]) atomicOr(&out[u].flag, 1);
   }
+}
+
+// k_leave_flags for every unit of a group in one launch, the flags of the units
+// one after another; after their scan, how many of each unit leave.
+struct GroupLeave {
+  const double4 *pos[kMaxUnits];
+  double s[kMaxUnits], e[kMaxUnits];  // the units' boxes along the direction's axis
+  int base[kMaxUnits + 1];
+  int n;
+};
+
+__global__ void k_group_leave_flags(GroupLeave G, int dir, int *__restrict__ flag) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= G.base[G.n]) return;
+  const int u = group_unit_of(G.base, G.n, t);
+  const double4 q = G.pos[u][t - G.base[u]];
+  const int a = dir >> 1;
+  const double v = a == 0 ? q.x : (a == 1 ? q.y : q.z);
+  flag[t] = (dir & 1) ? (v >= G.e[u]) : (v < G.s[u]);
+}
+
+// off: the exclusive scan of the flags, total[0] their sum; count is in pinned memory
+__global__ void k_group_leaving(GroupLeave G, const int *__restrict__ off, const long long *__restrict__ total,
+                                int *__restrict__ count) {
+  const int u = threadIdx.x;
+  if (u >= G.n) return;
+  const int all = G.base[G.n];
+  auto at = [&](int t) { return t < all ? off[t] : (int)total[0]; };
+  count[u] = at(G.base[u + 1]) - at(G.base[u]);
+}
+
+// MDUnit::ReceiveParticles (mdunit.cc:104-122): n particles from a send buffer
+// appended to a unit's pn.
+__global__ void k_receive(double4 *__restrict__ pos, double4 *__restrict__ mom, int *__restrict__ id,
+                          int *__restrict__ rep, int pn, int n, const double4 *__restrict__ spos,
+                          const double4 *__restrict__ smom, const int *__restrict__ sid) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  pos[pn + i] = spos[i];
+  mom[pn + i] = smom[i];
+  id[pn + i] = sid[i];
+  rep[pn + i] = 0;
 }
 
 // A unit's ghost sources follow their source units' row orders: the indices

@@ -151,3 +151,53 @@ def test_runs_of_a_group_match_single_steps(grid, precision, check):
             assert u.observe_raw() == v.observe_raw()  # the images are the last halo's
             assert u.time() == v.time()
     assert ra >= 2, ra
+
+
+@pytest.mark.parametrize("grid,n", [((1, 1, 1), 300), ((2, 2, 2), 4000), ((3, 1, 2), 4000), ((2, 2, 2), 9), ((2, 2, 2), 0)])
+def test_a_groups_construction_is_its_units_phases(grid, n):
+    """mdgpu_group_make_pair_list against MDManager's phases unit by unit, bit for bit, for
+    particles that leave through every face and corner, units that none leave, and empty units."""
+    print("case:", grid, n, flush=True)
+    L = 20.0
+    rng = np.random.default_rng(n + 1)
+    q = rng.uniform(0.0, L, (n, 3))
+    p = rng.normal(size=(n, 3))
+    ids = rng.permutation(n).astype(np.int32)
+    sides = []
+    for _ in range(2):
+        us = mdgpu.unit_grid(L, grid, dt=0.4, rc=2.5, margin=0.5, capacity=max(n, 1))
+        for u in us:
+            u.add_particles(q, p, ids)
+        sides.append(us)
+    a, b = sides
+    for _ in range(3):
+        for u in a + b:
+            u.update_position_half()  # 0.2 p: up to a search length across the faces
+        a[0].group_make_pair_list()
+        for d in range(6):
+            for u in b:
+                u.send_particles(d)
+            for u in b:
+                u.receive_particles(b[neighbor(grid, b.index(u), d ^ 1)])
+        for u in b:
+            u.adjust_periodic_boundary()
+        for u in b:
+            u.find_border_particles()
+        for u in b:
+            u.make_pair_list()
+        for u in a + b:
+            u.send_border_particles()
+        assert sum(u.counts()[0] for u in a) == n
+        for u, v in zip(a, b):
+            assert u.counts() == v.counts()
+            for x, y in zip(u.particles(), v.particles()):
+                assert np.array_equal(x, y)
+            assert u.observe_raw() == v.observe_raw()
+
+
+def neighbor(grid, k, d):
+    """Index in unit_grid's order of unit k's neighbour in direction d."""
+    boxes = [tuple(pos) for pos, _, _ in mdgpu.unit_boxes(20.0, grid)]
+    pos = list(boxes[k])
+    pos[d >> 1] = (pos[d >> 1] + (1 if d & 1 else -1)) % grid[d >> 1]
+    return boxes.index(tuple(pos))
