@@ -41,15 +41,23 @@ __device__ __forceinline__ LangevinConsts langevin_consts(const Replica &R, doub
 }
 
 // ---------------------------------------------------------------- drift
-__global__ void k_drift(double4 *__restrict__ pos, const double4 *__restrict__ mom, int pn, double dt2) {
+// With vmax, each block's max |p|^2 goes there (pinned memory), so that the
+// validity test after it needs no launches of its own.
+constexpr int kDriftBlocks = 1024;  // at most, with vmax
+__global__ void k_drift(double4 *__restrict__ pos, const double4 *__restrict__ mom, int pn, double dt2,
+                        double *__restrict__ vmax) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= pn) return;
-  double4 q = pos[i];
-  const double4 p = mom[i];
-  q.x += p.x * dt2;
-  q.y += p.y * dt2;
-  q.z += p.z * dt2;
-  pos[i] = q;
+  double v = 0.0;
+  if (i < pn) {
+    double4 q = pos[i];
+    const double4 p = mom[i];
+    q.x += p.x * dt2;
+    q.y += p.y * dt2;
+    q.z += p.z * dt2;
+    pos[i] = q;
+    v = p.x * p.x + p.y * p.y + p.z * p.z;
+  }
+  if (vmax != nullptr) block_max_to_partial(v, vmax, blockIdx.x);
 }
 
 // SendBorderParticles: ghosts [pn, pn + ng) from the current owned positions.

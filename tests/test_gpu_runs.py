@@ -201,3 +201,38 @@ def neighbor(grid, k, d):
     pos = list(boxes[k])
     pos[d >> 1] = (pos[d >> 1] + (1 if d & 1 else -1)) % grid[d >> 1]
     return boxes.index(tuple(pos))
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1024 * 256, 1024 * 256 + 1])
+def test_the_drifts_largest_momentum(n):
+    """The validity test reads max |p| from the half drift before it where that left it, from the
+    momenta otherwise: the same number, the momenta's at that time."""
+    print("case:", n, flush=True)
+    L = max(9.0, (n / 0.5) ** (1.0 / 3.0))
+    rng = np.random.default_rng(n)
+    q = fcc(L, 0.7)
+    q = q[np.sort(rng.choice(len(q), n, replace=False))]
+    p = rng.normal(size=(n, 3))
+    p[rng.integers(n)] *= 300.0 / np.linalg.norm(p, axis=1).max()
+    d = mdgpu.Domain(L, dt=0.005, rc=2.5, margin=0.5, capacity=n)
+    d.set_thermostat(mdgpu.LANGEVIN, T=1.0, gamma=1.0)
+    d.add_particles(q, p, np.arange(n, dtype=np.int32))
+
+    def fastest():
+        return np.sqrt((d.particles()[1] ** 2).sum(axis=1).max())
+
+    def tested():
+        with pytest.raises(Exception, match="Too fast") as e:
+            d.is_pair_list_expired()
+        return float(str(e.value).split("max_velocity = ")[1].split(")")[0])
+
+    d.make_pair_list()
+    bar = dict(rel=1e-12, abs=1e-6)  # the message has six decimals
+    assert tested() == pytest.approx(fastest(), **bar)
+    d.update_position_half()
+    assert tested() == pytest.approx(fastest(), **bar)
+    d.langevin()
+    v = fastest()
+    assert tested() == pytest.approx(v, **bar)
+    d.update_position_half()
+    assert tested() == pytest.approx(v, **bar)
