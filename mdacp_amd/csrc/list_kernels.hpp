@@ -221,7 +221,7 @@ __device__ __forceinline__ double4 gather_pos(const double4 *__restrict__ src, c
 // kImgBits bits and, above them, two bits per axis (0: no shift, 1: +L, 2: -L).
 // A fused step's kick stages the ghost images from these straight from the
 // half-drifted owned positions, so no halo refresh runs before it: one launch
-// less per step (8 us of 375 at 4M particles, 6 of 40 at 2,048).
+// less per step (8.3 us of 375 at 4M particles, 3.4 of 40 at 2,048).
 constexpr int kImgBits = 26;
 static_assert(kMaxParticles < (1 << kImgBits), "an owned index fits a gather entry");
 
@@ -871,7 +871,7 @@ __device__ __forceinline__ void cursor_run(MaskCursor &c, const RowCell &rc, con
 }
 
 // MeshList::MakeList (meshlist.cc:58-87) in sliced-ELL form: one wavefront per
-// 64-row slice (rows in the order of k_brick_row_order, rowsrc[row] = the
+// 64-row slice (rows in the order of k_order_rows, rowsrc[row] = the
 // row's index in the search) turns the rows' candidate masks into staged
 // indices and, with kCodes, cell offset codes.  All lanes produce entry j of
 // group g together, each from its own row's mask (or the brick's pad entry

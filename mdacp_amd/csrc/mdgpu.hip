@@ -3057,11 +3057,10 @@ void launch_group_kick(mdgpu_domain *d, const GroupKick &k) {
   }
 }
 
-// The group kick's indices ahead: unless set, 8 for both precisions.  The
-// FP64 group kernel with 16 takes 136 registers, which fits one 512-thread
-// workgroup per CU instead of two (94 registers with 8): 0.381 against
-// 0.310 ms per launch for 2x2x2 units of 4M particles.  The sums are the same
-// at any depth.
+// The group kick's indices ahead: unless set, 8 for both precisions.  With 16
+// the FP64 kernel (113 registers against 107) takes the same time, 351 to 356
+// against 355 to 364 us for 2x2x2 units of 4M particles, and the mixed one 326
+// against 321 us.  The sums are the same at any depth.
 int group_unroll(const mdgpu_domain *d) { return d->unroll ? d->unroll : 8; }
 
 template <int W>
