@@ -409,8 +409,16 @@ __global__ void k_unit_count(const SrcUnit *__restrict__ tab, int nsrc, int tota
 
 // The images of k_unit_count's count, at off[t]: source index and a word
 // holding the shift code and the source unit (ghost_word), the position, the
+// Owned positions of every unit of a group, by unit slot.
+struct UnitPos {
+  const double4 *pos[kMaxUnits];
+};
+
 // receiver's cell and a slot in it.  The shift is added as image_of adds it.
-__global__ void k_unit_emit(const SrcUnit *__restrict__ tab, int nsrc, int total, int self, double SL,
+// The positions come in the arguments, not from the table: making room for the
+// ghosts may have moved them since it was copied, and the pinned table is free
+// to be written again as soon as this is queued.
+__global__ void k_unit_emit(const SrcUnit *__restrict__ tab, UnitPos P, int nsrc, int total, int self, double SL,
                             const int *__restrict__ off, int ng, double Lx, double Ly, double Lz,
                             const Replica *__restrict__ reps, int *__restrict__ gsrc, int *__restrict__ gword,
                             double4 *__restrict__ gpos, int *__restrict__ gcell, int *__restrict__ gslot,
@@ -420,7 +428,7 @@ __global__ void k_unit_emit(const SrcUnit *__restrict__ tab, int nsrc, int total
   const int w = unit_source(tab, nsrc, t);
   const SrcUnit &S = tab[w];
   const int i = t - S.base;
-  const double4 q = S.pos[i];
+  const double4 q = P.pos[w][i];
   int ox[3], oy[3], oz[3];
   const int nx = unit_axis_options(S, 0, q.x, SL, ox);
   const int ny = unit_axis_options(S, 1, q.y, SL, oy);
@@ -445,11 +453,6 @@ __global__ void k_unit_emit(const SrcUnit *__restrict__ tab, int nsrc, int total
         k++;
       }
 }
-
-// Owned positions of every unit of a group, by unit slot.
-struct UnitPos {
-  const double4 *pos[kMaxUnits];
-};
 
 // The row order each unit of a group gave its owned particles at its last
 // construction (old index -> new), by unit slot.

@@ -2465,7 +2465,9 @@ int ensure_unit_counts(mdgpu_domain *d, long long total) {
 // its own.  Every unit of the group must have been through unit_adjust.  The
 // group's lock keeps the units' positions where this reads them: another
 // unit placing its ghosts may reallocate its arrays.
-// In parts, so that a group counts for all its units before one wait.
+// In parts, so that a group counts for all its units before one wait; the
+// pinned table is copied here only, and that wait comes before it is written
+// again.
 int queue_unit_ghost_count(mdgpu_domain *d) {
   UnitGroup *g = d->group;
   hipStream_t st = d->stream;
@@ -2521,19 +2523,12 @@ int place_unit_ghosts(mdgpu_domain *d) {
   const int pn = d->pn, total = d->src_total;
   const int nsrc = (int)g->units.size();
   const int ng = total > 0 ? (int)d->h_bs->ng : 0;
-  bool moved = false;  // positions moved with their unit's room: the table follows
-  for (int w = 0; w < nsrc; w++) {
-    const mdgpu_domain *W = g->units[w];
-    if (!W || d->h_src_tab[w].pos == W->pos) continue;
-    d->h_src_tab[w].pos = W->pos;
-    moved = true;
-  }
-  if (moved)
-    HIPCHK(d, hipMemcpyAsync(d->src_tab, d->h_src_tab, nsrc * sizeof(SrcUnit), hipMemcpyHostToDevice, st));
+  UnitPos P{};  // where the units' positions are now that there is room
+  for (int w = 0; w < nsrc; w++) P.pos[w] = g->units[w] ? g->units[w]->pos : nullptr;
   HIPCHK(d, hipMemsetAsync(d->c_gcount, 0, sizeof(int) * d->ncell, st));  // placed twice: counted twice
   if (ng > 0) {
     // pos_tmp[0..ng) holds the unsorted images
-    hipLaunchKernelGGL(k_unit_emit, dim3(nblk(total)), dim3(kBlock), 0, st, d->src_tab, nsrc, total,
+    hipLaunchKernelGGL(k_unit_emit, dim3(nblk(total)), dim3(kBlock), 0, st, d->src_tab, P, nsrc, total,
                        d->unit_slot, d->SL, d->uoff, ng, g->L[0], g->L[1], g->L[2], d->reps, d->t_gsrc, d->t_gcode,
                        d->pos_tmp, d->t_gcell, d->slot, d->c_gcount);
     CHK(check_launch(d, "unit ghosts"));
@@ -2551,8 +2546,6 @@ int place_unit_ghosts(mdgpu_domain *d) {
   d->ghosts_ready = true;
   d->ghost_epoch = g->epoch;
   d->ghost_remap = true;
-  // the host table is read by the copies above before it is written again:
-  // the next write follows a wait of this unit's next migration
   return check_launch(d, "unit ghosts");
 }
 
