@@ -32,12 +32,14 @@ constexpr int kErrSearchCap = 16;   // a row has more candidates than its bitmas
 constexpr int kErrGhostCap = 32;    // more ghost images than there is room for
 constexpr int kErrGatherCap = 64;   // ... gather-list entries
 constexpr int kErrSlotCap = 128;    // ... list slots
+constexpr int kErrStagedCap = 256;  // a brick stages more entries than 16 bits index
 // A construction's kernels run one after another without the host, on the
 // room the last construction needed and a little more.  One that finds too
 // little sets its bit; the kernels after it do nothing; and the host, which
 // reads the state once at the end, makes room and queues them again from
 // there.  Bits set before the rows are ordered:
-constexpr int kErrBeforeRows = kErrInvalidPosition | kErrInvalidIndex | kErrSearchCap | kErrGhostCap | kErrGatherCap;
+constexpr int kErrBeforeRows =
+    kErrInvalidPosition | kErrInvalidIndex | kErrSearchCap | kErrGhostCap | kErrGatherCap | kErrStagedCap;
 
 // What a construction's kernels count (device; copied to the host at its end).
 struct BuildState {

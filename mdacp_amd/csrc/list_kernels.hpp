@@ -94,15 +94,20 @@ struct ScanBricks {
 // empty).  tstart = first index in the owned+ghost arrays (ghosts from pn on),
 // tbase = offset in the staged array (tbase[R] = staged count = pad slot).
 // One wavefront per brick, a lane per neighbourhood cell, the offsets from a
-// wavefront prefix sum.  A brick without rows stages nothing.
+// wavefront prefix sum.  A brick without rows stages nothing.  One that would
+// stage more than kMaxStaged entries stops the construction here, before a
+// search whose work grows with the square of that number.
+constexpr int kMaxStaged = 65534;  // list entries are 16-bit staged indices, the pad entry's among them
+
 __global__ __launch_bounds__(kBlock) void k_brick_ranges(Bricks B, CellTables T, int nbrick, int pn,
                                                          const int *__restrict__ nrow, int *__restrict__ tstart,
                                                          int *__restrict__ tbase, int *__restrict__ nrange,
                                                          int *__restrict__ btotal,
-                                                         const BuildState *__restrict__ bs) {
+                                                         BuildState *__restrict__ bs) {
   const int b = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave;
-  if (b >= nbrick || bs->err) return;  // the whole wavefront
+  // the whole wavefront (the one bit this kernel sets is left out: every lane decides alike)
+  if (b >= nbrick || (bs->err & ~kErrStagedCap)) return;
   if (nrow[b] == 0) {
     if (lane == 0) {
       nrange[b] = 0;
@@ -151,6 +156,7 @@ __global__ __launch_bounds__(kBlock) void k_brick_ranges(Bricks B, CellTables T,
     tb[kRangesPerCell * nc] = base;
     nrange[b] = kRangesPerCell * nc;
     btotal[b] = base;
+    if (base > kMaxStaged) atomicOr(&bs->err, kErrStagedCap);
   }
 }
 

@@ -1082,22 +1082,20 @@ int ensure_build(mdgpu_domain *d) {
     CHK(dalloc(d, &d->mask, need + need / 8));
     d->mask_cap = need + need / 8;
   }
-  double entries = 0.0, slots = 0.0;
+  double entries = 0.0, slots = 0.0, staged = 0.0;
   for (int r = 0; r < d->nrep; r++) {
     const Replica &R = d->rh[r];
     const double pn = d->nrep == 1 ? d->pn : R.pn, rho = pn / (R.L[0] * R.L[1] * R.L[2]);
-    entries += rho * R.w[0] * R.w[1] * R.w[2] * R.nb[0] * R.nb[1] * R.nb[2] *
-               ((R.bd[0] + 2) * (R.bd[1] + 2) * (R.bd[2] + 2));
+    staged = rho * R.w[0] * R.w[1] * R.w[2] * ((R.bd[0] + 2) * (R.bd[1] + 2) * (R.bd[2] + 2));
+    if (staged > kMaxStaged) continue;  // k_brick_ranges will refuse it: no room for its list
+    entries += staged * R.nb[0] * R.nb[1] * R.nb[2];
     slots += pn * (rho * (4.0 / 3.0) * M_PI * d->SL * d->SL * d->SL * 1.25 + 16.0);
   }
   if (d->glist_cap == 0) CHK(grow_glist(d, (long long)(1.1 * entries)));
   if (d->nbr_cap == 0) CHK(grow_slots(d, (long long)slots));
-  if (d->staged_guess == 0 && d->nrep == 1 && d->pn > 0) {
-    // new bricks: the mean neighbourhood and a sixth more
-    const Replica &R = d->rh[0];
-    d->staged_guess = (int)std::min(65534.0, 1.16 * (d->pn / (R.L[0] * R.L[1] * R.L[2])) * R.w[0] * R.w[1] * R.w[2] *
-                                                 ((R.bd[0] + 2) * (R.bd[1] + 2) * (R.bd[2] + 2)));
-  }
+  // new bricks: the mean neighbourhood and a sixth more
+  if (d->staged_guess == 0 && d->nrep == 1 && d->pn > 0)
+    d->staged_guess = (int)std::min((double)kMaxStaged, 1.16 * staged);
   return MDGPU_OK;
 }
 
@@ -1142,6 +1140,10 @@ int finish_queued_build(mdgpu_domain *d, BuildStage from) {
       if (from == kStageImages && pn > 0) swap_owned(d);  // k_sort_owned did not run
       return build_error(d, S.err);
     }
+    if (S.err & kErrStagedCap) {
+      d->err = "a brick's neighbourhood exceeds 16-bit indexing (extreme local density): use smaller bricks";
+      return MDGPU_ERR_CAPACITY;
+    }
     if (S.err & kErrGhostCap) {
       if (S.ng + pn + 1 > kMaxParticles) {
         d->err = "particle capacity exceeded (owned + ghosts)";
@@ -1172,10 +1174,6 @@ int finish_queued_build(mdgpu_domain *d, BuildStage from) {
   }
   const BuildState &S = *d->h_bs;
   d->max_staged = S.max_staged;
-  if (d->max_staged > 65534) {
-    d->err = "a brick's neighbourhood exceeds 16-bit indexing (extreme local density): use smaller bricks";
-    return MDGPU_ERR_CAPACITY;
-  }
   d->staged_guess = std::max(1, d->max_staged);
   d->ng = d->ng_last = (int)S.ng;
   d->tn = pn + d->ng;

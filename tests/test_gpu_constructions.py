@@ -1,12 +1,22 @@
 """Constructions off the usual path on the GPU: phases of a unit repeated, room that runs out at each
 stage, and states that are refused."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from mdacp_amd import mdgpu
 from mdacp_amd.lattice import fcc, initial_velocity
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
+
+
+def free_bytes():
+    """Free device memory (the HIP runtime that the library has loaded)."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert mdgpu.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 @pytest.mark.parametrize("grid", [(2, 2, 2), (1, 1, 1), (3, 1, 2)])
@@ -40,3 +50,33 @@ def test_a_units_ghosts_placed_again(grid):
             assert np.array_equal(x, y)
         assert np.array_equal(u.pairs(), v.pairs())
         assert u.observe_raw() == v.observe_raw()
+
+
+@pytest.mark.parametrize("state", ["even", "cluster"])
+def test_a_neighbourhood_beyond_16_bits_is_refused_before_the_search(state):
+    """More particles around a brick than 16-bit indices reach: the capacity error, without the masks
+    and lists that a search of them would need (2 GB and more), and a domain that still works."""
+    print("case: refused neighbourhood", state, flush=True)
+    rng = np.random.default_rng(3)
+    if state == "even":
+        L, q = 12.0, rng.uniform(0.0, 12.0, (165000, 3))  # 69,600 in 27 of 64 cells
+    else:
+        L, q = 20.0, np.concatenate([fcc(20.0, 0.5), rng.uniform(7.5, 8.5, (66000, 3))])
+    d = mdgpu.Domain(L, dt=0.005, rc=2.5, margin=0.5, capacity=len(q))
+    d.add_particles(q)
+    before = free_bytes()
+    with pytest.raises(mdgpu.MDGPUError, match="16-bit") as e:
+        d.make_pair_list()
+    assert e.value.code == mdgpu.ERR_CAPACITY
+    assert before - free_bytes() < 1 << 29
+    assert np.array_equal(np.sort(d.particles()[2]), np.arange(len(q)))
+    d.clear_particles()
+    x = fcc(L, 0.6)
+    fresh = mdgpu.Domain(L, dt=0.005, rc=2.5, margin=0.5, capacity=len(x))
+    for f in (d, fresh):
+        f.add_particles(x, initial_velocity(len(x), 1.0, seed=1))
+        f.make_pair_list()
+    assert np.array_equal(O.canonical_pairs(d.pairs()), O.canonical_pairs(fresh.pairs()))
+    d.calculate(20)
+    for f in (d, fresh):
+        f.close()
