@@ -170,7 +170,7 @@ struct mdgpu_domain {
   // test at the end of the step before, k_run_tail): at most run_ahead steps
   // per run (0: every step waits)
   int run_ahead = 64;
-  StepGraph gated[2];
+  StepGraph gated[2], single[2];  // steps of a run; the step of a run of one
   RunGate *gate = nullptr, *h_gate = nullptr;  // device state and its pinned mirror
   RunRep *rr = nullptr, *h_rr = nullptr;       // per replica: list state of a run, and its pinned mirror
   RunCand *run_cand = nullptr;                 // candidates of the runs' displacement tests
@@ -179,7 +179,7 @@ struct mdgpu_domain {
   double *kpart = nullptr;                     // one kinetic energy per brick workgroup (Nose-Hoover)
   bool run_halted = false;  // the last run stopped at a step that the host decides
   bool run_keep = false;    // what the last run's last step measured still holds
-  int since_build = 0;      // run steps since the last construction
+  int since_build = 0;      // steps since the last construction
   int list_span = 0;        // ... when the last list expired (0: none has)
 
   // thermostat
@@ -1794,13 +1794,18 @@ bool inner_steps(const mdgpu_domain *d) { return d->prune_delta > 0.0 && d->ther
 
 // The fused step's launches.  gated: a step of a run, whose launches do nothing
 // once the run has halted, and which leaves the halo refresh out where the
-// kick takes the images from their owners (run_gated writes the ghosts once
-// after the run).
-int enqueue_fused(mdgpu_domain *d, unsigned long long *clock, bool prune = false, bool gated = false) {
+// kick takes the images from their owners, and the positions at its end
+// (final_positions writes both once after the run).  single: the step of a run
+// of one, which refreshes the halo and writes the positions itself: one step a
+// call at 3.88M particles takes 452 us so, 495 with the launch after the run
+// that reads and writes every particle again (119,000: 46 and 48).
+int enqueue_fused(mdgpu_domain *d, unsigned long long *clock, bool prune = false, bool gated = false,
+                  bool single = false) {
   hipStream_t st = d->stream;
   const bool mixed = rel_frame(d);
   RunGate *gate = gated ? d->gate : nullptr;
-  if (d->ng > 0 && !(gated && fused_images(d))) {
+  const bool later = gated && !single;  // final_positions follows
+  if (d->ng > 0 && !(later && fused_images(d))) {
     if (mixed)
       hipLaunchKernelGGL((k_refresh_from_drifted<true>), dim3(nblk(d->ng)), dim3(kBlock), 0, st, d->pos, d->pos_tmp,
                          d->gsrc, d->gcode, d->pn, d->ng, d->reps, d->cell, d->org, d->rel_tmp, gate);
@@ -1814,11 +1819,10 @@ int enqueue_fused(mdgpu_domain *d, unsigned long long *clock, bool prune = false
                   : d->thermostat == MDGPU_NOSEHOOVER ? kKickNoseHoover
                                                       : kKickDrift;
   const NextDrift nd{d->pos_next, mixed ? d->rel_next : nullptr, d->cell, d->org};
-  // a run's steps leave the final owned positions out (run_gated writes them
-  // after the run); a timed step does too and writes them after its timed kick,
-  // so that the events time the kernel the runs launch
+  // a timed step writes the final positions after its timed kick, so that the
+  // events time the kernel the runs launch
   const bool timed = d->timing && clock == nullptr && !gated;
-  CHK(launch_force(d, d->pos_tmp, d->rel_tmp, gated || timed ? nullptr : d->pos, epi, true, nd, clock,
+  CHK(launch_force(d, d->pos_tmp, d->rel_tmp, later || timed ? nullptr : d->pos, epi, true, nd, clock,
                    inner_steps(d), gated));
   if (timed && d->pn > 0) CHK(final_positions(d, d->pos_tmp));
   return MDGPU_OK;
@@ -1835,8 +1839,8 @@ void drop_graph(StepGraph &g) {
 // buffers: one per parity of the swapped position buffers, both recaptured
 // after anything that changes what the launches read (a construction,
 // reallocation, option or thermostat change).
-int launch_fused_graph(mdgpu_domain *d, bool gated = false) {
-  StepGraph *gs = gated ? d->gated : d->graphs;
+int launch_fused_graph(mdgpu_domain *d, bool gated = false, bool single = false) {
+  StepGraph *gs = single ? d->single : gated ? d->gated : d->graphs;
   StepGraph *g = nullptr;
   for (int k = 0; k < 2; k++)
     if (gs[k].exec && gs[k].epoch == d->epoch && gs[k].key == (const void *)d->pos_tmp) g = &gs[k];
@@ -1850,7 +1854,7 @@ int launch_fused_graph(mdgpu_domain *d, bool gated = false) {
     drop_graph(*g);
     hipGraph_t graph = nullptr;
     HIPCHK(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeRelaxed));
-    const int r = enqueue_fused(d, d->clock, false, gated);
+    const int r = enqueue_fused(d, d->clock, false, gated, single);
     const hipError_t e = hipStreamEndCapture(d->stream, &graph);
     if (r != MDGPU_OK) {
       if (e == hipSuccess && graph) (void)hipGraphDestroy(graph);
@@ -1977,6 +1981,7 @@ int calculate_step(mdgpu_domain *d) {
     d->mid_valid = true;
     d->vmax_valid = true;
   }
+  d->since_build++;
   d->sim_time += d->dt;
   d->step++;
   return MDGPU_OK;
@@ -1986,10 +1991,27 @@ int calculate_step(mdgpu_domain *d) {
 // (replayed from graphs or launched) on the full list.
 bool can_run(const mdgpu_domain *d) { return d->run_ahead > 0 && !d->timing && !inner_steps(d) && d->pn > 0; }
 
-double &zeta_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->zeta : d->rst[r].zeta; }
-
 double &budget_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->buffer_length : d->rst[r].buffer_length; }
 int &lifetime_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->lifetime : d->rst[r].lifetime; }
+
+// Whether the host has all that the next step's validity test needs: every
+// budget outlasts the step and the one after it, at the largest |p| of the last
+// step.  The only step of a call is then taken by calculate_step, without a
+// run's first launch: one step a call takes 42 us at 119,000 particles and 444
+// at 3.88M, 46 and 452 as a run of one.  With less budget the run of one
+// measures displacements on the device, where calculate_step would stop for
+// checks (119,000 particles with checks and constructions: 50 us a step, 54
+// with calculate_step alone), and a Nose-Hoover step taken alone would wait for
+// its temperatures.
+bool host_settles(mdgpu_domain *d) {
+  if (d->thermostat == MDGPU_NOSEHOOVER || !d->initialized || !d->mid_valid || !d->vmax_valid || d->run_halted)
+    return false;
+  for (int r = 0; r < d->nrep; r++)
+    if (!(budget_of(d, r) > kMeasureAhead * std::sqrt(d->h_rep_v2[r]) * d->dt)) return false;
+  return true;
+}
+
+double &zeta_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->zeta : d->rst[r].zeta; }
 
 // Steps to queue at once: as many as the list should still last, by what the
 // last one lasted (a list's life varies little from one to the next), or, for
@@ -2069,13 +2091,14 @@ int run_steps(mdgpu_domain *d, int limit, int *done) {
                      d->run_cand, d->reps, d->grng, d->ng, approved ? 1 : 0, keep ? 1 : 0, ke, d->clock,
                      (unsigned long long)d->step, d->h_gate);
   const double4 *qh = d->pos_tmp, *qh2 = d->pos_next;
+  const bool single = k == 1;
   for (int j = 0; j < k; j++) {
-    if (d->use_graph) CHK(launch_fused_graph(d, true));
-    else CHK(enqueue_fused(d, d->clock, false, true));  // the same launches, each queued directly
+    if (d->use_graph) CHK(launch_fused_graph(d, true, single));
+    else CHK(enqueue_fused(d, d->clock, false, true, single));  // the same launches, each queued directly
     std::swap(d->pos_tmp, d->pos_next);
     if (mixed) std::swap(d->rel_tmp, d->rel_next);
   }
-  CHK(final_positions(d, qh, qh2, d->gate));
+  if (!single) CHK(final_positions(d, qh, qh2, d->gate));
   CHK(sync(d));
   const int n = d->h_gate->done;
   if (n < 0 || n > k) {
@@ -3504,6 +3527,7 @@ int mdgpu_destroy(mdgpu_domain *d) {
                   d->rep_factor};
   for (StepGraph &g : d->graphs) drop_graph(g);
   for (StepGraph &g : d->gated) drop_graph(g);
+  for (StepGraph &g : d->single) drop_graph(g);
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   if (d->pinned) (void)hipHostFree(d->pinned);
@@ -3833,7 +3857,7 @@ int mdgpu_calculate(mdgpu_domain *d, int nsteps, int *rebuilds) {
   int r = MDGPU_OK;
   int s = 0;
   while (s < nsteps && r == MDGPU_OK) {
-    if (can_run(d)) {
+    if (can_run(d) && !(nsteps - s == 1 && host_settles(d))) {
       int done = 0;
       r = run_steps(d, nsteps - s, &done);
       s += done;

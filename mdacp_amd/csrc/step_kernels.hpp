@@ -581,6 +581,12 @@ struct RunShared {
 };
 static_assert(kTailThreads / kWave * kWaveCands >= kGroupCands, "a replica's candidates fit");
 
+// A step is measured once the budget is down to this many times max|p| dt: from
+// two tests before it is spent (2 max|p| dt each, a little more if max|p|
+// grows), so that the step that spends it knows what its displacements can
+// reach.
+constexpr double kMeasureAhead = 4.5;
+
 // CheckByDisplacement's last part for one replica, by the T lanes t of a
 // wavefront or workgroup: true when a pair of candidates was beyond SL at the
 // construction and is now inside rc.  The m candidates are at sh.c[.][base..].
@@ -711,14 +717,11 @@ __device__ __forceinline__ bool run_gate(RunRep *rr, int nrep, const RunRules &U
       }
       S.lifetime++;
     }
-    // the next step, measured from two tests before the budget is spent (2
-    // max|p| dt each, a little more if max|p| grows), so that the step that
-    // spends it knows what its displacements can reach: no displacement grows
-    // by more than max|p| dt
+    // the next step: no displacement grows by more than max|p| dt
     const double v = sqrt(S.v2), reach = sqrt(S.dmax2) + 1.05 * v * U.dt;
     const bool bound = S.measured && reach < U.margin;
     S.cthr = bound ? U.margin - reach : 1.0e200;
-    S.measured = !(S.budget > 4.5 * v * U.dt);
+    S.measured = !(S.budget > kMeasureAhead * v * U.dt);
     S.ncand = 0;
     // Nose-Hoover: the step starts with a HeatbathZeta at the temperature the
     // last one ended with, and scales the momenta by this factor (HeatbathMomenta,
