@@ -847,14 +847,35 @@ long long axis_staged_cells(int ms, int bd) {
 // the neighbourhood is the per-brick overhead of the search and force kernels.
 // A box too small to give every CU a workgroup that way takes smaller bricks:
 // the ones that stage the fewest cells among those that reach kBrickFill of
-// the CUs (shared out over the replicas), or, smaller still, the most bricks
-// there are.  With 8 bricks of 5x5x3 cells on 256 CUs a kick of 2,048
-// particles took 15.5 us, with 216 of one cell 12.3 (8,000 particles: 22.1
-// and 14.3; 32,000: 23.5 and 15.6), a construction 360 and 290 us.
+// the CUs (shared out over the replicas, or over the units that one launch
+// kicks), or, smaller still, the most bricks there are.  With 8 bricks of 5x5x3
+// cells on 256 CUs a kick of 2,048 particles took 15.5 us, with 216 of one cell
+// 12.3 (8,000 particles: 22.1 and 14.3; 32,000: 23.5 and 15.6), a construction
+// 360 and 290 us.
+//
+// Units go beyond their share, to the CUs' worth of bricks in each, while the
+// bricks keep kBrickRows rows, about three slices for the eight wavefronts: a
+// launch of three and more rounds of workgroups wastes less of its last one.
+// Kicks of 2x2x2 units, share / as many as CUs in each (us): 19,652 particles
+// 15.8 / 30.2, 78,732 22.1 / 41.2 (25.2 / 51.6 at rho = 0.9), where each brick
+// would hold 11 to 40 rows; 953,312 104.7 / 95.2 (172 / 150), with 440 to 490.
 constexpr double kBrickFill = 0.9;
+constexpr double kBrickRows = 200.0;
+
+// Systems that share a kick's launch: the replicas, or the units of a grid of
+// up to kMaxKickUnits (group_batched; larger grids kick unit by unit).
+int kicked_together(const mdgpu_domain *d) {
+  if (!d->group) return d->nrep;
+  const int *g = d->group->grid;
+  const long long n = (long long)g[0] * g[1] * g[2];
+  return n <= kMaxKickUnits ? (int)n : 1;
+}
 
 void auto_brick(const mdgpu_domain *d, double rho, const double L[3], int kb, int bd[3], double fill) {
-  const long long least = (long long)(kBrickFill * d->num_cu / d->nrep);
+  const double cus = kBrickFill * d->num_cu;
+  double want = cus / kicked_together(d);
+  if (d->group) want = std::max(want, std::min(cus, rho * L[0] * L[1] * L[2] / kBrickRows));
+  const long long least = (long long)want;
   const double budget = fill * std::min(kb, d->lds_max_kb) * 1024.0;
   int ms[3];
   double vol = 1.0;

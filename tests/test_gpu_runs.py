@@ -274,3 +274,27 @@ def test_steps_one_a_call_match_a_long_run(form, thermostat):
     assert a.time() == b.time()
     for d in ds:
         d.close()
+
+
+@pytest.mark.parametrize("grid,L", [((2, 2, 2), 54.0), ((2, 1, 2), 40.0), ((3, 3, 3), 54.0)])
+def test_a_groups_bricks_fill_the_cus_once(grid, L):
+    """The bricks that the units of a small grid choose fill the CUs together, since one launch kicks
+    them all; the units of a grid of more than eight, kicked one by one, each do.  256 CUs, 0.9 of
+    them: 230 bricks, and no more than three times that where bricks of two cells would do."""
+    print("case: bricks of a group", grid, L, flush=True)
+    q = fcc(L, 0.5)
+    us = mdgpu.unit_grid(L, grid, dt=0.005, rc=2.5, margin=0.5, capacity=len(q))
+    for u in us:
+        u.add_particles(q, initial_velocity(len(q), 1.0, seed=2))
+    us[0].group_make_pair_list()
+    bricks, all_cells = [], []
+    for u in us:
+        v = u.get_option(mdgpu.OPT_BRICK)
+        ms = [int((e - s) / 3.0) for s, e in zip(u.s, u.e)]
+        bricks.append(math.prod((m + b) // b for m, b in zip(ms, (v & 255, v >> 8 & 255, v >> 16))))
+        all_cells.append(math.prod(m + 1 for m in ms))
+    print("bricks", bricks, "of", all_cells, flush=True)
+    if len(us) <= 8:
+        assert 200 <= sum(bricks) <= 3 * 256, bricks
+    else:
+        assert all(b >= min(230, c) for b, c in zip(bricks, all_cells)), bricks
