@@ -298,3 +298,40 @@ def test_a_groups_bricks_fill_the_cus_once(grid, L):
         assert 200 <= sum(bricks) <= 3 * 256, bricks
     else:
         assert all(b >= min(230, c) for b, c in zip(bricks, all_cells)), bricks
+
+
+@pytest.mark.parametrize("form", ["brick frame", "cell frame", "pipelined", "graph"])
+def test_nose_hoover_runs_in_every_form(form):
+    """Nose-Hoover in runs against steps that each wait for the host, for the kicks that
+    test_nose_hoover_runs_follow_single_steps does not run, with the time constant and the target
+    changed on the way.  FP64: to rounding, as there.  MIXED: a coordinate that the rounding puts on
+    the other side of an FP32 boundary moves by 1e-6, which changes a momentum by about 1e-6 (force
+    gradients up to some hundreds, dt 0.005) and grows over the steps: 1e-4."""
+    print("case: Nose-Hoover", form, flush=True)
+    (boxes, counts, q, p, ids), _ = replicas(1, lambda r: 8, lambda r: 0.5)
+    ds = []
+    for ahead in (64, 0):
+        d = mdgpu.Domain(boxes[0], dt=0.005, capacity=len(q))
+        d.set_precision(mdgpu.MIXED if "frame" in form else mdgpu.FP64)
+        d.set_option(mdgpu.OPT_MIXED_FRAME, 0 if form == "cell frame" else 1)
+        d.set_option(mdgpu.OPT_PIPELINE, form == "pipelined")
+        d.set_option(mdgpu.OPT_GRAPH, form == "graph")
+        d.set_option(mdgpu.OPT_RUN_AHEAD, ahead)
+        d.add_particles(q, p, ids)
+        ds.append(d)
+    a, b = ds
+    bar = 1e-4 if "frame" in form else 1e-10
+    ra = rb = 0
+    for chunk, T, tau in ((1, 1.2, 0.3), (40, 1.2, 0.3), (2, 1.2, 0.1), (17, 0.9, 0.1)):
+        for d in ds:
+            d.set_thermostat(mdgpu.NOSEHOOVER, T=T, tau=tau)
+        ra += a.calculate(chunk)
+        rb += b.calculate(chunk)
+        assert ra == rb, (chunk, ra, rb)
+        assert abs(a.zeta() - b.zeta()) < bar
+    assert ra >= 2 and abs(b.zeta()) > 1e-3, (ra, b.zeta())
+    (qa, pa, ta), (qb, pb, tb) = a.particles(), b.particles()
+    assert np.array_equal(ta, tb)
+    assert np.abs(qa - qb).max() < bar and np.abs(pa - pb).max() < bar
+    for d in ds:
+        d.close()
