@@ -20,6 +20,7 @@
 #include "build_kernels.hpp"
 #include "force_kernels.hpp"
 #include "list_kernels.hpp"
+#include "room.hpp"
 #include "scan.hpp"
 #include "step_kernels.hpp"
 
@@ -1110,7 +1111,9 @@ int ensure_build(mdgpu_domain *d) {
     staged = rho * R.w[0] * R.w[1] * R.w[2] * ((R.bd[0] + 2) * (R.bd[1] + 2) * (R.bd[2] + 2));
     if (staged > kMaxStaged) continue;  // k_brick_ranges will refuse it: no room for its list
     entries += staged * R.nb[0] * R.nb[1] * R.nb[2];
-    slots += pn * (rho * (4.0 / 3.0) * M_PI * d->SL * d->SL * d->SL * 1.25 + 16.0);
+    double bricks = 1.0;  // those of cells 1 .. m - 2: no row but at a box's upper face lies past them
+    for (int k = 0; k < 3; k++) bricks *= (R.m[k] - 2 + R.bd[k] - 1) / R.bd[k];
+    slots += expected_slots(pn, rho * (4.0 / 3.0) * M_PI * d->SL * d->SL * d->SL, bricks);
   }
   if (d->glist_cap == 0) CHK(grow_glist(d, (long long)(1.1 * entries)));
   if (d->nbr_cap == 0) CHK(grow_slots(d, (long long)slots));
