@@ -303,7 +303,8 @@ int mdgpu_get_timing(const mdgpu_domain *d, int *force_launches, double *force_m
                                    step's validity test, budget and displacement check, runs on
                                    the device at the end of the step before and stops the run
                                    where a list has expired, for the host to rebuild; the same
-                                   trajectory either way */
+                                   trajectory either way (Nose-Hoover: to rounding, its
+                                   temperature summed brick by brick in such steps) */
 #define MDGPU_OPT_PIPELINE 14  /* FP64 kick with 4, 8 or 16 wavefronts: 1 = persistent workgroups (one
                                   per CU) whose producer wavefronts stage the next brick's
                                   neighbourhood into a second LDS buffer with LDS-direct loads while

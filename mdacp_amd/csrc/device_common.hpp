@@ -25,9 +25,7 @@ __host__ __device__ __forceinline__ long long slot_of(int k, int lane) {
 
 // Error bits raised by kernels; read back at the existing sync points.
 constexpr int kErrInvalidPosition = 1;
-constexpr int kErrInvalidIndex = 2;
 constexpr int kErrCapacity = 4;
-constexpr int kErrLayout = 8;  // a listed partner outside its brick's staged ranges
 constexpr int kErrSearchCap = 16;   // a row has more candidates than its bitmask holds
 constexpr int kErrGhostCap = 32;    // more ghost images than there is room for
 constexpr int kErrGatherCap = 64;   // ... gather-list entries
@@ -38,8 +36,7 @@ constexpr int kErrStagedCap = 256;  // a brick stages more entries than 16 bits 
 // little sets its bit; the kernels after it do nothing; and the host, which
 // reads the state once at the end, makes room and queues them again from
 // there.  Bits set before the rows are ordered:
-constexpr int kErrBeforeRows =
-    kErrInvalidPosition | kErrInvalidIndex | kErrSearchCap | kErrGhostCap | kErrGatherCap | kErrStagedCap;
+constexpr int kErrBeforeRows = kErrInvalidPosition | kErrSearchCap | kErrGhostCap | kErrGatherCap | kErrStagedCap;
 
 // What a construction's kernels count (device; copied to the host at its end).
 struct BuildState {

@@ -620,7 +620,7 @@ __global__ __launch_bounds__(kWave *W, U <= 2 ? 4 : 1) void k_force_brick_fp64(c
 // unit's own kick does (CalculateForce in place, or the kick of a fused step),
 // on the unit's own arrays.  One launch of all the units' bricks fills the CUs where one
 // launch per unit ends each unit with a partial round of workgroups.  The
-// table travels in the kernel arguments (1 KB for kMaxKickUnits units).
+// table travels in the kernel arguments (1.2 KB for kMaxKickUnits units).
 struct UnitKick {
   const double4 *src;  // owned positions (the ghosts': bl.ghost)
   double4 *mom;
@@ -807,7 +807,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
       if (nrow > 0) {
         const Replica &Rp = bl.reps[bl.brep[b]];
         const LangevinConsts lc = langevin_consts(Rp, sc.dt, step_of(sc));
-  const double nhf = step_factor(sc, bl.brep[b], epilogue);
+        const double nhf = step_factor(sc, bl.brep[b], epilogue);
         const int row0 = bl.row0[b], vs0 = bl.vslice0[b];
         const long long g0 = bl.gbase[b];
         const int total = (int)(bl.gbase[b + 1] - g0);
@@ -842,7 +842,7 @@ __global__ __launch_bounds__(kWave *(W + P)) void k_force_pipe_fp64(const double
       for (int k = 1; k < W; k++) m = fmax(m, wmax[cur][k]);
       vpart[b] = m;
     }
-      if (sc.meas.rr != nullptr) {  // uniform: every wavefront, producers included
+    if (sc.meas.rr != nullptr) {  // uniform: every wavefront, producers included
       if (bl.nrow[b] > 0)
         measure_brick<kWave *(W + P)>(b, bl.brep[b], bl.row0[b], bl.nrow[b], src, mom, epilogue, fc.dt2,
                                       bl.reps[bl.brep[b]], sc.meas);

@@ -266,7 +266,7 @@ struct mdgpu_domain {
   double *bpart = nullptr;  // one maximum per brick workgroup
   int partial_n = 0;
   int *cand = nullptr;
-  // small device scalars: u64 [0] vmax2 [1] dmax2 [2] max staged; i32 [0] err [1] count [2] flag
+  // small device scalars: u64 [0] vmax2 [1] dmax2; i32 [1] count [2] flag
   unsigned long long *u64 = nullptr;
   long long *i64 = nullptr;
   int *i32 = nullptr;
@@ -357,14 +357,14 @@ int check_launch(mdgpu_domain *d, const char *what) {
   return MDGPU_OK;
 }
 
-// Invalidate the captured steps and the half drift the next fused step would
-// reuse (state that the step reads has changed).
-// what is known of the largest |p| is no longer
+// The largest |p| is no longer known (the momenta have changed).
 void momenta_changed(mdgpu_domain *d) {
   d->vmax_valid = false;
   d->drift_blocks = 0;
 }
 
+// Invalidate the captured steps and the half drift the next fused step would
+// reuse (state that the step reads has changed).
 void invalidate(mdgpu_domain *d) {
   d->mid_valid = false;
   d->inner_valid = false;
@@ -665,14 +665,6 @@ int build_error(mdgpu_domain *d, int e) {
   if (e & kErrInvalidPosition) {
     d->err = "Invalid position";
     return MDGPU_ERR_INVALID_POSITION;
-  }
-  if (e & kErrInvalidIndex) {
-    d->err = "Invalid index";
-    return MDGPU_ERR_INVALID_INDEX;
-  }
-  if (e & kErrLayout) {
-    d->err = "internal: a listed partner lies outside its brick's staged ranges";
-    return MDGPU_ERR_HIP;
   }
   if (e & kErrCapacity) {
     d->err = "pair list capacity";
@@ -1029,7 +1021,8 @@ int queue_images(mdgpu_domain *d) {
     CHK(scan(d, ScanImages{d->nimg, d->goff, d->bs, d->gcap}, pn, &d->bs->err));
     // pos_tmp[0..ng) holds the unsorted images
     hipLaunchKernelGGL(k_emit_images, dim3(nblk(pn)), dim3(kBlock), 0, st, d->pos, pn, d->rep, d->reps, d->SL,
-                       d->goff, d->bs, GhostArrays{d->t_gsrc, d->t_gcode, d->pos_tmp, d->t_gcell, d->slot, d->c_gcount});
+                       d->goff, d->bs,
+                       GhostArrays{d->t_gsrc, d->t_gcode, d->pos_tmp, d->t_gcell, d->slot, d->c_gcount});
   }
   CHK(scan(d, ScanArray<int, int>{d->c_gcount, d->c_gstart, nullptr}, d->ncell));
   if (pn > 0) {
@@ -1136,8 +1129,8 @@ int queue_from(mdgpu_domain *d, BuildStage from) {
     CHK(queue_rows(d));
   }
   if (rows) CHK(launch_emit(d, bricks_of(d), search_tables(d)));
-  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kPublishThreads), 0, d->stream, d->bs, d->btotal, rows ? d->bsum : nullptr,
-                     d->nbrick, d->h_bs);
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kPublishThreads), 0, d->stream, d->bs, d->btotal,
+                     rows ? d->bsum : nullptr, d->nbrick, d->h_bs);
   return check_launch(d, "construction");
 }
 
@@ -1655,8 +1648,8 @@ int launch_force(mdgpu_domain *d, const double4 *src, const float4 *rel, double4
       hipLaunchKernelGGL(k_run_max, dim3(d->nrep), dim3(kBlock), 0, st, d->gate, d->bpart, d->dpart,
                          bath ? d->kpart : nullptr, d->reps, d->rr);
     hipLaunchKernelGGL(k_run_tail, dim3(1), dim3(kTailThreads), 0, st, d->gate, own ? nullptr : d->bpart, d->dpart,
-                       d->kpart, d->rr, d->nrep, run_rules(d), d->run_cand, d->reps, d->grng, d->ng, d->clock, d->h_gate,
-                       d->h_rr);
+                       d->kpart, d->rr, d->nrep, run_rules(d), d->run_cand, d->reps, d->grng, d->ng, d->clock,
+                       d->h_gate, d->h_rr);
   } else if (want_vmax) {
     hipLaunchKernelGGL(k_replica_max, dim3(d->nrep), dim3(kBlock), 0, st, d->bpart, d->reps, d->rep_v2, clock);
     HIPCHK(d, hipMemcpyAsync(d->h_rep_v2, d->rep_v2, d->nrep * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -2023,10 +2016,9 @@ int &lifetime_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->lifetime : d
 // step.  The only step of a call is then taken by calculate_step, without a
 // run's first launch: one step a call takes 42 us at 119,000 particles and 444
 // at 3.88M, 46 and 452 as a run of one.  With less budget the run of one
-// measures displacements on the device, where calculate_step would stop for
-// checks (119,000 particles with checks and constructions: 50 us a step, 54
-// with calculate_step alone), and a Nose-Hoover step taken alone would wait for
-// its temperatures.
+// measures displacements on the device, where calculate_step would launch the
+// host's checks and wait for them, and a Nose-Hoover step taken alone would wait
+// for its temperatures.
 bool host_settles(mdgpu_domain *d) {
   if (d->thermostat == MDGPU_NOSEHOOVER || !d->initialized || !d->mid_valid || !d->vmax_valid || d->run_halted)
     return false;
@@ -2038,8 +2030,9 @@ bool host_settles(mdgpu_domain *d) {
 double &zeta_of(mdgpu_domain *d, int r) { return d->nrep == 1 ? d->zeta : d->rst[r].zeta; }
 
 // Steps to queue at once: as many as the list should still last, by what the
-// last one lasted (a list's life varies little from one to the next), or, for
-// the first, by the budgets at the last maxima of |p|.  A run past its list's
+// last one lasted (a list's life varies little from one to the next), or, until
+// one has expired, by the budgets at the last maxima of |p|, which count neither
+// the displacement checks nor what they re-arm (a list lives longer).  A run past its list's
 // end wastes two launches that return at once per step (about 6 us), and one
 // that ends before it costs a wait for the host and the final positions (30 to
 // 80 us), hence at least kRunLeast.
@@ -2066,8 +2059,9 @@ int run_length(mdgpu_domain *d, int limit) {
 // last operation was no fused step (its maxima of |p|, or its next half drift,
 // which moves the ghosts that the check reads, are not there): the
 // displacement check or the construction that step needs, after which the run
-// goes on with it.  *done receives the steps completed.  The lists' state goes to the device with the
-// run's first launch and comes back with its last (pinned memory both ways).
+// goes on with it.  *done receives the steps completed.  The lists' state goes
+// to the device with the run's first launch and comes back with its last
+// (pinned memory both ways).
 int run_steps(mdgpu_domain *d, int limit, int *done) {
   hipStream_t st = d->stream;
   const int R = d->nrep;
@@ -2603,7 +2597,7 @@ int unit_ghosts(mdgpu_domain *d) {
 }
 
 // The unit's ghost sources after every source unit has built its list and
-// ordered its rows (order_rows permutes a unit's owned particles): each
+// ordered its rows (k_order_rows permutes a unit's owned particles): each
 // source index mapped through its unit's row order, once per construction.
 // The group's lock is held.
 int remap_unit_ghosts_locked(mdgpu_domain *d) {
@@ -3546,7 +3540,8 @@ int mdgpu_destroy(mdgpu_domain *d) {
                   d->i32,     d->d3,          d->reps,        d->brep,      d->rep,      d->rep_alt,
                   d->grng,    d->rep_v2,      d->rep_out,     d->which,     d->rep_exp,  d->clock,
                   d->nbr_in,      d->ncode_in,    d->slen_in,   d->chk_dmax, d->chk_cnt,
-                  d->chk_cand, d->gate,       d->gimg,       d->rr,          d->run_cand,  d->dpart,     d->kpart,     d->xfer,     d->gunit,
+                  d->chk_cand, d->gate,       d->gimg,        d->rr,        d->run_cand, d->dpart,
+                  d->kpart,   d->xfer,        d->gunit,
                   d->st_pos,  d->st_mom,      d->st_id,       d->src_tab,   d->ucnt,     d->uoff,
                   d->rep_factor};
   for (StepGraph &g : d->graphs) drop_graph(g);

@@ -464,7 +464,7 @@ __global__ __launch_bounds__(kBlock) void k_replica_max(const double *__restrict
 }
 
 // The maxima of a run's step into its replicas' RunRep, one workgroup per
-// replica (k_run_tail's first part, for kTailReplicas replicas and more).
+// replica (k_run_tail's first part, for more than kTailReplicas replicas).
 __global__ __launch_bounds__(kBlock) void k_run_max(const RunGate *__restrict__ gate, const double *__restrict__ part,
                                                     const double *__restrict__ dpart,
                                                     const double *__restrict__ kpart,
@@ -779,9 +779,9 @@ __global__ __launch_bounds__(kTailThreads) void k_run_begin(RunGate *gate, int l
 // the host's pinned copies (host, to).  One workgroup, the whole of it over
 // the bricks of a single replica, or a wavefront per replica: one launch in
 // place of the maxima's and the next step's gate, whose cost per step is their
-// launches (4.6 + 4.3 us and a gap, against 4.6).  From kTailReplicas replicas
-// on, a wavefront would take more than 8 of them in turn, about 1 us each: the
-// maxima then have a launch of their own with a workgroup per replica
+// launches (4.6 + 4.3 us and a gap, against 4.6).  With more than kTailReplicas
+// replicas a wavefront would take more than 8 of them in turn, about 1 us each:
+// the maxima then have a launch of their own with a workgroup per replica
 // (k_run_max) and part is nullptr here.
 constexpr int kTailReplicas = 128;
 
