@@ -707,8 +707,12 @@ int lds_cap_for(const mdgpu_domain *d, int bytes_per_entry, int kb) {
 constexpr int kSearchLdsKb = 96;
 
 // Room per brick for the search's staging: what the last construction with
-// these bricks needed and a little more (not known: all of the budget).  A
-// brick that needs more reads its candidates from memory.
+// these bricks needed and a little more (not known: all of the budget), so that
+// small neighbourhoods leave room for a second workgroup on the CU.  A brick
+// that needs more reads its candidates from memory.  Constructions with all of
+// the budget and with this: 48 replicas at rho = 0.85 775 and 716 us, 128 at
+// 0.35 1765 and 1715, 953,312 particles at 0.3 613 and 599, 1,372 at 0.9 183
+// and 175; from 27,000 to 4M particles at 0.5 and above the same.
 int search_lds_cap(const mdgpu_domain *d) {
   const int budget = std::min(kSearchLdsKb, d->lds_max_kb) * 1024 / (3 * (int)sizeof(double));
   return d->staged_guess ? std::max(1, std::min(d->staged_guess + d->staged_guess / 16 + 32, budget)) : budget;
